@@ -1,21 +1,34 @@
-// Fused dense gates of K = 5 or 6 targets in complex64, applied as real
-// GEMMs on FP32 matrix cores (v_mfma_f32_16x16x4f32, FP32 accumulation).
+// Fused dense gates of K = 3 to 6 targets, applied as real GEMMs on matrix
+// cores: complex64 through v_mfma_f32_16x16x4f32, complex128 through
+// v_mfma_f64_16x16x4f64 (accumulation in the state's precision).
 //
 // A column is one group of D = 2^K amplitudes the gate mixes (the iteration
 // index spread over the non-target, non-control bits, as in k_dense). With
-// U = Ur + i Ui and a column a = ar + i ai, the output is
-//     [or; oi] = R [ar; ai],   R = [[Ur, -Ui], [Ui, Ur]]   (2D x 2D real),
-// so a block of NC columns is the real product (2D x 2D) x (2D x NC).
-// A workgroup of WAVES waves (4 for K = 5, 8 for K = 6: one 16-row tile of R
-// each) stages each block's amplitudes through LDS (coalesced loads and
-// stores, the next block's loads in flight during the products); each wave
-// keeps its rows of R in registers for the whole launch and computes those
-// rows of the output for all NC columns. Blocks of 32 columns keep a 6-qubit
-// workgroup at 78 VGPRs, so three share a CU (six waves per SIMD); the grid
-// is 12 workgroups per CU. (Measured on the 32-qubit precision form: 64
-// columns at 4 workgroups per CU 0.855 s, 32 at 12 0.826 s, 128 at 4 0.987 s;
-// an XOR-swizzled LDS layout without bank conflicts 1.13 s, its per-lane
-// operand addresses costing more than the conflicts.)
+// U = Ur + i Ui the output's parts are real dot products of the column's
+// parts with the rows of a 2D x 2D real matrix R, so a block of NC columns is
+// the product (2D x 2D) x (2D x NC). R's rows and columns interleave the real
+// and imaginary part of each index, so that the four accumulators of a lane
+// are two whole amplitudes of one column: they go to memory straight from
+// the accumulators, 16 neighbouring columns (128 or 256 bytes) at a time.
+//
+// A workgroup has one wave per 16 rows of R (8 for K = 6, 1 for K = 3); each
+// wave keeps its rows in registers for the whole launch. Blocks of NC columns
+// pass through two LDS buffers: while the waves multiply block b, block b + 1
+// is in flight from memory, and it is written to the other buffer before the
+// one barrier of the iteration.
+//
+// Bounds at 28 qubits (2^28 columns x amplitudes): one pass is 0.79 ms in
+// complex64 and 1.58 ms in complex128 at the 5.4 TB/s of a large copy; the
+// products of a 6-qubit gate are 0.87 ms at the FP32 matrix peak and 1.75 ms
+// at the FP64 one (78.6 TFLOP/s, as the FP64 vector rate), half of that for 5
+// qubits. Measured, host call included: K = 6 1.23 ms and 2.14 ms (the
+// products, at 71 and 82 % of their peak), K = 5 0.95 ms and 1.67-1.84 ms
+// (memory). Before, with one LDS buffer, outputs through LDS and four barriers
+// per block, FP32 K = 6 took 1.38 ms and K = 5 0.97 ms; complex128 ran on
+// vector FMAs with the matrix in LDS: 12.0 ms and 9.1 ms. Blocks of 64
+// columns: 1.26 and 2.46 ms. Workgroups per CU: two for K = 6, what its
+// registers allow (12: 1.28 ms, each workgroup loading its rows of R again);
+// many small ones for the others (K = 5 in FP32: 2 1.04, 3 0.92, 12 0.92 ms).
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -27,8 +40,39 @@ namespace qvd {
 
 namespace {
 
+typedef float floatx4 __attribute__((ext_vector_type(4)));
+typedef double doublex4 __attribute__((ext_vector_type(4)));
+
+// The 16 x 16 x 4 matrix instruction of a precision. Operand A: lane l holds
+// row l % 16, k = l / 16; operand B: column l % 16, k = l / 16. Accumulator
+// e of lane l is column l % 16 and row 4 (l / 16) + e in FP32, row
+// 4 e + l / 16 in FP64.
+template <typename T2> struct Mfma;
+template <> struct Mfma<float2> {
+    using R = float;
+    using V = floatx4;
+    static __device__ __forceinline__ V mul(float a, float b, V c) {
+        return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+    }
+    // Row r of a tile is accumulator `e` of the lanes l with l / 16 = `q`.
+    static __device__ __forceinline__ uint32_t q_of(uint32_t r) { return r >> 2; }
+    static __device__ __forceinline__ uint32_t e_of(uint32_t r) { return r & 3; }
+};
+template <> struct Mfma<double2> {
+    using R = double;
+    using V = doublex4;
+    static __device__ __forceinline__ V mul(double a, double b, V c) {
+        return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
+    }
+    static __device__ __forceinline__ uint32_t q_of(uint32_t r) { return r & 3; }
+    static __device__ __forceinline__ uint32_t e_of(uint32_t r) { return r >> 2; }
+};
+
 constexpr int NC = 32;         // columns per block
-constexpr int PAD = NC + 1;    // row pitch of the staged block (floats)
+constexpr int CB = 5;          // column bits of a block
+static_assert(NC == 1 << CB, "a block's columns are all values of its column bits");
+constexpr int PITCH = NC + 1;  // row pitch of a staged block (amplitudes)
+constexpr int SLOTS = 3;       // column bases of the block multiplied, loaded and prepared
 
 __device__ __forceinline__ uint64_t spread(uint64_t x, const uint32_t *pos, uint32_t m) {
     for (uint32_t j = 0; j < m; j++) {
@@ -39,158 +83,190 @@ __device__ __forceinline__ uint64_t spread(uint64_t x, const uint32_t *pos, uint
     return x;
 }
 
-template <int K, int WAVES>
-__global__ __launch_bounds__(64 * WAVES) void k_dense_mfma(float2 *__restrict__ s, const GateDesc d,
-                                                           const float2 *__restrict__ mat) {
-    constexpr int D = 1 << K, M = 2 * D;       // R is M x M
-    constexpr int MPW = M / 16 / WAVES;        // 16-row tiles of R per wave
-    constexpr int KS = M / 4;                  // k steps of 4
-    constexpr int PER = D * NC / (64 * WAVES); // amplitudes staged per thread
-    extern __shared__ float lds[];
-    float *Br = lds;                                 // D x PAD: real parts (row j, column c)
-    float *Bi = Br + D * PAD;                        // D x PAD: imaginary parts
-    uint64_t *colbase = (uint64_t *)(Bi + D * PAD);  // 2 x NC: first amplitude of each column (double-buffered)
-    uint64_t *offs = colbase + 2 * NC;               // D: offset of target index j
-    const uint32_t tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+template <typename T2, int K>
+constexpr size_t mfma_lds_bytes() {
+    return 2 * sizeof(T2) * (size_t(1) << K) * PITCH + SLOTS * NC * sizeof(uint64_t);
+}
+
+template <typename T2, int K>
+__global__ __launch_bounds__(64 << (K - 3)) void k_dense_mfma(T2 *__restrict__ s, const GateDesc d,
+                                                              const T2 *__restrict__ mat) {
+    using M = Mfma<T2>;
+    using R = typename M::R;
+    using V = typename M::V;
+    constexpr int D = 1 << K, THREADS = 8 * D;  // 2D / 16 waves
+    constexpr int KS = 2 * D / 4;               // k steps of 4
+    constexpr int PER = D * NC / THREADS;       // amplitudes staged per thread
+    constexpr uint64_t NONE = ~uint64_t(0);     // a column past the last one
+    extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
+    T2 *const buf = reinterpret_cast<T2 *>(smem_raw);                       // 2 x D x PITCH
+    uint64_t *const colbase = reinterpret_cast<uint64_t *>(buf + 2 * D * PITCH);  // SLOTS x NC
+    const uint32_t tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, q = lane >> 4, cl = lane & 15;
     const uint64_t blocks = (d.iterations + NC - 1) / NC;
-    // Target index fastest when the lowest target is qubit 0 (a column's
-    // amplitudes are then contiguous), else column fastest.
-    const bool jfast = d.offsets[1] == 1;
-    auto elem = [&](uint32_t e, uint32_t &j, uint32_t &c) {
-        j = jfast ? e % D : e / NC;
-        c = jfast ? e / D : e % NC;
-    };
-    auto bases = [&](uint64_t blk, uint64_t *out) {
-        if (tid < (uint32_t)NC) {
-            const uint64_t col = blk * NC + tid;
-            out[tid] = col < d.iterations ? (spread(col, d.ins, d.nins) | d.ctrl_val) : ~uint64_t(0);
+    uint64_t blk = blockIdx.x;
+    if (blk >= blocks) return;  // uniform over the workgroup
+    const uint64_t step = gridDim.x;
+    auto bases = [&](uint64_t b, uint32_t slot) {
+        if (tid < (uint32_t)NC && b < blocks) {
+            const uint64_t col = b * NC + tid;
+            colbase[slot * NC + tid] = col < d.iterations ? (spread(col, d.ins, d.nins) | d.ctrl_val) : NONE;
         }
     };
 
-    // This wave's rows of R stay in registers for the whole launch: lane l
-    // holds R[row][4 ks + l / 16] of row = 16 mt + l % 16.
-    float ra[MPW][KS];
-#pragma unroll
-    for (int i = 0; i < MPW; i++) {
-        const uint32_t row = (wave * MPW + i) * 16 + (lane & 15);
-        const uint32_t rr = row % D;
-        const bool rim = row >= (uint32_t)D;
+    // This wave's rows of R. Row (and column) indices pair up as (index of
+    // U, part): the lane's accumulators e are index 2q + e / 2 of the wave's
+    // 8 and part e % 2, and k = 4 ks + q is index k / 2, part k % 2.
+    R ra[KS];
+    {
+        const uint32_t jr = wave * 8 + 2 * M::q_of(cl) + (M::e_of(cl) >> 1), im = M::e_of(cl) & 1;
 #pragma unroll
         for (int ks = 0; ks < KS; ks++) {
-            const uint32_t k = ks * 4 + (lane >> 4), kk = k % D;
-            const bool kim = k >= (uint32_t)D;
-            const float2 u = mat[rr * D + kk];
-            ra[i][ks] = rim == kim ? u.x : (rim ? u.y : -u.y);
+            const uint32_t k = 4 * ks + q;
+            const T2 u = mat[jr * D + (k >> 1)];
+            ra[ks] = (k & 1) == im ? u.x : (im ? u.y : -u.y);
         }
     }
-    if (tid < (uint32_t)D) offs[tid] = d.offsets[tid];
-    uint64_t blk = blockIdx.x;
-    if (blk >= blocks) return;
-    uint32_t cur = 0;
-    bases(blk, colbase);
-    __syncthreads();
-    float2 pre[PER];
+    // Staging order: element e of a block takes its index bits in ascending
+    // order of the qubits they stand for (targets, and the lowest free qubits
+    // that the columns of a block span), so neighbouring threads load
+    // neighbouring amplitudes whichever qubits the targets are. `tq` and `fq`
+    // walk both sets; a free bit past the last qubit is a column past the
+    // last one.
+    uint32_t tbits[K + CB];  // bit i of e: index bit (below K) or K + column bit
+    {
+        uint32_t f = 0, fq = 0, ins = 0;  // next column bit, its qubit, the inserted (target or control) qubits passed
+        uint32_t used = 0;                // targets taken
+        for (int i = 0; i < K + CB; i++) {
+            while (ins < d.nins && d.ins[ins] <= fq) {  // fq: the next qubit that is no target or control
+                if (d.ins[ins] == fq) fq++;
+                ins++;
+            }
+            uint32_t lowest = 0;
+            uint64_t lo = ~uint64_t(0);
 #pragma unroll
-    for (int i = 0; i < PER; i++) {
-        uint32_t j, c;
-        elem(tid + i * 64 * WAVES, j, c);
-        const uint64_t b = colbase[c];
-        pre[i] = b != ~uint64_t(0) ? s[b + offs[j]] : make_float2(0.0f, 0.0f);
-    }
-    for (;;) {
-        __syncthreads();  // the previous block's output has been stored
-#pragma unroll
-        for (int i = 0; i < PER; i++) {
-            uint32_t j, c;
-            elem(tid + i * 64 * WAVES, j, c);
-            Br[j * PAD + c] = pre[i].x;
-            Bi[j * PAD + c] = pre[i].y;
-        }
-        const uint64_t next = blk + gridDim.x;
-        if (next < blocks) bases(next, colbase + (cur ^ 1) * NC);
-        __syncthreads();
-        // The next block's loads fly while the matrix cores work.
-        if (next < blocks) {
-            const uint64_t *nb = colbase + (cur ^ 1) * NC;
-#pragma unroll
-            for (int i = 0; i < PER; i++) {
-                uint32_t j, c;
-                elem(tid + i * 64 * WAVES, j, c);
-                const uint64_t b = nb[c];
-                pre[i] = b != ~uint64_t(0) ? s[b + offs[j]] : make_float2(0.0f, 0.0f);
+            for (int t = 0; t < K; t++)
+                if (!((used >> t) & 1) && d.offsets[1 << t] < lo) {
+                    lo = d.offsets[1 << t];
+                    lowest = t;
+                }
+            if (f < (uint32_t)CB && (used == (1u << K) - 1 || (uint64_t(1) << fq) < lo)) {
+                tbits[i] = K + f++;
+                fq++;
+            } else {
+                tbits[i] = lowest;
+                used |= 1u << lowest;
             }
         }
-        floatx4 acc[MPW][NC / 16];
+    }
+    uint64_t eo[PER];           // offset of each staged amplitude within its column
+    uint32_t ec[PER], ea[PER];  // its column in the block, its place in the buffer
 #pragma unroll
-        for (int i = 0; i < MPW; i++)
+    for (int i = 0; i < PER; i++) {
+        const uint32_t e = tid + i * THREADS;
+        uint32_t jc = 0;
+        for (int b = 0; b < K + CB; b++) jc |= ((e >> b) & 1) << tbits[b];
+        const uint32_t j = jc & (D - 1);
+        ec[i] = jc >> K;
+        ea[i] = j * PITCH + ec[i];
+        eo[i] = d.offsets[j];
+    }
+    const uint64_t so0 = d.offsets[wave * 8 + 2 * q], so1 = d.offsets[wave * 8 + 2 * q + 1];
+
+    // Qubit 0 is matrix bit 0: a lane's two amplitudes are neighbours, the
+    // first at an even index (16-byte aligned in complex64).
+    const bool adjacent = d.offsets[1] == 1;
+
+    bases(blk, 0);
+    bases(blk + step, 1);
+    __syncthreads();
+    T2 pre[PER];
+    auto fetch = [&](uint32_t slot) {
 #pragma unroll
-            for (int g = 0; g < NC / 16; g++) acc[i][g] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
+        for (int i = 0; i < PER; i++) {
+            const uint64_t b = colbase[slot * NC + ec[i]];
+            pre[i].x = pre[i].y = 0;
+            if (b != NONE) pre[i] = s[b + eo[i]];
+        }
+    };
+    fetch(0);
+#pragma unroll
+    for (int i = 0; i < PER; i++) buf[ea[i]] = pre[i];
+    __syncthreads();
+    uint32_t cur = 0, slot = 0;
+    for (;;) {
+        const uint64_t next = blk + step;
+        const bool more = next < blocks;
+        const uint32_t slot1 = slot + 1 == SLOTS ? 0 : slot + 1, slot2 = slot1 + 1 == SLOTS ? 0 : slot1 + 1;
+        if (more) fetch(slot1);
+        bases(next + step, slot2);
+        const T2 *const cb = buf + cur * (D * PITCH);
+        const R *const bp = reinterpret_cast<const R *>(cb + (q >> 1) * PITCH + cl) + (q & 1);
+        V acc[NC / 16];
+#pragma unroll
+        for (int g = 0; g < NC / 16; g++) acc[g] = V{0, 0, 0, 0};
 #pragma unroll
         for (int ks = 0; ks < KS; ks++) {
-            const uint32_t k = ks * 4 + (lane >> 4);
-            const float *row = k < (uint32_t)D ? Br + k * PAD : Bi + (k - D) * PAD;
-            float b[NC / 16];
 #pragma unroll
-            for (int g = 0; g < NC / 16; g++) b[g] = row[g * 16 + (lane & 15)];
-#pragma unroll
-            for (int i = 0; i < MPW; i++)
-#pragma unroll
-                for (int g = 0; g < NC / 16; g++)
-                    acc[i][g] = __builtin_amdgcn_mfma_f32_16x16x4f32(ra[i][ks], b[g], acc[i][g], 0, 0, 0);
+            for (int g = 0; g < NC / 16; g++) acc[g] = M::mul(ra[ks], bp[2 * (2 * ks * PITCH + 16 * g)], acc[g]);
         }
-        __syncthreads();  // every wave has read Br / Bi
-        // Accumulator element e of lane l: row 4 * (l / 16) + e, column l % 16.
 #pragma unroll
-        for (int i = 0; i < MPW; i++)
-#pragma unroll
-            for (int g = 0; g < NC / 16; g++)
-#pragma unroll
-                for (int e = 0; e < 4; e++) {
-                    const uint32_t row = (wave * MPW + i) * 16 + 4 * (lane >> 4) + e;
-                    const uint32_t c = g * 16 + (lane & 15);
-                    if (row < (uint32_t)D) Br[row * PAD + c] = acc[i][g][e];
-                    else Bi[(row - D) * PAD + c] = acc[i][g][e];
+        for (int g = 0; g < NC / 16; g++) {
+            const uint64_t b = colbase[slot * NC + 16 * g + cl];
+            if (b != NONE) {
+                T2 o0, o1;
+                o0.x = acc[g][0];
+                o0.y = acc[g][1];
+                o1.x = acc[g][2];
+                o1.y = acc[g][3];
+                if (sizeof(T2) == 8 && adjacent) {
+                    *reinterpret_cast<float4 *>(s + b + so0) = make_float4(o0.x, o0.y, o1.x, o1.y);
+                } else {
+                    s[b + so0] = o0;
+                    s[b + so1] = o1;
                 }
-        __syncthreads();
-        const uint64_t *cb = colbase + cur * NC;
-        for (uint32_t e = tid; e < (uint32_t)(D * NC); e += 64 * WAVES) {
-            uint32_t j, c;
-            elem(e, j, c);
-            const uint64_t b = cb[c];
-            if (b != ~uint64_t(0)) s[b + offs[j]] = make_float2(Br[j * PAD + c], Bi[j * PAD + c]);
+            }
         }
-        if (next >= blocks) break;
-        blk = next;
+        if (!more) break;
+        T2 *const nb = buf + (cur ^ 1) * (D * PITCH);
+#pragma unroll
+        for (int i = 0; i < PER; i++) nb[ea[i]] = pre[i];
+        __syncthreads();
         cur ^= 1;
+        slot = slot1;
+        blk = next;
     }
 }
 
-template <int K, int WAVES>
-hipError_t launch_k(float2 *s, const GateDesc &d, const float2 *mat, unsigned grid, hipStream_t st) {
-    constexpr int D = 1 << K;
-    const size_t lds = (size_t)(2 * D * PAD) * sizeof(float) + (2 * NC + D) * sizeof(uint64_t);
+template <typename T2, int K>
+hipError_t launch_k(T2 *s, const GateDesc &d, const T2 *mat, unsigned cus, hipStream_t st) {
+    constexpr size_t lds = mfma_lds_bytes<T2, K>();
     static std::atomic<uint64_t> attr_set{0};
     int dev = 0;
     hipError_t e = hipGetDevice(&dev);
     if (e != hipSuccess) return e;
     const uint64_t bit = uint64_t(1) << (dev & 63);
     if (!(attr_set.load() & bit)) {
-        e = hipFuncSetAttribute((const void *)k_dense_mfma<K, WAVES>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+        e = hipFuncSetAttribute((const void *)k_dense_mfma<T2, K>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
         if (e != hipSuccess) return e;
         attr_set.fetch_or(bit);
     }
-    k_dense_mfma<K, WAVES><<<grid, 64 * WAVES, lds, st>>>(s, d, mat);
+    const uint64_t blocks = (d.iterations + NC - 1) / NC;
+    const unsigned grid = (unsigned)std::min<uint64_t>(blocks, (uint64_t)cus * (K == 6 ? 2 : K == 5 ? 12 : 32));
+    k_dense_mfma<T2, K><<<grid, 64 << (K - 3), lds, st>>>(s, d, mat);
     return hipGetLastError();
 }
 
 }  // namespace
 
-hipError_t launch_dense_mfma(float2 *s, const GateDesc &d, const float2 *mat, unsigned cus, hipStream_t st) {
-    const uint64_t blocks = (d.iterations + NC - 1) / NC;
-    const unsigned grid = (unsigned)std::min<uint64_t>(blocks, (uint64_t)cus * 12);
-    if (d.k == 5) return launch_k<5, 4>(s, d, mat, grid, st);
-    if (d.k == 6) return launch_k<6, 8>(s, d, mat, grid, st);
+template <typename T2>
+hipError_t launch_dense_mfma(T2 *s, const GateDesc &d, const T2 *mat, unsigned cus, hipStream_t st) {
+    if (d.k == 3) return launch_k<T2, 3>(s, d, mat, cus, st);
+    if (d.k == 4) return launch_k<T2, 4>(s, d, mat, cus, st);
+    if (d.k == 5) return launch_k<T2, 5>(s, d, mat, cus, st);
+    if (d.k == 6) return launch_k<T2, 6>(s, d, mat, cus, st);
     return hipErrorInvalidValue;
 }
+template hipError_t launch_dense_mfma<float2>(float2 *, const GateDesc &, const float2 *, unsigned, hipStream_t);
+template hipError_t launch_dense_mfma<double2>(double2 *, const GateDesc &, const double2 *, unsigned, hipStream_t);
 
 }  // namespace qvd

@@ -15,6 +15,13 @@
 #include "device.h"
 #include "kernels.h"
 
+// Constant address space: uniform loads through these pointers are scalar.
+#if defined(__HIP_DEVICE_COMPILE__)
+#define QVD_CONST __attribute__((address_space(4)))
+#else
+#define QVD_CONST
+#endif
+
 namespace qvd {
 
 // ---------------------------------------------------------------------------
@@ -124,28 +131,33 @@ __global__ void k_scale(T2 *__restrict__ s, uint64_t len, double factor) {
 // ---------------------------------------------------------------------------
 
 // A dense op on K targets: each thread owns one group of 2^K amplitudes
-// (the iteration index spread over the non-target, non-control bits).
+// (the iteration index spread over the non-target, non-control bits). The
+// matrix is the same for every thread: its rows come through the scalar
+// cache and enter the FMAs as scalar operands, so a pass is bound by memory up
+// to K = 4 (28 qubits, targets 4-7: 0.82 ms in complex64 and 1.60 ms in
+// complex128, a copy of the state taking 0.79 and 1.58; read from LDS, each
+// element per FMA pair, the matrix bound it at 1.72 and 7.9 ms).
 template <typename T2, int K>
 __global__ __launch_bounds__(256) void k_dense(T2 *__restrict__ s, const GateDesc d, const T2 *__restrict__ mat) {
     constexpr int D = 1 << K;
-    extern __shared__ unsigned char smem_raw[];
-    T2 *m = reinterpret_cast<T2 *>(smem_raw);
-    for (int i = threadIdx.x; i < D * D; i += blockDim.x) m[i] = mat[i];
-    __syncthreads();
+    const QVD_CONST T2 *const m = (const QVD_CONST T2 *)mat;
     const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
     for (uint64_t it = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; it < d.iterations; it += stride) {
-        const uint64_t base = insert_zeros(it, d.ins, d.nins) | d.ctrl_val;
+        T2 *const g = s + (insert_zeros(it, d.ins, d.nins) | d.ctrl_val);
         T2 a[D];
 #pragma unroll
-        for (int j = 0; j < D; j++) a[j] = s[base + d.offsets[j]];
-#pragma unroll
+        for (int j = 0; j < D; j++) a[j] = g[d.offsets[j]];
+        // One row at a time from K = 3 on: unrolled, the compiler loads the
+        // whole matrix ahead and spills it.
+        constexpr int U = K < 3 ? D : 1;
+#pragma unroll U
         for (int r = 0; r < D; r++) {
             T2 acc;
             acc.x = 0;
             acc.y = 0;
 #pragma unroll
-            for (int c = 0; c < D; c++) cmac(acc, m[r * D + c], a[c]);
-            s[base + d.offsets[r]] = acc;
+            for (int c = 0; c < D; c++) cmac(acc, (T2)m[r * D + c], a[c]);
+            g[d.offsets[r]] = acc;
         }
     }
 }
@@ -1079,15 +1091,14 @@ void launch_scale(T2 *s, uint64_t len, double factor, hipStream_t st) {
 
 template <typename T2>
 void launch_dense(T2 *s, const GateDesc &d, const T2 *mat, hipStream_t st) {
-    const size_t lds = sizeof(T2) << (2 * d.k);
     const unsigned grid = grid_for(d.iterations, 256, 65536);
     switch (d.k) {
-        case 1: k_dense<T2, 1><<<grid, 256, lds, st>>>(s, d, mat); break;
-        case 2: k_dense<T2, 2><<<grid, 256, lds, st>>>(s, d, mat); break;
-        case 3: k_dense<T2, 3><<<grid, 256, lds, st>>>(s, d, mat); break;
-        case 4: k_dense<T2, 4><<<grid, 256, lds, st>>>(s, d, mat); break;
-        case 5: k_dense<T2, 5><<<grid, 256, lds, st>>>(s, d, mat); break;
-        case 6: k_dense<T2, 6><<<grid, 256, lds, st>>>(s, d, mat); break;
+        case 1: k_dense<T2, 1><<<grid, 256, 0, st>>>(s, d, mat); break;
+        case 2: k_dense<T2, 2><<<grid, 256, 0, st>>>(s, d, mat); break;
+        case 3: k_dense<T2, 3><<<grid, 256, 0, st>>>(s, d, mat); break;
+        case 4: k_dense<T2, 4><<<grid, 256, 0, st>>>(s, d, mat); break;
+        case 5: k_dense<T2, 5><<<grid, 256, 0, st>>>(s, d, mat); break;
+        case 6: k_dense<T2, 6><<<grid, 256, 0, st>>>(s, d, mat); break;
         default: break;
     }
 }
