@@ -8,7 +8,7 @@
 
 namespace qvd {
 
-// One pass of a dense op with d.k = 5 or 6 targets over the controlled
+// One pass of a dense op with d.k = 5 or 6 (complex128: 3 to 6) targets over the controlled
 // subspace (same descriptor as launch_dense); mat is the 2^k x 2^k matrix,
 // row-major, in device memory. cus = compute units (grid size).
 template <typename T2>

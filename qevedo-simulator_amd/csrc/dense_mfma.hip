@@ -1,15 +1,18 @@
-// Fused dense gates of K = 3 to 6 targets, applied as real GEMMs on matrix
-// cores: complex64 through v_mfma_f32_16x16x4f32, complex128 through
-// v_mfma_f64_16x16x4f64 (accumulation in the state's precision).
+// Fused dense gates, applied as real GEMMs on matrix cores: complex64 with
+// K = 5 or 6 targets through v_mfma_f32_16x16x4f32, complex128 with 3 to 6
+// through v_mfma_f64_16x16x4f64 (accumulation in the state's precision).
 //
 // A column is one group of D = 2^K amplitudes the gate mixes (the iteration
 // index spread over the non-target, non-control bits, as in k_dense). With
 // U = Ur + i Ui the output's parts are real dot products of the column's
 // parts with the rows of a 2D x 2D real matrix R, so a block of NC columns is
-// the product (2D x 2D) x (2D x NC). R's rows and columns interleave the real
-// and imaginary part of each index, so that the four accumulators of a lane
+// the product (2D x 2D) x (2D x NC). R's rows interleave the real and
+// imaginary part of each index, so that the four accumulators of a lane
 // are two whole amplitudes of one column: they go to memory straight from
 // the accumulators, 16 neighbouring columns (128 or 256 bytes) at a time.
+// The sums run over the real parts of the column and then the imaginary ones
+// in complex64 (the staged block holds them as two planes), over both
+// parts of each index in turn in complex128.
 //
 // A workgroup has one wave per 16 rows of R (8 for K = 6, 1 for K = 3); each
 // wave keeps its rows in registers for the whole launch. Blocks of NC columns
@@ -71,7 +74,11 @@ template <> struct Mfma<double2> {
 constexpr int NC = 32;         // columns per block
 constexpr int CB = 5;          // column bits of a block
 static_assert(NC == 1 << CB, "a block's columns are all values of its column bits");
-constexpr int PITCH = NC + 1;  // row pitch of a staged block (amplitudes)
+// Row pitch of a staged block: amplitudes in complex128; in complex64 floats
+// of a plane, a multiple of 16 but not of 32, so that the four rows a
+// wave reads at once (16 columns each) lie in different banks.
+template <typename T2> constexpr int PITCH = sizeof(T2) == 8 ? NC + 16 : NC + 1;
+template <typename T2, int K> constexpr int BLOCK = (1 << K) * PITCH<T2>;  // amplitudes of one staged block
 constexpr int SLOTS = 3;       // column bases of the block multiplied, loaded and prepared
 
 __device__ __forceinline__ uint64_t spread(uint64_t x, const uint32_t *pos, uint32_t m) {
@@ -85,7 +92,7 @@ __device__ __forceinline__ uint64_t spread(uint64_t x, const uint32_t *pos, uint
 
 template <typename T2, int K>
 constexpr size_t mfma_lds_bytes() {
-    return 2 * sizeof(T2) * (size_t(1) << K) * PITCH + SLOTS * NC * sizeof(uint64_t);
+    return 2 * sizeof(T2) * (size_t)BLOCK<T2, K> + SLOTS * NC * sizeof(uint64_t);
 }
 
 template <typename T2, int K>
@@ -99,8 +106,8 @@ __global__ __launch_bounds__(64 << (K - 3)) void k_dense_mfma(T2 *__restrict__ s
     constexpr int PER = D * NC / THREADS;       // amplitudes staged per thread
     constexpr uint64_t NONE = ~uint64_t(0);     // a column past the last one
     extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
-    T2 *const buf = reinterpret_cast<T2 *>(smem_raw);                       // 2 x D x PITCH
-    uint64_t *const colbase = reinterpret_cast<uint64_t *>(buf + 2 * D * PITCH);  // SLOTS x NC
+    T2 *const buf = reinterpret_cast<T2 *>(smem_raw);                       // two blocks
+    uint64_t *const colbase = reinterpret_cast<uint64_t *>(buf + 2 * BLOCK<T2, K>);  // SLOTS x NC
     const uint32_t tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, q = lane >> 4, cl = lane & 15;
     const uint64_t blocks = (d.iterations + NC - 1) / NC;
     uint64_t blk = blockIdx.x;
@@ -113,17 +120,19 @@ __global__ __launch_bounds__(64 << (K - 3)) void k_dense_mfma(T2 *__restrict__ s
         }
     };
 
-    // This wave's rows of R. Row (and column) indices pair up as (index of
-    // U, part): the lane's accumulators e are index 2q + e / 2 of the wave's
-    // 8 and part e % 2, and k = 4 ks + q is index k / 2, part k % 2.
+    // This wave's rows of R. Row indices pair up as (index of U, part): the
+    // lane's accumulators e are index 2q + e / 2 of the wave's 8 and part
+    // e % 2. k = 4 ks + q is index k % D, part k / D in complex64, index k / 2,
+    // part k % 2 in complex128.
+    constexpr bool PLANES = sizeof(T2) == 8;
     R ra[KS];
     {
         const uint32_t jr = wave * 8 + 2 * M::q_of(cl) + (M::e_of(cl) >> 1), im = M::e_of(cl) & 1;
 #pragma unroll
         for (int ks = 0; ks < KS; ks++) {
             const uint32_t k = 4 * ks + q;
-            const T2 u = mat[jr * D + (k >> 1)];
-            ra[ks] = (k & 1) == im ? u.x : (im ? u.y : -u.y);
+            const T2 u = mat[jr * D + (PLANES ? k & (D - 1) : k >> 1)];
+            ra[ks] = (PLANES ? k >> K : k & 1) == im ? u.x : (im ? u.y : -u.y);
         }
     }
     // Staging order: element e of a block takes its index bits in ascending
@@ -167,7 +176,7 @@ __global__ __launch_bounds__(64 << (K - 3)) void k_dense_mfma(T2 *__restrict__ s
         for (int b = 0; b < K + CB; b++) jc |= ((e >> b) & 1) << tbits[b];
         const uint32_t j = jc & (D - 1);
         ec[i] = jc >> K;
-        ea[i] = j * PITCH + ec[i];
+        ea[i] = j * PITCH<T2> + ec[i];
         eo[i] = d.offsets[j];
     }
     const uint64_t so0 = d.offsets[wave * 8 + 2 * q], so1 = d.offsets[wave * 8 + 2 * q + 1];
@@ -188,9 +197,21 @@ __global__ __launch_bounds__(64 << (K - 3)) void k_dense_mfma(T2 *__restrict__ s
             if (b != NONE) pre[i] = s[b + eo[i]];
         }
     };
-    fetch(0);
+    auto stage = [&](T2 *b) {
+        if constexpr (PLANES) {
+            R *const f = reinterpret_cast<R *>(b);
 #pragma unroll
-    for (int i = 0; i < PER; i++) buf[ea[i]] = pre[i];
+            for (int i = 0; i < PER; i++) {
+                f[ea[i]] = pre[i].x;
+                f[BLOCK<T2, K> + ea[i]] = pre[i].y;
+            }
+        } else {
+#pragma unroll
+            for (int i = 0; i < PER; i++) b[ea[i]] = pre[i];
+        }
+    };
+    fetch(0);
+    stage(buf);
     __syncthreads();
     uint32_t cur = 0, slot = 0;
     for (;;) {
@@ -199,15 +220,18 @@ __global__ __launch_bounds__(64 << (K - 3)) void k_dense_mfma(T2 *__restrict__ s
         const uint32_t slot1 = slot + 1 == SLOTS ? 0 : slot + 1, slot2 = slot1 + 1 == SLOTS ? 0 : slot1 + 1;
         if (more) fetch(slot1);
         bases(next + step, slot2);
-        const T2 *const cb = buf + cur * (D * PITCH);
-        const R *const bp = reinterpret_cast<const R *>(cb + (q >> 1) * PITCH + cl) + (q & 1);
+        const R *const cb = reinterpret_cast<const R *>(buf + cur * BLOCK<T2, K>);
+        const R *const bp = PLANES ? cb + q * PITCH<T2> + cl : cb + 2 * ((q >> 1) * PITCH<T2> + cl) + (q & 1);
+        // k step ks from bp: 4 rows of a plane (the second plane follows the
+        // first), or 2 rows of amplitudes.
+        constexpr int STEP = 4 * PITCH<T2>, COL = PLANES ? 1 : 2;
         V acc[NC / 16];
 #pragma unroll
         for (int g = 0; g < NC / 16; g++) acc[g] = V{0, 0, 0, 0};
 #pragma unroll
         for (int ks = 0; ks < KS; ks++) {
 #pragma unroll
-            for (int g = 0; g < NC / 16; g++) acc[g] = M::mul(ra[ks], bp[2 * (2 * ks * PITCH + 16 * g)], acc[g]);
+            for (int g = 0; g < NC / 16; g++) acc[g] = M::mul(ra[ks], bp[ks * STEP + COL * 16 * g], acc[g]);
         }
 #pragma unroll
         for (int g = 0; g < NC / 16; g++) {
@@ -227,9 +251,7 @@ __global__ __launch_bounds__(64 << (K - 3)) void k_dense_mfma(T2 *__restrict__ s
             }
         }
         if (!more) break;
-        T2 *const nb = buf + (cur ^ 1) * (D * PITCH);
-#pragma unroll
-        for (int i = 0; i < PER; i++) nb[ea[i]] = pre[i];
+        stage(buf + (cur ^ 1) * BLOCK<T2, K>);
         __syncthreads();
         cur ^= 1;
         slot = slot1;
@@ -260,8 +282,10 @@ hipError_t launch_k(T2 *s, const GateDesc &d, const T2 *mat, unsigned cus, hipSt
 
 template <typename T2>
 hipError_t launch_dense_mfma(T2 *s, const GateDesc &d, const T2 *mat, unsigned cus, hipStream_t st) {
-    if (d.k == 3) return launch_k<T2, 3>(s, d, mat, cus, st);
-    if (d.k == 4) return launch_k<T2, 4>(s, d, mat, cus, st);
+    if constexpr (sizeof(T2) == 16) {
+        if (d.k == 3) return launch_k<T2, 3>(s, d, mat, cus, st);
+        if (d.k == 4) return launch_k<T2, 4>(s, d, mat, cus, st);
+    }
     if (d.k == 5) return launch_k<T2, 5>(s, d, mat, cus, st);
     if (d.k == 6) return launch_k<T2, 6>(s, d, mat, cus, st);
     return hipErrorInvalidValue;

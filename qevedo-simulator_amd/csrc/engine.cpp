@@ -352,15 +352,16 @@ void apply_full(qvd_sv *sv, T2 *s, const Op &op, const T2 *coef, bool valu_only 
     }
     d.ctrl_val = cval;
     d.iterations = uint64_t(1) << (sv->n - d.nins);
-    // Matrix cores for 5- and 6-qubit gates, and for 3- and 4-qubit ones with
-    // two or more targets inside a 128-byte line, whose groups k_dense would
-    // load as pieces of a line (28 qubits, targets 0-3: complex64 2.05 ms
-    // against 0.95, complex128 2.63 against 1.76). With at most one target
-    // there k_dense moves whole lines and is ahead (targets 4-7: 0.82 ms
-    // against 0.93, 1.60 against 1.77): it needs no staging through LDS.
+    // Matrix cores for 5- and 6-qubit gates, and in complex128 for 3- and
+    // 4-qubit ones with two or more targets inside a 128-byte line, whose
+    // groups k_dense would load as pieces of a line (28 qubits, targets 0-3:
+    // 2.63 ms against 1.76). With at most one target there k_dense moves whole
+    // lines and is ahead (targets 4-7: 1.60 against 1.77): it needs no
+    // staging through LDS. In complex64 3- and 4-qubit gates keep k_dense
+    // and its order of the FP32 sums.
     uint32_t in_line = 0;
     for (uint32_t t : op.targets) in_line += (sizeof(T2) << t) < 128;
-    if ((k >= 5 || (k >= 3 && in_line >= 2)) && !valu_only) {
+    if ((k >= 5 || (sizeof(T2) == 16 && k >= 3 && in_line >= 2)) && !valu_only) {
         QVD_HIP(launch_dense_mfma<T2>(s, d, coef, (unsigned)num_cus(sv->device), sv->stream));
         return;
     }
