@@ -1169,7 +1169,7 @@ void build_batch(qvd_batch *b, const qvd_circuit *circuits, uint32_t count, cons
         if (steps.empty() || stale) b->init_states = true;
         b->gates += ci.num_ops;
         ExpDesc &e = ed[c];
-        e = expect_desc(npad, ci.num_qubits);
+        e = expect_desc(npad, ci.num_qubits, expect_batch_segment_bits(npad));
         e.state_off = off;
         e.seg_off = seg_off;
         e.z_off = (uint32_t)b->num_z;
@@ -1285,7 +1285,7 @@ void build_batch(qvd_batch *b, const qvd_circuit *circuits, uint32_t count, cons
                                             b->ldsops.as<StageOp>(), b->ints.as<uint32_t>(), b->grid, b->stream));
         launch_expect_batch<T2>(s, b->edescs.as<ExpDesc>(), count, b->seg_start.as<uint64_t>(), seg_start[count],
                                 b->out_start.as<uint32_t>(), out_start[count], b->seg_sums.as<double>(),
-                                b->z.as<double>(), b->zz.as<double>(), b->stream);
+                                b->z.as<double>(), b->zz.as<double>(), ed[0], b->stream);
         QVD_HIP(hipGetLastError());
     };
     enqueue();
@@ -1851,14 +1851,13 @@ int qvd_sv_norm_sqr(const qvd_sv *sv_c, double *out) {
         require(out != nullptr, "null output");
         qvd_sv *sv = const_cast<qvd_sv *>(sv_c);
         sv->bind();
-        const unsigned blocks = 1024;
-        double *buf = sv->scratch_doubles(blocks + 1);
+        double *buf = sv->scratch_doubles(NORM_BLOCKS + 1);
         with_type(sv, [&](auto *s) {
-            launch_masked_norm(s, sv->len, 0, 0, buf, blocks, buf + blocks, sv->stream);
+            launch_norm(s, sv->len, -1, buf, buf + NORM_BLOCKS, sv->stream);
             return 0;
         });
         QVD_HIP(hipGetLastError());
-        QVD_HIP(hipMemcpyAsync(out, buf + blocks, sizeof(double), hipMemcpyDeviceToHost, sv->stream));
+        QVD_HIP(hipMemcpyAsync(out, buf + NORM_BLOCKS, sizeof(double), hipMemcpyDeviceToHost, sv->stream));
         sv->sync();
     });
 }
@@ -1876,18 +1875,22 @@ int qvd_sv_scale(qvd_sv *sv, double factor) {
     });
 }
 
-static double probability_one_impl(qvd_sv *sv, uint32_t qubit) {
+// Queues P(qubit = 1) into device memory (returned).
+static const double *enqueue_probability_one(qvd_sv *sv, uint32_t qubit) {
     require(qubit < sv->n, "qubit " + std::to_string(qubit) + " out of range for " + std::to_string(sv->n) + " qubits");
-    const unsigned blocks = 1024;
-    double *buf = sv->scratch_doubles(blocks + 1);
-    const uint64_t m = uint64_t(1) << qubit;
+    double *buf = sv->scratch_doubles(NORM_BLOCKS + 1);
     with_type(sv, [&](auto *s) {
-        launch_masked_norm(s, sv->len, m, m, buf, blocks, buf + blocks, sv->stream);
+        launch_norm(s, sv->len, (int)qubit, buf, buf + NORM_BLOCKS, sv->stream);
         return 0;
     });
     QVD_HIP(hipGetLastError());
+    return buf + NORM_BLOCKS;
+}
+
+static double probability_one_impl(qvd_sv *sv, uint32_t qubit) {
     double r = 0;
-    QVD_HIP(hipMemcpyAsync(&r, buf + blocks, sizeof(double), hipMemcpyDeviceToHost, sv->stream));
+    const double *p = enqueue_probability_one(sv, qubit);
+    QVD_HIP(hipMemcpyAsync(&r, p, sizeof(double), hipMemcpyDeviceToHost, sv->stream));
     sv->sync();
     return r;
 }
@@ -1937,41 +1940,68 @@ int qvd_sv_expect_pauli(const qvd_sv *sv_c, const uint64_t *x_masks, const uint6
         for (uint64_t t = 0; t < num_terms; t++)
             require(((x_masks[t] | z_masks[t]) & ~all) == 0, "Pauli string acts on a qubit out of range");
         sv->bind();
-        // Terms grouped by their X part: each group of up to PAULI_TERMS
-        // terms is one pass over the state.
+        // Strings grouped by their X part, up to PAULI_TERMS a group, wide
+        // groups first (runs of equal width share a launch); whole groups go
+        // through one upload, launch and copy back per PAULI_CALL strings.
         std::vector<uint64_t> order(num_terms);
         for (uint64_t t = 0; t < num_terms; t++) order[t] = t;
         std::stable_sort(order.begin(), order.end(), [&](uint64_t a, uint64_t b) { return x_masks[a] < x_masks[b]; });
-        const unsigned blocks = 1024;
-        const uint32_t W = 2 * PAULI_TERMS;
-        double *buf = sv->scratch_doubles((size_t)blocks * W + W + PAULI_TERMS);
-        double *partial = buf, *sums = buf + (size_t)blocks * W;
-        uint64_t *dz = reinterpret_cast<uint64_t *>(sums + W);
-        std::vector<uint64_t> zs;
-        std::vector<double> h(W);
+        struct Run { uint64_t at; uint32_t n; };
+        std::vector<Run> runs;
         for (uint64_t g = 0; g < num_terms;) {
-            const uint64_t x = x_masks[order[g]];
-            zs.clear();
             uint64_t e = g;
-            while (e < num_terms && x_masks[order[e]] == x && zs.size() < PAULI_TERMS) zs.push_back(z_masks[order[e++]]);
-            const uint32_t k = (uint32_t)zs.size();
-            QVD_HIP(hipMemcpyAsync(dz, zs.data(), k * sizeof(uint64_t), hipMemcpyHostToDevice, sv->stream));
+            while (e < num_terms && x_masks[order[e]] == x_masks[order[g]] && e - g < PAULI_TERMS) e++;
+            runs.push_back({g, (uint32_t)(e - g)});
+            g = e;
+        }
+        std::stable_sort(runs.begin(), runs.end(), [](const Run &a, const Run &b) { return a.n > b.n; });
+        constexpr uint32_t PAULI_CALL = 4096;
+        std::vector<PauliGroup> groups;
+        std::vector<uint32_t> widths;
+        std::vector<uint64_t> zs, terms;
+        std::vector<double> h;
+        for (size_t r = 0; r < runs.size();) {
+            groups.clear();
+            widths.clear();
+            zs.clear();
+            terms.clear();
+            for (; r < runs.size() && zs.size() + runs[r].n <= PAULI_CALL; r++) {
+                PauliGroup g{x_masks[order[runs[r].at]], (uint32_t)zs.size(), runs[r].n, 0, 0};
+                for (uint32_t t = 0; t < g.nterms; t++) {
+                    const uint64_t idx = order[runs[r].at + t];
+                    zs.push_back(z_masks[idx]);
+                    terms.push_back(idx);
+                    g.odd |= (uint32_t)(__builtin_popcountll(g.x & z_masks[idx]) & 1) << t;
+                }
+                groups.push_back(g);
+                widths.push_back(g.nterms);
+            }
+            const size_t k = zs.size(), gw = sizeof(PauliGroup) / sizeof(double) * groups.size();
+            const unsigned blocks = pauli_blocks(sv->len, (uint32_t)groups.size());
+            std::vector<uint64_t> up(gw + k);
+            std::memcpy(up.data(), groups.data(), groups.size() * sizeof(PauliGroup));
+            std::memcpy(up.data() + gw, zs.data(), k * sizeof(uint64_t));
+            // sums, descriptors and Z parts, then the blocks' partial sums
+            double *buf = sv->scratch_doubles(k + up.size() + k * blocks);
+            uint64_t *dg = reinterpret_cast<uint64_t *>(buf + k);
+            QVD_HIP(hipMemcpyAsync(dg, up.data(), up.size() * sizeof(uint64_t), hipMemcpyHostToDevice, sv->stream));
             with_type(sv, [&](auto *s) {
-                launch_expect_pauli(s, sv->len, x, dz, k, partial, blocks, sums, sv->stream);
+                launch_expect_pauli(s, sv->len, reinterpret_cast<const PauliGroup *>(dg), widths, dg + gw, (uint32_t)k,
+                                    buf + k + up.size(), blocks, buf, sv->stream);
                 return 0;
             });
             QVD_HIP(hipGetLastError());
-            QVD_HIP(hipMemcpyAsync(h.data(), sums, 2 * k * sizeof(double), hipMemcpyDeviceToHost, sv->stream));
+            h.resize(k);
+            QVD_HIP(hipMemcpyAsync(h.data(), buf, k * sizeof(double), hipMemcpyDeviceToHost, sv->stream));
             sv->sync();
-            for (uint32_t t = 0; t < k; t++) {
-                // P = i^popcount(x & z) X^x Z^z; its expectation is real for
-                // a Hermitian string, so only the real part is kept.
-                const uint64_t idx = order[g + t];
+            for (size_t t = 0; t < k; t++) {
+                // P = i^popcount(x & z) X^x Z^z; the sum is over half of the
+                // indices where x != 0.
+                const uint64_t idx = terms[t], x = x_masks[idx];
                 const int ny = __builtin_popcountll(x & z_masks[idx]) & 3;
-                const double re = h[2 * t], im = h[2 * t + 1];
-                out[idx] = ny == 0 ? re : ny == 1 ? -im : ny == 2 ? -re : im;
+                const double v = x ? 2 * h[t] : h[t];
+                out[idx] = ny == 0 || ny == 3 ? v : -v;
             }
-            g = e;
         }
     });
 }
@@ -2002,19 +2032,20 @@ int qvd_sv_expect_z(const qvd_sv *sv_c, double *z, double *zz) {
     });
 }
 
-static uint8_t measure_impl(qvd_sv *sv, uint32_t qubit, double uniform) {
-    double p1 = probability_one_impl(sv, qubit);
-    p1 = std::min(std::max(p1, 0.0), 1.0);
-    const bool outcome = uniform < p1;
-    const double p = outcome ? p1 : 1.0 - p1;
-    const double keep = 1.0 / std::sqrt(p);
+// Measures a qubit (flip: and resets it). The collapse reads P(1) from device
+// memory and comes to the outcome found here.
+static uint8_t measure_impl(qvd_sv *sv, uint32_t qubit, double uniform, bool flip) {
+    double p1 = 0;
+    const double *p = enqueue_probability_one(sv, qubit);
     with_type(sv, [&](auto *s) {
-        launch_collapse(s, sv->len, qubit, outcome ? 1u : 0u, keep, sv->stream);
+        launch_collapse(s, sv->len, qubit, uniform, p, flip, sv->stream);
         return 0;
     });
     QVD_HIP(hipGetLastError());
+    QVD_HIP(hipMemcpyAsync(&p1, p, sizeof(double), hipMemcpyDeviceToHost, sv->stream));
     sv->sync();
-    return outcome ? 1 : 0;
+    p1 = std::min(std::max(p1, 0.0), 1.0);
+    return uniform < p1 ? 1 : 0;
 }
 
 int qvd_sv_measure(qvd_sv *sv, uint32_t qubit, double uniform, uint8_t *outcome) {
@@ -2022,7 +2053,7 @@ int qvd_sv_measure(qvd_sv *sv, uint32_t qubit, double uniform, uint8_t *outcome)
         check_handle(sv);
         require(outcome != nullptr, "null output");
         sv->bind();
-        *outcome = measure_impl(sv, qubit, uniform);
+        *outcome = measure_impl(sv, qubit, uniform, false);
     });
 }
 
@@ -2030,22 +2061,7 @@ int qvd_sv_reset(qvd_sv *sv, uint32_t qubit, double uniform) {
     return guard([&] {
         check_handle(sv);
         sv->bind();
-        if (measure_impl(sv, qubit, uniform)) {
-            Op x;
-            x.targets = {qubit};
-            x.m = HMatrix(1);
-            x.m.at(0, 1) = C64(1, 0);
-            x.m.at(1, 0) = C64(1, 0);
-            x.diagonal = false;
-            with_type(sv, [&](auto *s) {
-                using T2 = std::remove_pointer_t<decltype(s)>;
-                Upload up;
-                const size_t o = up.put(full_coefficients<T2>(x));
-                apply_full(sv, s, x, reinterpret_cast<const T2 *>(up.to_device(sv) + o));
-                sv->sync();
-                return 0;
-            });
-        }
+        (void)measure_impl(sv, qubit, uniform, true);
     });
 }
 

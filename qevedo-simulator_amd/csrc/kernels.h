@@ -5,6 +5,7 @@
 
 #include <cstddef>
 #include <cstdint>
+#include <vector>
 
 #include "device.h"
 
@@ -45,9 +46,21 @@ template <typename T2> void launch_init_zero(T2 *s, uint64_t len, hipStream_t st
 // Zero over every amplitude whose index has a bit of `stale` set.
 template <typename T2> void launch_zero_stale(T2 *s, uint64_t len, uint64_t stale, hipStream_t st);
 template <typename T2> void launch_probabilities(const T2 *s, uint64_t len, double *out, hipStream_t st);
+// Pauli strings [first, first + nterms) share the X part x; bit t of `odd`: the
+// string's sum is of imaginary parts (an odd number of Y).
+struct PauliGroup {
+    uint64_t x;
+    uint32_t first, nterms, odd, pad;
+};
+// Blocks per group for a launch over ngroups groups.
+unsigned pauli_blocks(uint64_t len, uint32_t ngroups);
+// out[t] = string t's sum over half of the indices where x != 0 (the value is
+// twice that), over all where x = 0. widths: the groups' nterms; partial holds
+// nterms * blocks doubles; groups and zs (one per string) are in device memory.
 template <typename T2>
-void launch_expect_pauli(const T2 *s, uint64_t len, uint64_t x, const uint64_t *zs, uint32_t nterms, double *partial,
-                         unsigned blocks, double *out, hipStream_t st);
+void launch_expect_pauli(const T2 *s, uint64_t len, const PauliGroup *groups, const std::vector<uint32_t> &widths,
+                         const uint64_t *zs, uint32_t nterms, double *partial, unsigned blocks, double *out,
+                         hipStream_t st);
 template <typename T2> void launch_widen(const T2 *s, double2 *out, uint64_t count, hipStream_t st);
 template <typename T2> void launch_narrow(const double2 *in, T2 *s, uint64_t count, hipStream_t st);
 template <typename T2> void launch_scale(T2 *s, uint64_t len, double factor, hipStream_t st);
@@ -58,14 +71,17 @@ void launch_diag(T2 *s, uint64_t len, uint32_t k, const DiagTargets &t, uint64_t
 template <typename T2> size_t stage_lds_bytes(uint32_t L);
 template <typename T2>
 void launch_stage(T2 *s, const StageDesc &d, const StageOp *ops, const T2 *coefs, unsigned grid, hipStream_t st);
+// out = the sum of |a|^2 over the state, or over the amplitudes with bit `qubit`
+// set (qubit >= 0); partial holds NORM_BLOCKS doubles.
+constexpr unsigned NORM_BLOCKS = 1024;
 template <typename T2>
-void launch_masked_norm(const T2 *s, uint64_t len, uint64_t mask, uint64_t val, double *partial, unsigned blocks,
-                        double *out, hipStream_t st);
+void launch_norm(const T2 *s, uint64_t len, int qubit, double *partial, double *out, hipStream_t st);
 template <typename TA, typename TB>
 void launch_compare(const TA *a, const TB *b, uint64_t len, double *partial, unsigned blocks, hipStream_t st);
-uint32_t expect_segment_bits(uint32_t n);
-// <Z_q> and <Z_q Z_{q+1}> of one state among several: segment sums over
-// 2^B-amplitude segments, then one combine thread per output value.
+uint32_t expect_segment_bits(uint32_t n);        // a single state's segments
+uint32_t expect_batch_segment_bits(uint32_t n);  // those of a state of a batch
+// <Z_q> and <Z_q Z_{q+1}> of one state among several: sums over
+// 2^B-amplitude segments, then a wave or a block per output value.
 struct ExpDesc {
     uint64_t state_off;  // first amplitude of the state
     uint64_t seg_off;    // first double of its segment sums (2 B per segment)
@@ -74,20 +90,22 @@ struct ExpDesc {
     uint32_t n;          // qubits reported: n values of z, n - 1 of zz
     uint32_t z_off, zz_off;
 };
-ExpDesc expect_desc(uint32_t state_qubits, uint32_t n);
+ExpDesc expect_desc(uint32_t state_qubits, uint32_t n, uint32_t segment_bits);
 template <typename T2>
 void launch_expect_z(const T2 *s, uint32_t n, double *seg_sums, double *z, double *zz, hipStream_t st);
 template <typename T2>
 void launch_expect_batch(const T2 *s, const ExpDesc *descs, uint32_t ndesc, const uint64_t *seg_start,
                          uint64_t total_segs, const uint32_t *out_start, uint32_t total_outs, double *seg_sums,
-                         double *z, double *zz, hipStream_t st);
+                         double *z, double *zz, const ExpDesc &first, hipStream_t st);
 // Zero-fills n 32-bit words with a kernel.
 void launch_zero_words(uint32_t *p, uint32_t n, hipStream_t st);
 // Zero-fills `len` amplitudes and sets amplitude offs[i] to 1 for each state i.
 template <typename T2>
 void launch_batch_init(T2 *s, uint64_t len, const uint64_t *offs, uint32_t count, hipStream_t st);
+// Measures `qubit` given P(1) at p_one (device memory); flip: and resets it.
 template <typename T2>
-void launch_collapse(T2 *s, uint64_t len, uint32_t qubit, uint32_t outcome, double keep, hipStream_t st);
+void launch_collapse(T2 *s, uint64_t len, uint32_t qubit, double uniform, const double *p_one, bool flip,
+                     hipStream_t st);
 size_t sort_temp_bytes(uint64_t shots);
 // Two-pass sampling (src/measure.rs:104-174) in three parts: the chunk sums
 // and their prefix; the uniforms' sort into w.targets (on any stream); then,

@@ -10,6 +10,7 @@
 #include <hip/hip_runtime.h>
 #include <hipcub/hipcub.hpp>
 
+#include <algorithm>
 #include <mutex>
 
 #include "device.h"
@@ -331,33 +332,27 @@ __device__ __forceinline__ double prob(const T2 a) {
     return re * re + im * im;
 }
 
-// Per-block partial sums of |a_i|^2 over amplitudes with (i & mask) == val.
-template <typename T2>
-__global__ __launch_bounds__(RED_THREADS) void k_masked_norm(const T2 *__restrict__ s, uint64_t len, uint64_t mask,
-                                                             uint64_t val, double *__restrict__ partial) {
+// Per-block partial sums of |a_i|^2: over all amplitudes, or (HALF) over those
+// whose index has bit `qubit` set, which are the only ones it visits.
+template <typename T2, bool HALF>
+__global__ __launch_bounds__(RED_THREADS) void k_norm(const T2 *__restrict__ s, uint64_t count, uint32_t qubit,
+                                                      double *__restrict__ partial) {
     __shared__ double scratch[RED_THREADS / 64];
     double acc = 0;
     const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
     uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    // U loads in flight per thread, summed in index order. An amplitude
-    // outside the mask adds +0.0, which leaves the sum (never -0.0) as it is;
-    // its load re-reads the batch's first address (cached) instead, so the
-    // loads need no branch, which would wait for each of them.
+    const uint64_t bit = HALF ? uint64_t(1) << qubit : 0;
+    auto at = [&](uint64_t it) { return HALF ? ((it & ~(bit - 1)) << 1) | bit | (it & (bit - 1)) : it; };
+    // U loads in flight per thread, summed in index order.
     constexpr int U = 8;
-    for (; i + (U - 1) * stride < len; i += U * stride) {
+    for (; i + (U - 1) * stride < count; i += U * stride) {
         T2 a[U];
-        bool in[U];
 #pragma unroll
-        for (int u = 0; u < U; u++) {
-            const uint64_t k = i + u * stride;
-            in[u] = (k & mask) == val;
-            a[u] = s[in[u] ? k : i];
-        }
+        for (int u = 0; u < U; u++) a[u] = s[at(i + u * stride)];
 #pragma unroll
-        for (int u = 0; u < U; u++) acc += in[u] ? prob(a[u]) : 0.0;
+        for (int u = 0; u < U; u++) acc += prob(a[u]);
     }
-    for (; i < len; i += stride)
-        if ((i & mask) == val) acc += prob(s[i]);
+    for (; i < count; i += stride) acc += prob(s[at(i)]);
     const double r = block_sum(acc, scratch);
     if (threadIdx.x == 0) partial[blockIdx.x] = r;
 }
@@ -369,79 +364,87 @@ __global__ void k_probabilities(const T2 *__restrict__ s, uint64_t len, double *
     for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < len; i += stride) out[i] = prob(s[i]);
 }
 
-// Pauli strings sharing one X part x (qubits with X or Y) and differing in
-// their Z parts z[t] (qubits with Z or Y): per block, the sums over j of
-// (-1)^popcount((j ^ x) & z[t]) conj(a_j) a_(j ^ x), real and imaginary
-// parts in FP64, written to partial[block * 2 * nterms + 2 t (+1)]. With the
-// phase i^popcount(x & z[t]) applied afterwards this is <P_t>. KT >= nterms
-// slots are computed (a power of two, so a group of few terms does not pay
-// for PAULI_TERMS).
+// Pauli strings in groups that share one X part x (qubits with X or Y) and
+// differ in their Z parts z[t] (qubits with Z or Y); blockIdx.y names the
+// group. With v_j = conj(a_j) a_(j ^ x), a string's value is
+// i^popcount(x & z) times the sum over j of (-1)^popcount((j ^ x) & z) v_j. The
+// terms of j and j ^ x differ only in the sign of the part that the factor i^..
+// makes imaginary: the other part counts twice and that one cancels. So for
+// x != 0 only the j without x's highest bit are visited, each amplitude is
+// read once, and only the part that stays is summed: the imaginary one where
+// popcount(x & z) is odd. Per block and string the sum goes to
+// partial[string * blocks + block]. KT >= a group's strings (a power of two, so
+// a group of few strings does not pay for PAULI_TERMS).
+//
+// Bound by memory (one read of the state per group): 30 qubits in complex64,
+// one string 1.6 ms; reading both amplitudes of every j and summing both
+// parts took 2.8 ms for a string with X on every qubit.
 template <typename T2, int KT>
-__global__ __launch_bounds__(RED_THREADS) void k_expect_pauli(const T2 *__restrict__ s, uint64_t len, uint64_t x,
-                                                              const uint64_t *__restrict__ zs, uint32_t nterms,
+__global__ __launch_bounds__(RED_THREADS) void k_expect_pauli(const T2 *__restrict__ s, uint64_t len,
+                                                              const PauliGroup *__restrict__ groups,
+                                                              const uint64_t *__restrict__ zs,
                                                               double *__restrict__ partial) {
     __shared__ double scratch[RED_THREADS / 64];
-    double re[KT], im[KT];
+    const PauliGroup g = groups[blockIdx.y];
+    double sum[KT];
     uint64_t z[KT];
 #pragma unroll
     for (int t = 0; t < KT; t++) {
-        re[t] = im[t] = 0;
-        z[t] = t < (int)nterms ? zs[t] : 0;
+        sum[t] = 0;
+        z[t] = t < (int)g.nterms ? zs[g.first + t] : 0;
     }
+    const uint64_t x = g.x;
+    const uint64_t top = x ? uint64_t(1) << (63 - __builtin_clzll(x)) : 0;
+    const uint64_t count = x ? len >> 1 : len;
+    const uint64_t low = x ? top - 1 : ~uint64_t(0);
     const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
+    auto index = [&](uint64_t it) { return (it & low) | ((it & ~low) << 1); };
     auto add = [&](uint64_t j, const T2 a, const T2 b) {
         const double ar = a.x, ai = a.y, br = b.x, bi = b.y;
         const double vr = ar * br + ai * bi, vi = ar * bi - ai * br;  // conj(a) b
         const uint64_t k = j ^ x;
 #pragma unroll
         for (int t = 0; t < KT; t++) {  // every slot: unused ones have z = 0 and are not written
-            const bool neg = __popcll(k & z[t]) & 1;
-            re[t] += neg ? -vr : vr;
-            im[t] += neg ? -vi : vi;
+            const double v = (g.odd >> t) & 1 ? vi : vr;
+            sum[t] += (__popcll(k & z[t]) & 1) ? -v : v;
         }
     };
     // U iterations' loads in flight per thread, summed in index order.
     constexpr int U = 4;
-    uint64_t j = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    for (; j + (U - 1) * stride < len; j += U * stride) {
+    uint64_t it = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    for (; it + (U - 1) * stride < count; it += U * stride) {
         T2 a[U], b[U];
 #pragma unroll
         for (int u = 0; u < U; u++) {
-            a[u] = s[j + u * stride];
-            b[u] = s[(j + u * stride) ^ x];
+            const uint64_t j = index(it + u * stride);
+            a[u] = s[j];
+            b[u] = s[j ^ x];
         }
 #pragma unroll
-        for (int u = 0; u < U; u++) add(j + u * stride, a[u], b[u]);
+        for (int u = 0; u < U; u++) add(index(it + u * stride), a[u], b[u]);
     }
-    for (; j < len; j += stride) add(j, s[j], s[j ^ x]);
+    for (; it < count; it += stride) {
+        const uint64_t j = index(it);
+        add(j, s[j], s[j ^ x]);
+    }
 #pragma unroll
     for (int t = 0; t < KT; t++) {
-        const double r = block_sum(re[t], scratch);
-        const double i = block_sum(im[t], scratch);
-        if (threadIdx.x == 0 && t < (int)nterms) {
-            partial[(uint64_t)blockIdx.x * 2 * nterms + 2 * t] = r;
-            partial[(uint64_t)blockIdx.x * 2 * nterms + 2 * t + 1] = i;
-        }
+        const double r = block_sum(sum[t], scratch);
+        if (threadIdx.x == 0 && t < (int)g.nterms) partial[(uint64_t)(g.first + t) * gridDim.x + blockIdx.x] = r;
     }
 }
 
-// out[v] = sum over blocks b, in block order, of partial[b * width + v].
-__global__ void k_sum_columns(const double *__restrict__ partial, uint32_t blocks, uint32_t width,
-                              double *__restrict__ out) {
-    const uint32_t v = blockIdx.x * blockDim.x + threadIdx.x;
-    if (v >= width) return;
+// out[v] = the sum of row v of partial[rows][m], one block per row: a thread
+// per value where one walks them in order costs a memory round trip per few
+// values (1024 partial sums: 66 to 90 us, this 3).
+__global__ __launch_bounds__(RED_THREADS) void k_sum_rows(const double *__restrict__ partial, uint32_t m,
+                                                          double *__restrict__ out) {
+    __shared__ double scratch[RED_THREADS / 64];
+    const double *const row = partial + (uint64_t)blockIdx.x * m;
     double r = 0;
-    for (uint32_t b = 0; b < blocks; b++) r += partial[(uint64_t)b * width + v];
-    out[v] = r;
-}
-
-// Sequential sum of partial[0..m) into out[0].
-__global__ void k_sum_partials(const double *__restrict__ partial, uint32_t m, double *__restrict__ out) {
-    if (threadIdx.x == 0 && blockIdx.x == 0) {
-        double r = 0;
-        for (uint32_t i = 0; i < m; i++) r += partial[i];
-        out[0] = r;
-    }
+    for (uint32_t i = threadIdx.x; i < m; i += RED_THREADS) r += row[i];
+    r = block_sum(r, scratch);
+    if (threadIdx.x == 0) out[blockIdx.x] = r;
 }
 
 // Per-block max |a-b|, sum |a-b|^2 and sum |b|^2 over two states.
@@ -479,10 +482,17 @@ __global__ __launch_bounds__(RED_THREADS) void k_compare(const TA *__restrict__ 
 }
 
 // <Z_q> and <Z_q Z_q+1> in one pass. A block covers a segment of 2^B
-// contiguous amplitudes; per segment it writes 2B values: the total T, the
-// per-bit sums Q[q] = sum p [bit q] (q < B) and the per-pair sums
-// R[q] = sum p [bit q xor bit q+1] (q < B-1). Bits above B are constant in a
-// segment and are resolved by k_expect_combine.
+// contiguous amplitudes; per segment it writes 2B sums of p = |a|^2: the total,
+// the signed sums of p (-1)^(bit q) (q < B) and of p (-1)^(bit q + bit q+1)
+// (q < B-1), value v of segment g at out[v * segments + g]. Bits above B are
+// constant in a segment and are resolved by k_expect_combine.
+//
+// The lanes' sums go through a Walsh-Hadamard transform over the wave's six
+// lane bits: afterwards lane l holds the sum over the wave with sign
+// (-1)^popcount(lane & l), so lanes 0, 1 << q and 3 << q hold every total,
+// single and pair sum of those bits after 6 exchanges (one wave sum per value
+// took 6 each: 34 us for a 20-qubit state against 9 now). Signs of the wave
+// bits are applied where one thread per value adds up the waves.
 constexpr int EZ_TID_BITS = 10;  // bits from the thread index (1024 threads)
 constexpr int EZ_MAX_M_BITS = 6; // bits from the per-thread loop
 
@@ -504,8 +514,7 @@ __global__ __launch_bounds__(1 << EZ_TID_BITS) void k_expect_segments(const T2 *
                                                          const ExpDesc *__restrict__ descs, uint32_t ndesc,
                                                          const uint64_t *__restrict__ seg_start,
                                                          double *__restrict__ out_all) {
-    constexpr int MAXV = 2 * (EZ_TID_BITS + EZ_MAX_M_BITS);  // values per segment, at most
-    __shared__ double scratch[(1 << EZ_TID_BITS) / 64][MAXV];
+    __shared__ double scratch[(1 << EZ_TID_BITS) / 64][12 + 2 * EZ_MAX_M_BITS];
     ExpDesc d = one;
     uint64_t seg = blockIdx.x;
     if (ndesc > 1) {
@@ -520,7 +529,7 @@ __global__ __launch_bounds__(1 << EZ_TID_BITS) void k_expect_segments(const T2 *
     const uint32_t mb = B - tb;
     const uint32_t tid = threadIdx.x;
     const bool active = tid < (1u << tb);
-    double T = 0, S[EZ_MAX_M_BITS], P[EZ_MAX_M_BITS];
+    double T = 0, S[EZ_MAX_M_BITS], P[EZ_MAX_M_BITS];  // the thread's total, and its signed sums over loop bits
 #pragma unroll
     for (int j = 0; j < EZ_MAX_M_BITS; j++) S[j] = P[j] = 0;
     if (active) {
@@ -531,9 +540,8 @@ __global__ __launch_bounds__(1 << EZ_TID_BITS) void k_expect_segments(const T2 *
 #pragma unroll
             for (int j = 0; j < EZ_MAX_M_BITS; j++) {
                 if ((uint32_t)j < mb) {
-                    const uint32_t bj = (m >> j) & 1;
-                    if (bj) S[j] += p;
-                    if ((uint32_t)j + 1 < mb && (bj ^ ((m >> (j + 1)) & 1))) P[j] += p;
+                    S[j] += ((m >> j) & 1) ? -p : p;
+                    if ((uint32_t)j + 1 < mb) P[j] += (((m >> j) ^ (m >> (j + 1))) & 1) ? -p : p;
                 }
             }
         };
@@ -554,115 +562,102 @@ __global__ __launch_bounds__(1 << EZ_TID_BITS) void k_expect_segments(const T2 *
             for (uint32_t m = 0; m < M; m++) add(m, prob(s[base + ((uint64_t)m << tb)]));
         }
     }
-    // The segment's 2B values: T, Q[q] (q < B) and R[q] (q < B - 1), each
-    // summed over the wave, then over the waves in order by one thread per
-    // value after a single barrier.
+    // A wave's sums: slot 0 its total, 1 + q lane bit q, 7 + q lane bits q and
+    // q + 1, 12 + j loop bit j, 18 + j loop bits j and j + 1.
     const uint32_t lane = tid & 63, wave = tid >> 6;
-    auto value = [&](uint32_t k) -> double {
-        if (k == 0) return T;
-        if (k <= B) {  // Q[q]: T times the thread's bit q for q < tb, else S[q - tb]
-            const uint32_t q = k - 1;
-            if (q < tb) return ((tid >> q) & 1) ? T : 0.0;
-            double v = 0;
+    constexpr uint32_t SL = 12, PL = SL + EZ_MAX_M_BITS;
+    double w = T;
 #pragma unroll
-            for (int j = 0; j < EZ_MAX_M_BITS; j++)
-                if ((uint32_t)j == q - tb) v = S[j];
-            return v;
-        }
-        const uint32_t q = k - 1 - B;  // R[q]
-        if (q + 1 < tb) return (((tid >> q) ^ (tid >> (q + 1))) & 1) ? T : 0.0;
-        if (q + 1 == tb) {
-            // bit q from the thread, bit q+1 = loop bit 0.
-            const double s0 = mb > 0 ? S[0] : 0.0;
-            return ((tid >> q) & 1) ? T - s0 : s0;
-        }
-        double v = 0;
+    for (int o = 1; o < 64; o <<= 1) {
+        const double other = __shfl_xor(w, o, 64);
+        w = (lane & o) ? other - w : w + other;
+    }
+    const uint32_t first = lane & -lane;
+    if (lane == 0) scratch[wave][0] = w;
+    else if (lane == first) scratch[wave][1 + __builtin_ctz(lane)] = w;
+    else if (lane == 3 * first) scratch[wave][7 + __builtin_ctz(lane)] = w;
 #pragma unroll
-        for (int j = 0; j < EZ_MAX_M_BITS; j++)
-            if ((uint32_t)j == q - tb) v = P[j];
-        return v;
-    };
-    const uint32_t nv = 2 * B;  // T, B values Q, B - 1 values R
-    for (uint32_t k = 0; k < nv; k++) {
-        const double w = wave_sum(value(k));
-        if (lane == 0) scratch[wave][k] = w;
+    for (int j = 0; j < EZ_MAX_M_BITS; j++) {
+        if ((uint32_t)j < mb) {
+            const double v = wave_sum(S[j]);
+            if (lane == 0) scratch[wave][SL + j] = v;
+            if ((uint32_t)j + 1 < mb) {
+                const double u = wave_sum(P[j]);
+                if (lane == 0) scratch[wave][PL + j] = u;
+            }
+        }
     }
     __syncthreads();
-    if (tid < nv) {
+    if (tid < 2 * B) {
+        uint32_t slot = 0, waves = 0;  // the value's slot, and the wave bits its sign takes
+        if (tid == 0) {
+        } else if (tid <= B) {
+            const uint32_t q = tid - 1;
+            if (q < 6) slot = 1 + q;
+            else if (q < EZ_TID_BITS) waves = 1u << (q - 6);
+            else slot = SL + q - EZ_TID_BITS;
+        } else {
+            const uint32_t q = tid - 1 - B;
+            if (q < 5) slot = 7 + q;
+            else if (q == 5) slot = 6, waves = 1;
+            else if (q + 1 < EZ_TID_BITS) waves = 3u << (q - 6);
+            else if (q + 1 == EZ_TID_BITS) slot = SL, waves = 1u << (EZ_TID_BITS - 7);
+            else slot = PL + q - EZ_TID_BITS;
+        }
         double r = 0;
-        for (int w = 0; w < (int)(blockDim.x >> 6); w++) r += scratch[w][tid];
-        out[seg * (2 * B) + tid] = r;
+        for (uint32_t v = 0; v < (blockDim.x >> 6); v++) {
+            const double x = scratch[v][slot];
+            r += (__popc(v & waves) & 1) ? -x : x;
+        }
+        out[(uint64_t)tid * d.nsegs + seg] = r;
     }
 }
 
-// Combines the segment sums into z[q] = sum p (1 - 2 bit q) and
-// zz[q] = sum p (1 - 2 (bit q xor bit q+1)). One thread per output, in
-// blocks of 64 threads.
-__global__ __launch_bounds__(64) void k_expect_combine(const double *__restrict__ seg_all, ExpDesc one, const ExpDesc *__restrict__ descs,
-                                 uint32_t ndesc, const uint32_t *__restrict__ out_start, double *__restrict__ z,
-                                 double *__restrict__ zz) {
-    const uint32_t wg = threadIdx.x + blockIdx.x * blockDim.x;
+// Combines the segment sums into z[q] and zz[q]: output w is the sum over the
+// segments g of value `idx` with sign (-1)^popcount(g & bits). TPO threads per
+// output (64 or the block): with one thread per output the 2^14 segments of a
+// 30-qubit state were a serial chain of 2.3 ms; now 20 us.
+template <int THREADS, int TPO>
+__global__ __launch_bounds__(THREADS) void k_expect_combine(const double *__restrict__ seg_all, ExpDesc one,
+                                                            const ExpDesc *__restrict__ descs, uint32_t ndesc,
+                                                            const uint32_t *__restrict__ out_start, uint32_t outs,
+                                                            double *__restrict__ z, double *__restrict__ zz) {
+    static_assert(TPO == 64 || TPO == THREADS, "an output's threads are a wave or the block");
+    __shared__ double scratch[THREADS / 64];
+    const uint32_t wg = blockIdx.x * (THREADS / TPO) + threadIdx.x / TPO, t = threadIdx.x % TPO;
     ExpDesc d = one;
     uint32_t w = wg;
+    if (wg >= outs) return;  // uniform over the output's threads
     if (ndesc > 1) {
-        if (wg >= out_start[ndesc]) return;
         const uint32_t di = find_range(out_start, ndesc, wg);
         d = descs[di];
         w = wg - out_start[di];
     }
     const uint32_t n = d.n, B = d.B;
-    if (w >= 2 * n - 1) return;
-    const double *seg_sums = seg_all + d.seg_off;
-    // What the output takes from segment g besides its total T = o[0]:
-    //   0: o[idx]                          (its bit, or both bits of its pair, inside the segment)
-    //   1: T where bit sh of g is set      (<Z_q>, q at or above the segment bits)
-    //   2: (g & 1) ? T - o[idx] : o[idx]   (<Z_q Z_q+1>, bit q the segment's top bit)
-    //   3: T where bits sh and sh + 1 of g differ
-    uint32_t mode, idx = 0, sh = 0;
+    uint32_t idx = 0;
+    uint64_t bits = 0;
     if (w < n) {
         const uint32_t q = w;
-        if (q < B) mode = 0, idx = 1 + q;
-        else mode = 1, sh = q - B;
+        if (q < B) idx = 1 + q;
+        else bits = uint64_t(1) << (q - B);
     } else {
         const uint32_t q = w - n;
-        if (q + 1 < B) mode = 0, idx = 1 + B + q;
-        else if (q + 1 == B) mode = 2, idx = 1 + q;
-        else mode = 3, sh = q - B;
+        if (q + 1 < B) idx = 1 + B + q;
+        else if (q + 1 == B) idx = 1 + q, bits = 1;
+        else bits = uint64_t(3) << (q - B);
     }
-    // Branch-free: where an output takes nothing from a segment it adds
-    // +0.0, which leaves the sum as it is (both sums start at +0.0 and add
-    // non-negative values, so neither is ever -0.0).
-    double tot = 0, part = 0;
-    auto add = [&](uint64_t g, double T, double V) {
-        tot += T;
-        const bool b0 = (g >> sh) & 1, b1 = (g >> (sh + 1)) & 1;
-        const double a = mode == 0 ? V : mode == 1 ? (b0 ? T : 0.0) : mode == 2 ? ((g & 1) ? T - V : V) : (b0 != b1 ? T : 0.0);
-        part += a;
-    };
-    // The segments in order; G segments' values are loaded at a time, so a
-    // state of many segments does not wait for one load per segment.
-    // One pointer steps through a batch (precomputed per-segment addresses
-    // would be loop invariants the compiler keeps, and spills).
-    constexpr uint32_t G = 32;
-    const uint64_t stride = 2 * (uint64_t)B;
-    uint64_t g = 0;
-    for (; g + G <= d.nsegs; g += G) {
-        double T[G], V[G];
-        const double *o = seg_sums + g * stride;
-#pragma unroll
-        for (uint32_t u = 0; u < G; u++, o += stride) {
-            T[u] = o[0];
-            V[u] = o[idx];
-        }
-#pragma unroll
-        for (uint32_t u = 0; u < G; u++) add(g + u, T[u], V[u]);
+    const double *const v = seg_all + d.seg_off + (uint64_t)idx * d.nsegs;
+    double r = 0;
+    for (uint64_t g = t; g < d.nsegs; g += TPO) {
+        const double x = v[g];
+        r += (__popcll(g & bits) & 1) ? -x : x;
     }
-    for (; g < d.nsegs; g++) {
-        const double *o = seg_sums + g * stride;
-        add(g, o[0], o[idx]);
+    if constexpr (TPO == 64) r = wave_sum(r);
+    else r = block_sum(r, scratch);
+    if (t == 0) {
+        if (w < n) z[d.z_off + w] = r;
+        else zz[d.zz_off + w - n] = r;
     }
-    if (w < n) z[d.z_off + w] = tot - 2 * part;
-    else zz[d.zz_off + w - n] = tot - 2 * part;
 }
 
 // Sets amplitude 0 of each state of a batch to 1 (after a zero fill).
@@ -685,23 +680,41 @@ __global__ void k_zero_words(uint32_t *__restrict__ p, uint32_t n) {
 
 // ---------------------------------------------------------------------------
 // Measurement collapse (src/measure.rs:68-80): the kept half scaled by
-// `keep` in the state's precision, the other half zeroed.
+// 1 / sqrt(its probability) in the state's precision, the other half zeroed. The outcome
+// follows from P(1) in device memory, so the host need not wait between the
+// two passes. FLIP (reset): outcome 1 is followed by an X on the qubit in the
+// same pass, with the arithmetic of k_dense on that matrix.
 // ---------------------------------------------------------------------------
-template <typename T2>
-__global__ void k_collapse(T2 *__restrict__ s, uint64_t len, uint32_t qubit, uint32_t outcome, double keep) {
+template <typename T2, bool FLIP>
+__global__ __launch_bounds__(256) void k_collapse(T2 *__restrict__ s, uint64_t len, uint32_t qubit, double uniform,
+                                                  const double *__restrict__ p_one) {
     using T = typename Real<T2>::T;
-    const T k = (T)keep;
+    double p1 = *p_one;
+    p1 = p1 < 0.0 ? 0.0 : p1;  // a NaN stays one, as in the host's clamp
+    p1 = 1.0 < p1 ? 1.0 : p1;
+    const bool outcome = uniform < p1;
+    T2 keep, drop;
+    keep.x = (T)(1.0 / sqrt(outcome ? p1 : 1.0 - p1));
+    keep.y = drop.x = drop.y = 0;
     const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
-    for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < len; i += stride) {
-        T2 f;
-        if (((i >> qubit) & 1) == outcome) {
-            f.x = k;
-            f.y = 0;
-        } else {
-            f.x = 0;
-            f.y = 0;
+    const uint64_t bit = uint64_t(1) << qubit;
+    for (uint64_t it = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; it < len >> 1; it += stride) {
+        const uint64_t i0 = ((it & ~(bit - 1)) << 1) | (it & (bit - 1)), i1 = i0 | bit;
+        T2 a = cmul_diag(outcome ? drop : keep, s[i0]), b = cmul_diag(outcome ? keep : drop, s[i1]);
+        if (FLIP && outcome) {
+            T2 one;
+            one.x = 1;
+            one.y = 0;
+            T2 o0 = drop, o1 = drop;
+            cmac(o0, drop, a);
+            cmac(o0, one, b);
+            cmac(o1, one, a);
+            cmac(o1, drop, b);
+            a = o0;
+            b = o1;
         }
-        s[i] = cmul_diag(f, s[i]);
+        s[i0] = a;
+        s[i1] = b;
     }
 }
 
@@ -1119,11 +1132,17 @@ void launch_stage(T2 *s, const StageDesc &d, const StageOp *ops, const T2 *coefs
     k_stage<T2><<<grid, STAGE_THREADS, stage_lds_bytes<T2>(d.L), st>>>(s, d, ops, coefs);
 }
 
+// One block while the whole sum is a few batches of loads per thread (up to
+// 2^13 amplitudes: a second launch would cost more), then 8 amplitudes a
+// thread up to 1024 blocks.
 template <typename T2>
-void launch_masked_norm(const T2 *s, uint64_t len, uint64_t mask, uint64_t val, double *partial, unsigned blocks,
-                        double *out, hipStream_t st) {
-    k_masked_norm<T2><<<blocks, RED_THREADS, 0, st>>>(s, len, mask, val, partial);
-    k_sum_partials<<<1, 64, 0, st>>>(partial, blocks, out);
+void launch_norm(const T2 *s, uint64_t len, int qubit, double *partial, double *out, hipStream_t st) {
+    const uint64_t count = qubit >= 0 ? len >> 1 : len;
+    const unsigned blocks = count <= (1u << 13) ? 1 : (unsigned)std::min<uint64_t>(count >> 11, NORM_BLOCKS);
+    double *const to = blocks == 1 ? out : partial;
+    if (qubit >= 0) k_norm<T2, true><<<blocks, RED_THREADS, 0, st>>>(s, count, (uint32_t)qubit, to);
+    else k_norm<T2, false><<<blocks, RED_THREADS, 0, st>>>(s, count, 0, to);
+    if (blocks > 1) k_sum_rows<<<1, RED_THREADS, 0, st>>>(partial, blocks, out);
 }
 
 template <typename T2>
@@ -1132,19 +1151,50 @@ void launch_probabilities(const T2 *s, uint64_t len, double *out, hipStream_t st
 }
 
 template <typename T2>
-void launch_expect_pauli(const T2 *s, uint64_t len, uint64_t x, const uint64_t *zs, uint32_t nterms, double *partial,
-                         unsigned blocks, double *out, hipStream_t st) {
-    if (nterms <= 1) k_expect_pauli<T2, 1><<<blocks, RED_THREADS, 0, st>>>(s, len, x, zs, nterms, partial);
-    else if (nterms <= 2) k_expect_pauli<T2, 2><<<blocks, RED_THREADS, 0, st>>>(s, len, x, zs, nterms, partial);
-    else if (nterms <= 4) k_expect_pauli<T2, 4><<<blocks, RED_THREADS, 0, st>>>(s, len, x, zs, nterms, partial);
-    else if (nterms <= 8) k_expect_pauli<T2, 8><<<blocks, RED_THREADS, 0, st>>>(s, len, x, zs, nterms, partial);
-    else k_expect_pauli<T2, PAULI_TERMS><<<blocks, RED_THREADS, 0, st>>>(s, len, x, zs, nterms, partial);
-    k_sum_columns<<<1, 64, 0, st>>>(partial, blocks, 2 * nterms, out);
+static void pauli_group_launch(const T2 *s, uint64_t len, const PauliGroup *groups, uint32_t ngroups, uint32_t width,
+                               const uint64_t *zs, double *partial, unsigned blocks, hipStream_t st) {
+    const dim3 grid(blocks, ngroups);
+    if (width <= 1) k_expect_pauli<T2, 1><<<grid, RED_THREADS, 0, st>>>(s, len, groups, zs, partial);
+    else if (width <= 2) k_expect_pauli<T2, 2><<<grid, RED_THREADS, 0, st>>>(s, len, groups, zs, partial);
+    else if (width <= 4) k_expect_pauli<T2, 4><<<grid, RED_THREADS, 0, st>>>(s, len, groups, zs, partial);
+    else if (width <= 8) k_expect_pauli<T2, 8><<<grid, RED_THREADS, 0, st>>>(s, len, groups, zs, partial);
+    else k_expect_pauli<T2, PAULI_TERMS><<<grid, RED_THREADS, 0, st>>>(s, len, groups, zs, partial);
 }
 
-ExpDesc expect_desc(uint32_t state_qubits, uint32_t n) {
+// Four pairs of amplitudes a thread where the state is small, and enough
+// blocks over all groups of a launch to fill the chip where it is large.
+unsigned pauli_blocks(uint64_t len, uint32_t ngroups) {
+    const uint64_t want = std::max<uint64_t>(1, len / (2 * 4 * RED_THREADS));
+    const uint64_t cap = std::max<uint64_t>(64, 2048 / std::max<uint32_t>(ngroups, 1));
+    return (unsigned)std::min(want, cap);
+}
+
+template <typename T2>
+void launch_expect_pauli(const T2 *s, uint64_t len, const PauliGroup *groups, const std::vector<uint32_t> &widths,
+                         const uint64_t *zs, uint32_t nterms, double *partial, unsigned blocks, double *out,
+                         hipStream_t st) {
+    double *const to = blocks == 1 ? out : partial;
+    // Runs of groups with the same number of term slots are one launch.
+    auto slots = [](uint32_t w) { return w <= 1 ? 1 : w <= 2 ? 2 : w <= 4 ? 4 : w <= 8 ? 8 : 16; };
+    for (size_t g = 0; g < widths.size();) {
+        size_t e = g + 1;
+        while (e < widths.size() && slots(widths[e]) == slots(widths[g])) e++;
+        pauli_group_launch(s, len, groups + g, (uint32_t)(e - g), widths[g], zs, to, blocks, st);
+        g = e;
+    }
+    if (blocks > 1) k_sum_rows<<<nterms, RED_THREADS, 0, st>>>(partial, blocks, out);
+}
+
+// Segments of 2^16 amplitudes, 64 a thread; a single state of fewer than 24
+// qubits takes smaller ones (at least 2^10), so that 256 of them fill the chip.
+uint32_t expect_segment_bits(uint32_t n) {
+    if (n <= EZ_TID_BITS) return n;
+    return std::min<uint32_t>(EZ_TID_BITS + EZ_MAX_M_BITS, n <= EZ_TID_BITS + 8 ? EZ_TID_BITS : n - 8);
+}
+
+ExpDesc expect_desc(uint32_t state_qubits, uint32_t n, uint32_t segment_bits) {
     ExpDesc d{};
-    d.B = expect_segment_bits(state_qubits);
+    d.B = segment_bits;
     d.nsegs = uint64_t(1) << (state_qubits - d.B);
     d.n = n;
     return d;
@@ -1152,19 +1202,20 @@ ExpDesc expect_desc(uint32_t state_qubits, uint32_t n) {
 
 template <typename T2>
 void launch_expect_z(const T2 *s, uint32_t n, double *seg_sums, double *z, double *zz, hipStream_t st) {
-    const ExpDesc d = expect_desc(n, n);
+    const ExpDesc d = expect_desc(n, n, expect_segment_bits(n));
     k_expect_segments<T2><<<(unsigned)d.nsegs, 1 << EZ_TID_BITS, 0, st>>>(s, d, nullptr, 1, nullptr, seg_sums);
     const uint32_t outs = 2 * n - 1;
-    k_expect_combine<<<(outs + 63) / 64, 64, 0, st>>>(seg_sums, d, nullptr, 1, nullptr, z, zz);
+    // A block per output once a wave would walk more than 4 segments a lane.
+    if (d.nsegs > 256) k_expect_combine<512, 512><<<outs, 512, 0, st>>>(seg_sums, d, nullptr, 1, nullptr, outs, z, zz);
+    else k_expect_combine<64, 64><<<outs, 64, 0, st>>>(seg_sums, d, nullptr, 1, nullptr, outs, z, zz);
 }
 
 template <typename T2>
 void launch_expect_batch(const T2 *s, const ExpDesc *descs, uint32_t ndesc, const uint64_t *seg_start,
                          uint64_t total_segs, const uint32_t *out_start, uint32_t total_outs, double *seg_sums,
-                         double *z, double *zz, hipStream_t st) {
-    const ExpDesc none{};
-    k_expect_segments<T2><<<(unsigned)total_segs, 1 << EZ_TID_BITS, 0, st>>>(s, none, descs, ndesc, seg_start, seg_sums);
-    k_expect_combine<<<(total_outs + 63) / 64, 64, 0, st>>>(seg_sums, none, descs, ndesc, out_start, z, zz);
+                         double *z, double *zz, const ExpDesc &first, hipStream_t st) {
+    k_expect_segments<T2><<<(unsigned)total_segs, 1 << EZ_TID_BITS, 0, st>>>(s, first, descs, ndesc, seg_start, seg_sums);
+    k_expect_combine<256, 64><<<(total_outs + 3) / 4, 256, 0, st>>>(seg_sums, first, descs, ndesc, out_start, total_outs, z, zz);
 }
 
 void launch_zero_words(uint32_t *p, uint32_t n, hipStream_t st) {
@@ -1187,11 +1238,14 @@ template void launch_compare<double2, float2>(const double2 *, const float2 *, u
 template void launch_compare<double2, double2>(const double2 *, const double2 *, uint64_t, double *, unsigned,
                                                hipStream_t);
 
-uint32_t expect_segment_bits(uint32_t n) { return n < EZ_TID_BITS + EZ_MAX_M_BITS ? n : EZ_TID_BITS + EZ_MAX_M_BITS; }
+uint32_t expect_batch_segment_bits(uint32_t n) { return std::min<uint32_t>(n, EZ_TID_BITS + EZ_MAX_M_BITS); }
 
 template <typename T2>
-void launch_collapse(T2 *s, uint64_t len, uint32_t qubit, uint32_t outcome, double keep, hipStream_t st) {
-    k_collapse<T2><<<grid_for(len, 256, 65536), 256, 0, st>>>(s, len, qubit, outcome, keep);
+void launch_collapse(T2 *s, uint64_t len, uint32_t qubit, double uniform, const double *p_one, bool flip,
+                     hipStream_t st) {
+    const unsigned grid = grid_for(len >> 1, 256, 65536);
+    if (flip) k_collapse<T2, true><<<grid, 256, 0, st>>>(s, len, qubit, uniform, p_one);
+    else k_collapse<T2, false><<<grid, 256, 0, st>>>(s, len, qubit, uniform, p_one);
 }
 
 // Workspace of the allocation-free sampler. In host code `scratch` names a
@@ -1263,16 +1317,16 @@ hipError_t launch_sample_walk(const T2 *s, uint64_t len, uint64_t chunk, uint64_
                                   hipStream_t);                                                                 \
     template size_t stage_lds_bytes<T2>(uint32_t);                                                              \
     template void launch_stage<T2>(T2 *, const StageDesc &, const StageOp *, const T2 *, unsigned, hipStream_t); \
-    template void launch_masked_norm<T2>(const T2 *, uint64_t, uint64_t, uint64_t, double *, unsigned, double *, \
-                                         hipStream_t);                                                          \
+    template void launch_norm<T2>(const T2 *, uint64_t, int, double *, double *, hipStream_t);                  \
     template void launch_expect_z<T2>(const T2 *, uint32_t, double *, double *, double *, hipStream_t);         \
     template void launch_probabilities<T2>(const T2 *, uint64_t, double *, hipStream_t);                        \
-    template void launch_expect_pauli<T2>(const T2 *, uint64_t, uint64_t, const uint64_t *, uint32_t, double *, \
-                                          unsigned, double *, hipStream_t);                                     \
+    template void launch_expect_pauli<T2>(const T2 *, uint64_t, const PauliGroup *, const std::vector<uint32_t> &, \
+                                          const uint64_t *, uint32_t, double *, unsigned, double *, hipStream_t); \
     template void launch_expect_batch<T2>(const T2 *, const ExpDesc *, uint32_t, const uint64_t *, uint64_t,    \
-                                          const uint32_t *, uint32_t, double *, double *, double *, hipStream_t); \
+                                          const uint32_t *, uint32_t, double *, double *, double *, const ExpDesc &, \
+                                          hipStream_t);                                                         \
     template void launch_batch_init<T2>(T2 *, uint64_t, const uint64_t *, uint32_t, hipStream_t);              \
-    template void launch_collapse<T2>(T2 *, uint64_t, uint32_t, uint32_t, double, hipStream_t);                 \
+    template void launch_collapse<T2>(T2 *, uint64_t, uint32_t, double, const double *, bool, hipStream_t);     \
     template void launch_sample_sums<T2>(const T2 *, uint64_t, uint64_t, SampleScratch &, hipStream_t);         \
     template hipError_t launch_sample_walk<T2>(const T2 *, uint64_t, uint64_t, uint64_t, SampleScratch &,       \
                                                uint64_t *, hipStream_t);
