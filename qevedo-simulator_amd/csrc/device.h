@@ -27,7 +27,7 @@ struct StageOp {
     uint32_t lc_mask, lc_val;
     uint64_t gc_mask, gc_val;
     uint32_t coef_off;  // first coefficient (complex) of this op
-    uint32_t pad;
+    uint32_t taken;     // the bits of ins[] as a mask (k_stage)
 };
 
 // One stage: the tile's qubits and the ops applied to every tile.
@@ -36,6 +36,7 @@ struct StageDesc {
     uint32_t nglob;    // non-tile bits
     uint32_t num_ops;
     uint32_t op_off;   // first StageOp of the stage in the op array
+    uint32_t from_zero;  // the tiles are |0...0>'s, made instead of loaded
     uint64_t num_tiles;
     uint32_t local_pos[MAX_QUBITS];  // tile bit j -> physical bit, ascending
     uint32_t glob_pos[MAX_QUBITS];   // tile-index bit j -> physical bit, ascending

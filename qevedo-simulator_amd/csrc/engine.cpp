@@ -463,7 +463,10 @@ void lower_stage(const Stage &st, uint32_t n, std::vector<StageOp> &ops, std::ve
         }
         std::sort(ins.begin(), ins.end());
         so.nins = (uint32_t)ins.size();
-        for (size_t j = 0; j < ins.size(); j++) so.ins[j] = ins[j];
+        for (size_t j = 0; j < ins.size(); j++) {
+            so.ins[j] = ins[j];
+            so.taken |= 1u << ins[j];
+        }
         ops.push_back(so);
         d.num_ops++;
     }
@@ -534,15 +537,15 @@ uint64_t run_plan(qvd_sv *sv, T2 *s, const std::vector<Step> &steps, qvd_stats &
     // each stage sets the amplitudes of the stale qubits to zero instead of
     // loading them and writes every tile it visits, and the qubits whose
     // tiles it skips (known to be |0>) are the stale ones after it. Another
-    // plan makes a pending |0...0> in its first stage when that is a
-    // register-tile stage visiting every tile; otherwise, and for stale
-    // qubits, the zeros are written first.
+    // plan makes a pending |0...0> in its first stage when that visits every
+    // tile (an LDS-tile stage does); otherwise, and for stale qubits, the
+    // zeros are written first.
     bool all_reg = true;
     for (const Step &step : steps) all_reg = all_reg && step.is_stage && step.stage.reg_tile;
     bool pending = sv->zero_pending;
     uint64_t stale = pending ? 0 : sv->stale_qubits;
     bool write_zeros = false;
-    if ((pending && !(steps[0].is_stage && steps[0].stage.reg_tile)) || (!all_reg && stale)) {
+    if ((pending && !steps[0].is_stage) || (!all_reg && stale)) {
         write_zeros = true;
         pending = false;
         stale = 0;
@@ -576,8 +579,13 @@ uint64_t run_plan(qvd_sv *sv, T2 *s, const std::vector<Step> &steps, qvd_stats &
         } else {
             StageDesc d;
             lower_stage<T2>(step.stage, sv->n, sops, coefs, d);
+            if (pending) {
+                pending = false;
+                if (d.num_ops != 0) d.from_zero = 1;
+                else write_zeros = true;  // no launch
+            }
             descs.push_back(d);
-            st.stage_bytes += 2 * state_bytes;
+            st.stage_bytes += (d.from_zero ? 1 : 2) * state_bytes;
         }
         for (const Op &op : step.stage.ops) zero = after_op(zero, op);
     }
@@ -635,8 +643,7 @@ uint64_t run_plan(qvd_sv *sv, T2 *s, const std::vector<Step> &steps, qvd_stats &
             const unsigned grid = (unsigned)std::min<uint64_t>(d.num_tiles, want);
             timer.begin(timer.stage);
             reg_launch.push_back(0);
-            launch_stage<T2>(s, d, dops, dcoef, grid, sv->stream);
-            QVD_HIP(hipGetLastError());
+            QVD_HIP(launch_stage<T2>(s, d, dops, dcoef, grid, sv->stream));
             timer.end(timer.stage);
             st.stages++;
             st.passes++;

@@ -70,7 +70,8 @@ void launch_diag(T2 *s, uint64_t len, uint32_t k, const DiagTargets &t, uint64_t
                  const T2 *entries, hipStream_t st);
 template <typename T2> size_t stage_lds_bytes(uint32_t L);
 template <typename T2>
-void launch_stage(T2 *s, const StageDesc &d, const StageOp *ops, const T2 *coefs, unsigned grid, hipStream_t st);
+hipError_t launch_stage(T2 *s, const StageDesc &d, const StageOp *ops, const T2 *coefs, unsigned grid,
+                        hipStream_t st);
 // out = the sum of |a|^2 over the state, or over the amplitudes with bit `qubit`
 // set (qubit >= 0); partial holds NORM_BLOCKS doubles.
 constexpr unsigned NORM_BLOCKS = 1024;

@@ -11,6 +11,7 @@
 #include <hipcub/hipcub.hpp>
 
 #include <algorithm>
+#include <atomic>
 #include <mutex>
 
 #include "device.h"
@@ -190,110 +191,224 @@ __global__ __launch_bounds__(256) void k_diag(T2 *__restrict__ s, uint64_t len, 
 // the tile back. Non-tile qubits are fixed per tile: non-tile controls
 // select whether an op runs on the tile at all, and non-tile diagonal targets
 // select the entries used.
+//
+// States smaller than a register tile are one such tile, so one workgroup
+// works through the ops and each op's latency counts. The op records and
+// matrices of a run of ops are therefore copied to LDS together (a load per
+// op was a memory round trip per op), and an op of fewer groups than threads
+// deals the rows of its matrix out as well: 12 qubits in complex128, 120 gates
+// fused to 4 qubits, 541 -> 91 us.
 // ---------------------------------------------------------------------------
-constexpr int STAGE_THREADS = 256;
-constexpr int STAGE_LOG_THREADS = 8;
+constexpr uint32_t STAGE_OPS = 48;             // op records held in LDS
+constexpr uint32_t STAGE_COEF_BYTES = 8192;    // their matrices and diagonals
+static_assert(STAGE_OPS <= 64, "one lane per op record");
+static_assert(sizeof(StageOp) % 4 == 0, "op records are copied by words");
 
-template <typename T2, int K>
+__device__ __forceinline__ uint32_t uniform(uint32_t v) { return __builtin_amdgcn_readfirstlane(v); }
+
+// Spreads x over the bits not set in `taken`.
+__device__ __forceinline__ uint32_t spread_around(uint32_t x, uint32_t taken) {
+    while (taken) {
+        const uint32_t p = __builtin_ctz(taken);
+        x = ((x >> p) << (p + 1)) | (x & ((1u << p) - 1));
+        taken &= taken - 1;
+    }
+    return x;
+}
+
+// A dense op with rows dealt out: 2^LR threads share a group of 2^K amplitudes,
+// each computing 2^(K - LR) rows.
+template <typename T2, int K, int LR>
+__device__ __forceinline__ void tile_rows(T2 *__restrict__ tile, const T2 *__restrict__ m, const uint32_t (&tb)[K],
+                                          uint32_t taken, uint32_t val, uint32_t lg) {
+    constexpr int D = 1 << K, RPT = D >> LR;
+    const uint32_t sub = threadIdx.x >> lg;
+    const bool active = sub < (1u << LR);
+    const uint32_t i0 = spread_around(threadIdx.x & ((1u << lg) - 1), taken) | val;
+    T2 acc[RPT];
+    if (active) {
+        T2 a[D];
+#pragma unroll
+        for (int j = 0; j < D; j++) {
+            uint32_t o = 0;
+#pragma unroll
+            for (int b = 0; b < K; b++)
+                if ((j >> b) & 1) o |= tb[b];
+            a[j] = tile[i0 | o];
+        }
+        const T2 *row = m + sub * RPT * D;
+#pragma unroll
+        for (int r = 0; r < RPT; r++) {
+            acc[r].x = 0;
+            acc[r].y = 0;
+#pragma unroll
+            for (int c = 0; c < D; c++) cmac(acc[r], row[r * D + c], a[c]);
+        }
+    }
+    __syncthreads();
+    if (active) {
+#pragma unroll
+        for (int r = 0; r < RPT; r++) {
+            const uint32_t j = sub * RPT + r;
+            uint32_t o = 0;
+#pragma unroll
+            for (int b = 0; b < K; b++)
+                if ((j >> b) & 1) o |= tb[b];
+            tile[i0 | o] = acc[r];
+        }
+    }
+}
+
+template <typename T2, int K, int LOG_THREADS>
 __device__ __forceinline__ void tile_dense(T2 *__restrict__ tile, const T2 *__restrict__ m, const StageOp &op,
                                            uint32_t L) {
     constexpr int D = 1 << K;
-    uint32_t off[D];
+    uint32_t tb[K];
 #pragma unroll
-    for (int j = 0; j < D; j++) {
-        uint32_t o = 0;
-#pragma unroll
-        for (int b = 0; b < K; b++) o |= (uint32_t)((j >> b) & 1) << op.tgt[b];
-        off[j] = o;
+    for (int b = 0; b < K; b++) tb[b] = 1u << uniform(op.tgt[b]);
+    const uint32_t taken = uniform(op.taken), val = uniform(op.lc_val);
+    const uint32_t lg = L - __builtin_popcount(taken);
+    if (lg < LOG_THREADS) {
+        const uint32_t lr = LOG_THREADS - lg;
+        if (lr == 1) tile_rows<T2, K, 1>(tile, m, tb, taken, val, lg);
+        else if (K == 2 || lr == 2) tile_rows<T2, K, K < 2 ? K : 2>(tile, m, tb, taken, val, lg);
+        else if (K == 3 || lr == 3) tile_rows<T2, K, K < 3 ? K : 3>(tile, m, tb, taken, val, lg);
+        else tile_rows<T2, K, K < 4 ? K : 4>(tile, m, tb, taken, val, lg);
+        return;
     }
-    const uint32_t groups = 1u << (L - op.nins);
-    for (uint32_t g = threadIdx.x; g < groups; g += STAGE_THREADS) {
-        uint32_t i0 = g;
-        for (uint32_t j = 0; j < op.nins; j++) {
-            const uint32_t p = op.ins[j];
-            i0 = ((i0 >> p) << (p + 1)) | (i0 & ((1u << p) - 1));
-        }
-        i0 |= op.lc_val;
+    for (uint32_t g = threadIdx.x; g < (1u << lg); g += 1u << LOG_THREADS) {
+        const uint32_t i0 = spread_around(g, taken) | val;
         T2 a[D];
 #pragma unroll
-        for (int j = 0; j < D; j++) a[j] = tile[i0 | off[j]];
+        for (int j = 0; j < D; j++) {
+            uint32_t o = 0;
 #pragma unroll
+            for (int b = 0; b < K; b++)
+                if ((j >> b) & 1) o |= tb[b];
+            a[j] = tile[i0 | o];
+        }
+        // Rows one at a time from K = 3 on, their offset rebuilt from r.
+        constexpr int U = K < 3 ? D : 1;
+#pragma unroll U
         for (int r = 0; r < D; r++) {
             T2 acc;
             acc.x = 0;
             acc.y = 0;
 #pragma unroll
             for (int c = 0; c < D; c++) cmac(acc, m[r * D + c], a[c]);
-            tile[i0 | off[r]] = acc;
+            uint32_t o = 0;
+#pragma unroll
+            for (int b = 0; b < K; b++) o |= ((r >> b) & 1) ? tb[b] : 0;
+            tile[i0 | o] = acc;
         }
     }
 }
 
-template <typename T2>
+template <typename T2, int LOG_THREADS>
 __device__ __forceinline__ void tile_diag(T2 *__restrict__ tile, const T2 *__restrict__ e, const StageOp &op,
                                           uint32_t L, uint64_t base) {
-    uint32_t gidx = 0, lmask[MAX_GATE_QUBITS];
-    for (uint32_t j = 0; j < op.k; j++) {
-        const uint32_t t = op.tgt[j];
-        if (t & GLOBAL_BIT) {
-            gidx |= (uint32_t)((base >> (t & ~GLOBAL_BIT)) & 1) << j;
-            lmask[j] = 0;
-        } else {
-            lmask[j] = 1u << t;
-        }
+    const uint32_t k = uniform(op.k), lc_mask = uniform(op.lc_mask), lc_val = uniform(op.lc_val);
+    uint32_t gidx = 0, pos[MAX_GATE_QUBITS];
+#pragma unroll
+    for (uint32_t j = 0; j < MAX_GATE_QUBITS; j++) {
+        pos[j] = 0;
+        if (j >= k) continue;
+        const uint32_t t = uniform(op.tgt[j]);
+        if (t & GLOBAL_BIT) gidx |= (uint32_t)((base >> (t & ~GLOBAL_BIT)) & 1) << j;
+        else pos[j] = 1u << t;
     }
     const uint32_t tsize = 1u << L;
-    for (uint32_t i = threadIdx.x; i < tsize; i += STAGE_THREADS) {
-        if ((i & op.lc_mask) != op.lc_val) continue;
+    for (uint32_t i = threadIdx.x; i < tsize; i += 1u << LOG_THREADS) {
+        if ((i & lc_mask) != lc_val) continue;
         uint32_t idx = gidx;
-        for (uint32_t j = 0; j < op.k; j++) idx |= (uint32_t)((i & lmask[j]) != 0) << j;
+#pragma unroll
+        for (uint32_t j = 0; j < MAX_GATE_QUBITS; j++) idx |= (i & pos[j]) ? 1u << j : 0;
         tile[i] = cmul_diag(e[idx], tile[i]);
     }
 }
 
-template <typename T2>
-__global__ __launch_bounds__(STAGE_THREADS) void k_stage(T2 *__restrict__ s, const StageDesc d,
-                                                         const StageOp *__restrict__ ops,
-                                                         const T2 *__restrict__ coefs) {
-    extern __shared__ unsigned char smem_raw[];
-    T2 *tile = reinterpret_cast<T2 *>(smem_raw);
+template <typename T2, int LOG_THREADS>
+__global__ __launch_bounds__(1 << LOG_THREADS) void k_stage(T2 *__restrict__ s, const StageDesc d,
+                                                            const StageOp *__restrict__ ops,
+                                                            const T2 *__restrict__ coefs) {
+    constexpr uint32_t THREADS = 1u << LOG_THREADS, CMAX = STAGE_COEF_BYTES / sizeof(T2);
+    extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
+    T2 *const tile = reinterpret_cast<T2 *>(smem_raw);
     const uint32_t L = d.L;
     const uint32_t tsize = 1u << L;
-    T2 *mat = tile + tsize;  // coefficients of the current op (<= 16 x 16)
+    T2 *const mat = tile + tsize;
+    StageOp *const lops = reinterpret_cast<StageOp *>(mat + CMAX);
     const uint32_t tid = threadIdx.x;
-    const uint32_t lowbits = L < STAGE_LOG_THREADS ? L : STAGE_LOG_THREADS;
+    const uint32_t lowbits = L < LOG_THREADS ? L : LOG_THREADS;
     uint64_t toff = 0;
     for (uint32_t j = 0; j < lowbits; j++) toff |= (uint64_t)((tid >> j) & 1) << d.local_pos[j];
     const bool active = tid < tsize;
+    // Copies the op records from o0 on and the coefficients of as many of them
+    // as fit (coefficients lie in op order); returns how many.
+    auto load_ops = [&](uint32_t o0) -> uint32_t {
+        const uint32_t cnt = d.num_ops - o0 < STAGE_OPS ? d.num_ops - o0 : STAGE_OPS;
+        const uint32_t *const src = reinterpret_cast<const uint32_t *>(ops + d.op_off + o0);
+        uint32_t *const dst = reinterpret_cast<uint32_t *>(lops);
+        for (uint32_t i = tid; i < cnt * (sizeof(StageOp) / 4); i += THREADS) dst[i] = src[i];
+        __syncthreads();
+        const uint32_t lane = tid & 63, first = uniform(lops[0].coef_off);
+        uint32_t end = 0;
+        if (lane < cnt) {
+            const StageOp &op = lops[lane];
+            end = op.coef_off + (1u << (op.kind == OP_DENSE ? 2 * op.k : op.k)) - first;
+        }
+        const uint32_t fit = (uint32_t)__popcll(__ballot(lane < cnt && end <= CMAX));
+        const uint32_t total = uniform(__shfl(end, fit - 1, 64));  // one op always fits
+        for (uint32_t i = tid; i < total; i += THREADS) mat[i] = coefs[first + i];
+        __syncthreads();
+        return fit;
+    };
+    uint32_t held = load_ops(0);  // the ops [0, held) are in LDS
     for (uint64_t t = blockIdx.x; t < d.num_tiles; t += gridDim.x) {
         uint64_t base = 0;
         for (uint32_t j = 0; j < d.nglob; j++) base |= ((t >> j) & 1) << d.glob_pos[j];
-        for (uint32_t m = 0; m < tsize; m += STAGE_THREADS) {
+        for (uint32_t m = 0; m < tsize; m += THREADS) {
             uint64_t moff = 0;
             for (uint32_t j = lowbits; j < L; j++) moff |= (uint64_t)((m >> j) & 1) << d.local_pos[j];
-            if (active) tile[m + tid] = s[base + moff + toff];
+            if (!active) continue;
+            if (d.from_zero) {
+                T2 v;
+                v.x = (base | moff | toff) == 0 ? 1 : 0;
+                v.y = 0;
+                tile[m + tid] = v;
+            } else {
+                tile[m + tid] = s[base + moff + toff];
+            }
         }
         __syncthreads();
-        for (uint32_t o = 0; o < d.num_ops; o++) {
-            const StageOp &op = ops[d.op_off + o];
-            if ((base & op.gc_mask) != op.gc_val) continue;
-            const uint32_t ncoef = op.kind == OP_DENSE ? (1u << (2 * op.k)) : (1u << op.k);
-            for (uint32_t c = tid; c < ncoef; c += STAGE_THREADS) mat[c] = coefs[op.coef_off + c];
-            __syncthreads();
-            if (op.kind == OP_DENSE) {
-                switch (op.k) {
-                    case 1: tile_dense<T2, 1>(tile, mat, op, L); break;
-                    case 2: tile_dense<T2, 2>(tile, mat, op, L); break;
-                    case 3: tile_dense<T2, 3>(tile, mat, op, L); break;
-                    case 4: tile_dense<T2, 4>(tile, mat, op, L); break;
-                    default: break;
+        for (uint32_t o0 = 0, cnt; o0 < d.num_ops; o0 += cnt) {
+            cnt = held;
+            if (held < d.num_ops) cnt = load_ops(o0);
+            const uint32_t first = uniform(lops[0].coef_off);
+            for (uint32_t o = 0; o < cnt; o++) {
+                const StageOp &op = lops[o];
+                const uint64_t gm = ((uint64_t)uniform(op.gc_mask >> 32) << 32) | uniform((uint32_t)op.gc_mask);
+                const uint64_t gv = ((uint64_t)uniform(op.gc_val >> 32) << 32) | uniform((uint32_t)op.gc_val);
+                if ((base & gm) != gv) continue;
+                const T2 *const m = mat + (uniform(op.coef_off) - first);
+                if (uniform(op.kind) == OP_DENSE) {
+                    switch (uniform(op.k)) {
+                        case 1: tile_dense<T2, 1, LOG_THREADS>(tile, m, op, L); break;
+                        case 2: tile_dense<T2, 2, LOG_THREADS>(tile, m, op, L); break;
+                        case 3: tile_dense<T2, 3, LOG_THREADS>(tile, m, op, L); break;
+                        case 4: tile_dense<T2, 4, LOG_THREADS>(tile, m, op, L); break;
+                        default: break;
+                    }
+                } else {
+                    tile_diag<T2, LOG_THREADS>(tile, m, op, L, base);
                 }
-            } else {
-                tile_diag(tile, mat, op, L, base);
+                __syncthreads();
             }
-            __syncthreads();
+            // A skipped op leaves no barrier behind: the next records may be
+            // written only when every wave has read these.
+            if (held < d.num_ops) __syncthreads();
         }
-        for (uint32_t m = 0; m < tsize; m += STAGE_THREADS) {
+        for (uint32_t m = 0; m < tsize; m += THREADS) {
             uint64_t moff = 0;
             for (uint32_t j = lowbits; j < L; j++) moff |= (uint64_t)((m >> j) & 1) << d.local_pos[j];
             if (active) s[base + moff + toff] = tile[m + tid];
@@ -1124,12 +1239,40 @@ void launch_diag(T2 *s, uint64_t len, uint32_t k, const DiagTargets &t, uint64_t
 
 template <typename T2>
 size_t stage_lds_bytes(uint32_t L) {
-    return (sizeof(T2) << L) + sizeof(T2) * 256;
+    return (sizeof(T2) << L) + STAGE_COEF_BYTES + STAGE_OPS * sizeof(StageOp);
 }
 
+template <typename T2, int LOG_THREADS>
+static hipError_t stage_launch(T2 *s, const StageDesc &d, const StageOp *ops, const T2 *coefs, unsigned grid,
+                               hipStream_t st) {
+    const size_t lds = stage_lds_bytes<T2>(d.L);
+    if (lds > 64 * 1024) {
+        // Once per device: the largest tile's LDS.
+        static std::atomic<uint64_t> attr_set{0};
+        int dev = 0;
+        hipError_t e = hipGetDevice(&dev);
+        if (e != hipSuccess) return e;
+        const uint64_t bit = uint64_t(1) << (dev & 63);
+        if (!(attr_set.load() & bit)) {
+            e = hipFuncSetAttribute((const void *)k_stage<T2, LOG_THREADS>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                    (int)stage_lds_bytes<T2>(sizeof(T2) == 8 ? 14 : 13));
+            if (e != hipSuccess) return e;
+            attr_set.fetch_or(bit);
+        }
+    }
+    k_stage<T2, LOG_THREADS><<<grid, 1u << LOG_THREADS, lds, st>>>(s, d, ops, coefs);
+    return hipGetLastError();
+}
+
+// A wave for tiles of up to 2^6 amplitudes (its barriers cost nothing), 4 up
+// to 2^9, 16 above: one tile's ops are a chain, so the more threads an op has, the
+// shorter it is, down to an amplitude or two a thread.
 template <typename T2>
-void launch_stage(T2 *s, const StageDesc &d, const StageOp *ops, const T2 *coefs, unsigned grid, hipStream_t st) {
-    k_stage<T2><<<grid, STAGE_THREADS, stage_lds_bytes<T2>(d.L), st>>>(s, d, ops, coefs);
+hipError_t launch_stage(T2 *s, const StageDesc &d, const StageOp *ops, const T2 *coefs, unsigned grid,
+                        hipStream_t st) {
+    if (d.L <= 6) return stage_launch<T2, 6>(s, d, ops, coefs, grid, st);
+    if (d.L <= 9) return stage_launch<T2, 8>(s, d, ops, coefs, grid, st);
+    return stage_launch<T2, 10>(s, d, ops, coefs, grid, st);
 }
 
 // One block while the whole sum is a few batches of loads per thread (up to
@@ -1316,7 +1459,8 @@ hipError_t launch_sample_walk(const T2 *s, uint64_t len, uint64_t chunk, uint64_
     template void launch_diag<T2>(T2 *, uint64_t, uint32_t, const DiagTargets &, uint64_t, uint64_t, const T2 *, \
                                   hipStream_t);                                                                 \
     template size_t stage_lds_bytes<T2>(uint32_t);                                                              \
-    template void launch_stage<T2>(T2 *, const StageDesc &, const StageOp *, const T2 *, unsigned, hipStream_t); \
+    template hipError_t launch_stage<T2>(T2 *, const StageDesc &, const StageOp *, const T2 *, unsigned,        \
+                                         hipStream_t);                                                          \
     template void launch_norm<T2>(const T2 *, uint64_t, int, double *, double *, hipStream_t);                  \
     template void launch_expect_z<T2>(const T2 *, uint32_t, double *, double *, double *, hipStream_t);         \
     template void launch_probabilities<T2>(const T2 *, uint64_t, double *, hipStream_t);                        \
