@@ -506,10 +506,19 @@ struct LaunchTimer {
     }
 };
 
+// A register-tile stage's program (every stage starts with no pending
+// diagonals: the previous one ends with a scale that applies them).
+std::shared_ptr<StageProgram> build_program(const Stage &st, uint32_t n, const VGeom &vg) {
+    auto prog = std::make_shared<StageProgram>();
+    PendingDiag pend(n);
+    prog->p = build_vprogram(st, n, vg, pend, prog->coefs, prog->ldsops, prog->ints, true);
+    return prog;
+}
+
 // Runs a plan on the state. zero: the qubits known to be |0> before it (all
 // of them when the state is a pending |0...0>); returns those after it.
 template <typename T2>
-uint64_t run_plan(qvd_sv *sv, T2 *s, const std::vector<Step> &steps, qvd_stats &st, uint32_t flags, uint64_t zero,
+uint64_t run_plan(qvd_sv *sv, T2 *s, std::vector<Step> &steps, qvd_stats &st, uint32_t flags, uint64_t zero,
                   uint32_t fixed_lanes) {
     const bool timing = (flags & QVD_FLAG_TIMING) != 0;
     LaunchTimer timer;
@@ -519,14 +528,12 @@ uint64_t run_plan(qvd_sv *sv, T2 *s, const std::vector<Step> &steps, qvd_stats &
     std::vector<StageOp> sops;
     std::vector<T2> coefs;
     std::vector<StageDesc> descs;
-    // Register-tile stages: programs, their coefficients (complex128 until
-    // upload), LDS ops and integer tables.
-    std::vector<VInstr> vins;
-    std::vector<C64> vco;
-    std::vector<StageOp> vlds;
-    std::vector<uint32_t> vints;
+    // Register-tile stages: descriptors, and where each one's program,
+    // coefficients, LDS ops and integer table lie in the upload.
     std::vector<VStageDesc> vdescs;
-    PendingDiag pend(sv->n);
+    struct Parts { size_t ins, co, lds, ints; };
+    std::vector<Parts> vparts;
+    Upload up;
     VGeom geom = vstage_geom<T2>();
     if (fixed_lanes) geom.f_bits = fixed_lanes;
     const bool skip_zero = (flags & QVD_FLAG_ALL_TILES) == 0;
@@ -550,16 +557,18 @@ uint64_t run_plan(qvd_sv *sv, T2 *s, const std::vector<Step> &steps, qvd_stats &
         pending = false;
         stale = 0;
     }
-    for (const Step &step : steps) {
+    for (Step &step : steps) {
         if (!step.is_stage) {
             zero = after_op(zero, step.op);
             st.other_bytes += 2 * state_bytes;
             continue;
         }
         if (step.stage.reg_tile) {
-            VProgram p = build_vprogram(step.stage, sv->n, geom, pend, vco, vlds, vints, true);
+            if (!step.program) step.program = build_program(step.stage, sv->n, geom);
+            StageProgram &prog = *step.program;
+            VProgram &p = prog.p;
             require(p.desc.ccount * sizeof(T2) <= VCONST_BYTES, "internal: stage coefficients exceed the LDS budget");
-            p.desc.instr_off = (uint32_t)vins.size();
+            p.desc.instr_off = 0;
             uint64_t glob = 0;  // the stage's non-tile qubits
             for (uint32_t j = 0; j < p.desc.nglob; j++) glob |= uint64_t(1) << p.desc.glob_pos[j];
             const uint64_t dropped = skip_zero ? drop_zero_tiles(p.desc, zero) : 0;
@@ -574,8 +583,12 @@ uint64_t run_plan(qvd_sv *sv, T2 *s, const std::vector<Step> &steps, qvd_stats &
             }
             if (all_reg) stale = skip_zero ? glob & zero : 0;
             st.stage_bytes += (sizeof(T2) << p.desc.L) * (p.desc.num_tiles + stage_read_tiles(p.desc));
-            vins.insert(vins.end(), p.instr.begin(), p.instr.end());
+            std::vector<T2> co(prog.coefs.size());
+            for (size_t i = 0; i < co.size(); i++) co[i] = to_t2<T2>(prog.coefs[i]);
+            inline_coefficients(p.instr, co);
+            inline_phase_records(p.instr, prog.ints, co);
             vdescs.push_back(p.desc);
+            vparts.push_back({up.put(p.instr), up.put(co), up.put(prog.ldsops), up.put(prog.ints)});
         } else {
             StageDesc d;
             lower_stage<T2>(step.stage, sv->n, sops, coefs, d);
@@ -594,15 +607,9 @@ uint64_t run_plan(qvd_sv *sv, T2 *s, const std::vector<Step> &steps, qvd_stats &
         materialize(sv);
         st.other_bytes += unwritten * sizeof(T2);
     }
-    std::vector<T2> vco_t(vco.size());
-    for (size_t i = 0; i < vco.size(); i++) vco_t[i] = to_t2<T2>(vco[i]);
-    inline_coefficients(vins, vco_t);
-    inline_phase_records(vins, vints, vco_t);
     // Everything the launches read goes up in one copy into the handle's
     // plan arena (kept between calls), full-state ops' coefficients included.
-    Upload up;
-    const size_t o_ops = up.put(sops), o_coef = up.put(coefs), o_vins = up.put(vins), o_vco = up.put(vco_t);
-    const size_t o_vlds = up.put(vlds), o_vints = up.put(vints), o_vdescs = up.put(vdescs);
+    const size_t o_ops = up.put(sops), o_coef = up.put(coefs), o_vdescs = up.put(vdescs);
     std::vector<size_t> o_full;
     for (const Step &step : steps)
         if (!step.is_stage) o_full.push_back(up.put(full_coefficients<T2>(step.op)));
@@ -611,10 +618,6 @@ uint64_t run_plan(qvd_sv *sv, T2 *s, const std::vector<Step> &steps, qvd_stats &
     sv->stale_qubits = stale;
     const StageOp *dops = reinterpret_cast<const StageOp *>(base + o_ops);
     const T2 *dcoef = reinterpret_cast<const T2 *>(base + o_coef);
-    const VInstr *dvins = reinterpret_cast<const VInstr *>(base + o_vins);
-    const T2 *dvco = reinterpret_cast<const T2 *>(base + o_vco);
-    const StageOp *dvlds = reinterpret_cast<const StageOp *>(base + o_vlds);
-    const uint32_t *dvints = reinterpret_cast<const uint32_t *>(base + o_vints);
     const VStageDesc *dvdescs = reinterpret_cast<const VStageDesc *>(base + o_vdescs);
     size_t fi = 0;
     const int cus = num_cus(sv->device);
@@ -627,7 +630,11 @@ uint64_t run_plan(qvd_sv *sv, T2 *s, const std::vector<Step> &steps, qvd_stats &
             const unsigned grid = (unsigned)std::min<uint64_t>(d.num_tiles, (uint64_t)cus);
             timer.begin(timer.stage);
             reg_launch.push_back(1);
-            QVD_HIP(launch_vstage<T2>(s, dvdescs + vi, 1, nullptr, dvins, dvco, dvlds, dvints, grid, sv->stream,
+            const Parts &pt = vparts[vi];
+            QVD_HIP(launch_vstage<T2>(s, dvdescs + vi, 1, nullptr, reinterpret_cast<const VInstr *>(base + pt.ins),
+                                      reinterpret_cast<const T2 *>(base + pt.co),
+                                      reinterpret_cast<const StageOp *>(base + pt.lds),
+                                      reinterpret_cast<const uint32_t *>(base + pt.ints), grid, sv->stream,
                                       d.from_zero != 0 || d.zero_mem != 0, geom.f_bits));
             vi++;
             timer.end(timer.stage);
@@ -677,16 +684,9 @@ uint64_t state_cap_bytes() {
     return std::strtoull(e, nullptr, 10);
 }
 
-// Coefficient bytes the register-tile program of one stage needs in LDS
-// (every stage starts with no pending diagonals: the previous one ends with
-// a scale that applies them).
-size_t stage_coef_bytes(const Stage &st, uint32_t n, int precision, const VGeom &vg) {
-    PendingDiag pend(n);
-    std::vector<C64> co;
-    std::vector<StageOp> lds;
-    std::vector<uint32_t> ints;
-    const VProgram p = build_vprogram(st, n, vg, pend, co, lds, ints, true);
-    return (size_t)p.desc.ccount * (precision == QVD_C64 ? sizeof(float2) : sizeof(double2));
+// Coefficient bytes a register-tile program needs in LDS.
+size_t coef_bytes(const StageProgram &prog, int precision) {
+    return (size_t)prog.p.desc.ccount * (precision == QVD_C64 ? sizeof(float2) : sizeof(double2));
 }
 
 // Splits register-tile stages whose programs would need more coefficients
@@ -697,7 +697,8 @@ size_t stage_coef_bytes(const Stage &st, uint32_t n, int precision, const VGeom 
 std::vector<Step> split_for_coefficients(std::vector<Step> steps, uint32_t n, int precision, const VGeom &vg) {
     std::vector<Step> out;
     for (Step &s : steps) {
-        if (!s.is_stage || !s.stage.reg_tile || stage_coef_bytes(s.stage, n, precision, vg) <= VCONST_BYTES) {
+        if (s.is_stage && s.stage.reg_tile) s.program = build_program(s.stage, n, vg);  // run_plan's too
+        if (!s.program || coef_bytes(*s.program, precision) <= VCONST_BYTES) {
             out.push_back(std::move(s));
             continue;
         }
@@ -709,7 +710,7 @@ std::vector<Step> split_for_coefficients(std::vector<Step> steps, uint32_t n, in
             part.stage.role_policy = s.stage.role_policy;
             auto fits = [&](size_t k) {
                 part.stage.ops.assign(rest.begin(), rest.begin() + (ptrdiff_t)k);
-                return stage_coef_bytes(part.stage, n, precision, vg) <= VCONST_BYTES;
+                return coef_bytes(*build_program(part.stage, n, vg), precision) <= VCONST_BYTES;
             };
             size_t lo = 1, hi = rest.size();
             require(fits(1), "internal: one op's coefficients exceed the LDS budget of a stage");
@@ -975,13 +976,13 @@ std::vector<Step> make_plan(uint32_t n, int precision, const qvd_op *ops, uint64
     }
     require(opt.variant < PLAN_VARIANTS, "plan variant out of range");
     p.variant = opt.variant;
-    if (!p.reg_tile) return plan_heuristic(v, p);
+    if (!p.reg_tile) return plan_heuristic(std::move(v), p);
     require(opt.planner <= QVD_PLANNER_LEARNED_ANY, "unknown planner");
     std::unique_lock<std::mutex> lock(g_model.mu);
     if (opt.planner == QVD_PLANNER_HEURISTIC || !g_model.net) {
         lock.unlock();
         if (chosen) *chosen = p.variant;
-        return split_for_coefficients(plan_heuristic(v, p), n, precision, vg);
+        return split_for_coefficients(plan_heuristic(std::move(v), p), n, precision, vg);
     }
     const bool same_amplitudes = opt.planner == QVD_PLANNER_LEARNED;
     // Learned: a choice made for the same ops before is reused.
@@ -990,7 +991,7 @@ std::vector<Step> make_plan(uint32_t n, int precision, const qvd_op *ops, uint64
     if (hit != g_model.chosen.end()) {
         p.variant = hit->second;
         if (chosen) *chosen = p.variant;
-        return split_for_coefficients(plan_heuristic(v, p), n, precision, vg);
+        return split_for_coefficients(plan_heuristic(std::move(v), p), n, precision, vg);
     }
     // Otherwise every variant is planned (in parallel; identical plans are
     // scored once). QVD_PLANNER_LEARNED keeps the variants whose plan image

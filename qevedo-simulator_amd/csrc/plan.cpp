@@ -127,10 +127,29 @@ std::vector<size_t> extract_masked(const std::vector<uint64_t> &qmask, const std
     return taken;
 }
 
+// How many ops extract_masked would take.
+template <typename F>
+size_t count_masked(const std::vector<uint64_t> &qmask, const std::vector<char> &done, F &&can_run) {
+    size_t taken = 0;
+    uint64_t blocked = 0;
+    for (size_t i = 0; i < qmask.size(); i++) {
+        if (done[i]) continue;
+        if (!(qmask[i] & blocked) && can_run(i)) taken++;
+        else blocked |= qmask[i];
+    }
+    return taken;
+}
+
 uint64_t mask_of(const std::vector<uint32_t> &qs) {
     uint64_t m = 0;
     for (uint32_t q : qs) m |= uint64_t(1) << q;
     return m;
+}
+
+std::vector<uint32_t> qubits_of(uint64_t mask) {
+    std::vector<uint32_t> qs;
+    for (; mask; mask &= mask - 1) qs.push_back((uint32_t)__builtin_ctzll(mask));
+    return qs;
 }
 
 }  // namespace
@@ -146,7 +165,7 @@ std::vector<Step> plan_unblocked(const std::vector<Op> &ops, uint32_t max_fused)
     return steps;
 }
 
-std::vector<Step> plan_heuristic(const std::vector<Op> &ops, const PlanParams &p) {
+std::vector<Step> plan_heuristic(std::vector<Op> ops, const PlanParams &p) {
     const uint32_t n = p.num_qubits;
     const size_t max_fused = std::max<uint32_t>(p.max_fused, 1);
     std::vector<Step> steps;
@@ -154,20 +173,15 @@ std::vector<Step> plan_heuristic(const std::vector<Op> &ops, const PlanParams &p
     const uint32_t L = std::min(p.tile_bits, n);
     const uint32_t contig = std::min(p.contig, L);
     require(n <= 64, "internal: the planner's qubit masks hold 64 qubits");
-    std::vector<char> is_local(n, 0);
-    std::vector<uint32_t> local;
-    for (uint32_t q = 0; q < L; q++) {
-        local.push_back(q);
-        is_local[q] = 1;
-    }
+    uint64_t local = L >= 64 ? ~uint64_t(0) : (uint64_t(1) << L) - 1;  // the tile's qubits
     // Every op's qubits and targets as masks, and whether it may run in a
     // tile at all (diagonal, or dense and narrow enough for the in-tile
     // kernel).
     std::vector<uint64_t> qmask(ops.size()), tmask(ops.size());
     std::vector<char> stageable(ops.size());
     for (size_t i = 0; i < ops.size(); i++) {
-        qmask[i] = mask_of(ops[i].qubits());
-        tmask[i] = mask_of(ops[i].targets);
+        tmask[i] = qmask[i] = mask_of(ops[i].targets);
+        for (auto &c : ops[i].controls) qmask[i] |= uint64_t(1) << c.first;
         stageable[i] = ops[i].diagonal || ops[i].targets.size() <= p.max_stage_op;
     }
     const uint64_t low = contig >= 64 ? ~uint64_t(0) : (uint64_t(1) << contig) - 1;
@@ -180,31 +194,29 @@ std::vector<Step> plan_heuristic(const std::vector<Op> &ops, const PlanParams &p
     // Coupling graph of the circuit (qubits that share an op), for the
     // region candidates (variant bit 4 clear).
     const bool regions = (p.variant & 16) == 0;
-    std::vector<std::vector<uint32_t>> adj;
+    std::vector<uint64_t> adj;
     if (regions) {
-        adj.assign(n, {});
-        for (const Op &op : ops) {
-            const std::vector<uint32_t> qs = op.qubits();
-            for (uint32_t a : qs)
-                for (uint32_t b : qs)
-                    if (a != b && !contains(adj[a], b)) adj[a].push_back(b);
-        }
-        for (auto &nb : adj) std::sort(nb.begin(), nb.end());
+        adj.assign(n, 0);
+        for (uint64_t m : qmask)
+            for (uint64_t r = m; r; r &= r - 1) {
+                const uint32_t a = (uint32_t)__builtin_ctzll(r);
+                adj[a] |= m & ~(uint64_t(1) << a);
+            }
     }
     std::vector<char> done(ops.size(), 0);
     size_t remaining = ops.size();
     while (remaining > 0) {
-        const uint64_t local_mask = mask_of(local);
-        std::vector<size_t> taken = extract_masked(qmask, done, [&](size_t i) { return runs_under(i, local_mask); });
+        std::vector<size_t> taken = extract_masked(qmask, done, [&](size_t i) { return runs_under(i, local); });
         if (!taken.empty()) {
             std::vector<Op> stage_ops;
+            stage_ops.reserve(taken.size());
             for (size_t i : taken) {
                 done[i] = 1;
-                stage_ops.push_back(ops[i]);
+                stage_ops.push_back(std::move(ops[i]));  // only its masks are read from here on
             }
             remaining -= taken.size();
             Step s;
-            s.stage.local = local;
+            s.stage.local = qubits_of(local);
             s.stage.reg_tile = p.reg_tile;
             s.stage.role_policy = (p.variant & 8) ? 0 : 1;
             if (p.reg_tile) {
@@ -217,7 +229,7 @@ std::vector<Step> plan_heuristic(const std::vector<Op> &ops, const PlanParams &p
                 // diagonal target into a dense matrix would need it in the tile.
                 s.stage.ops = fuse_where(stage_ops, std::min<size_t>(max_fused, p.max_stage_op), [&](const Op &op) {
                     for (uint32_t q : op.qubits())
-                        if (!is_local[q]) return false;
+                        if (!((local >> q) & 1)) return false;
                     return true;
                 });
             }
@@ -229,7 +241,7 @@ std::vector<Step> plan_heuristic(const std::vector<Op> &ops, const PlanParams &p
         const uint32_t full_cap = L - contig;
         auto wanted_set = [&](uint32_t capacity) {
             uint64_t wanted = 0;
-            extract_masked(qmask, done, [&](size_t i) {
+            count_masked(qmask, done, [&](size_t i) {
                 if (ops[i].diagonal) return true;
                 if (!stageable[i]) return false;
                 const uint64_t fresh = tmask[i] & ~low & ~wanted;
@@ -237,29 +249,28 @@ std::vector<Step> plan_heuristic(const std::vector<Op> &ops, const PlanParams &p
                 wanted |= fresh;
                 return true;
             });
-            std::vector<uint32_t> qs;
-            for (uint32_t q = 0; q < n; q++)
-                if ((wanted >> q) & 1) qs.push_back(q);
-            return qs;
+            return wanted;
         };
-        auto tile_of = [&](const std::vector<uint32_t> &wanted) {
-            std::vector<uint32_t> next;
-            for (uint32_t q = 0; q < contig; q++) next.push_back(q);
-            for (uint32_t q : wanted) next.push_back(q);
-            for (uint32_t q = contig; q < n && next.size() < L; q++)
-                if (!contains(next, q)) next.push_back(q);
-            std::sort(next.begin(), next.end());
+        // The lowest `contig` qubits, the wanted ones, and the lowest others
+        // up to the tile's size.
+        auto tile_of = [&](uint64_t wanted) {
+            uint64_t next = low | wanted;
+            uint32_t size = (uint32_t)__builtin_popcountll(next);
+            for (uint32_t q = contig; q < n && size < L; q++)
+                if (!((next >> q) & 1)) {
+                    next |= uint64_t(1) << q;
+                    size++;
+                }
             return next;
         };
+        auto runnable = [&](uint64_t tile) {
+            return count_masked(qmask, done, [&](size_t i) { return runs_under(i, tile); });
+        };
         const uint32_t cut = std::min<uint32_t>(p.variant & 3, full_cap > 1 ? full_cap - 1 : 0);
-        std::vector<uint32_t> next = tile_of(wanted_set(full_cap - cut));
+        uint64_t next = tile_of(wanted_set(full_cap - cut));
         if (p.variant & 4) {
             // The candidate tile that runs the most pending ops next.
-            auto runnable_count = [&](const std::vector<uint32_t> &tile) {
-                const uint64_t tm = mask_of(tile);
-                return extract_masked(qmask, done, [&](size_t i) { return runs_under(i, tm); }).size();
-            };
-            std::vector<std::vector<uint32_t>> cands;
+            std::vector<uint64_t> cands;
             for (uint32_t c = full_cap; c >= 1 && c + 4 > full_cap; c--) cands.push_back(tile_of(wanted_set(c)));
             // the most-targeted qubits among the next pending dense ops
             std::vector<uint32_t> count(n, 0), first(n, UINT32_MAX);
@@ -280,11 +291,11 @@ std::vector<Step> plan_heuristic(const std::vector<Op> &ops, const PlanParams &p
                 return count[a] != count[b] ? count[a] > count[b] : first[a] < first[b];
             });
             if (byuse.size() > full_cap) byuse.resize(full_cap);
-            cands.push_back(tile_of(byuse));
-            size_t best = next == local ? 0 : runnable_count(next);
-            for (const auto &cnd : cands) {
+            cands.push_back(tile_of(mask_of(byuse)));
+            size_t best = next == local ? 0 : runnable(next);
+            for (uint64_t cnd : cands) {
                 if (cnd == local) continue;
-                const size_t k = runnable_count(cnd);
+                const size_t k = runnable(cnd);
                 if (k > best) {
                     best = k;
                     next = cnd;
@@ -298,27 +309,24 @@ std::vector<Step> plan_heuristic(const std::vector<Op> &ops, const PlanParams &p
             // candidate (with the lookahead's) under which the most pending
             // ops run now, so the tiles sweep the circuit's light cones
             // instead of chasing its earliest pending op.
-            auto runnable = [&](const std::vector<uint32_t> &tile) {
-                const uint64_t tm = mask_of(tile);
-                return extract_masked(qmask, done, [&](size_t i) { return runs_under(i, tm); }).size();
-            };
-            std::vector<std::vector<uint32_t>> cands{next};
+            std::vector<uint64_t> cands{next};
             for (uint32_t seed = contig; seed < n; seed++) {
                 std::vector<uint32_t> region{seed};
+                uint64_t in = uint64_t(1) << seed;
                 for (size_t i = 0; i < region.size() && region.size() < full_cap; i++)
-                    for (uint32_t w : adj[region[i]]) {
-                        if (region.size() >= full_cap) break;
-                        if (w >= contig && !contains(region, w)) region.push_back(w);
+                    for (uint64_t nb = adj[region[i]] & ~low & ~in; nb && region.size() < full_cap; nb &= nb - 1) {
+                        region.push_back((uint32_t)__builtin_ctzll(nb));
+                        in |= nb & -nb;
                     }
-                std::vector<uint32_t> cand = tile_of(region);
-                if (std::find(cands.begin(), cands.end(), cand) == cands.end()) cands.push_back(std::move(cand));
+                const uint64_t cand = tile_of(in);
+                if (std::find(cands.begin(), cands.end(), cand) == cands.end()) cands.push_back(cand);
             }
             // A region replaces the lookahead's tile only when more pending
             // ops run under it; one under which nothing runs (an op wider
             // than a stage is next) never does, so such an op still gets its
             // own full-state pass below.
             size_t best = next == local ? 0 : runnable(next);
-            for (const auto &cnd : cands) {
+            for (uint64_t cnd : cands) {
                 if (cnd == local) continue;
                 const size_t k = runnable(cnd);
                 if (k > best) {
@@ -337,13 +345,11 @@ std::vector<Step> plan_heuristic(const std::vector<Op> &ops, const PlanParams &p
             remaining--;
             Step s;
             s.is_stage = false;
-            s.op = ops[i];
+            s.op = std::move(ops[i]);
             steps.push_back(std::move(s));
             continue;
         }
         local = next;
-        std::fill(is_local.begin(), is_local.end(), 0);
-        for (uint32_t q : local) is_local[q] = 1;
     }
     return steps;
 }

@@ -11,6 +11,7 @@
 #pragma once
 
 #include <cstdint>
+#include <memory>
 #include <vector>
 
 #include "common.h"
@@ -34,10 +35,12 @@ struct Stage {
 
 // One step of a plan: an LDS-tile stage, or a single op applied as its own
 // HBM pass (an op with more non-tile targets than a tile holds).
+struct StageProgram;  // vprog.h
 struct Step {
     bool is_stage = true;
     Stage stage;
     Op op;
+    std::shared_ptr<StageProgram> program;  // a register-tile stage's, once built
 };
 
 struct PlanParams {
@@ -66,7 +69,7 @@ constexpr uint32_t PLAN_VARIANTS = 32;
 
 // The heuristic plan: src/blocking.rs's extract / plan_swaps loop with the
 // lookahead's wanted set becoming the next stage's tile qubits.
-std::vector<Step> plan_heuristic(const std::vector<Op> &ops, const PlanParams &p);
+std::vector<Step> plan_heuristic(std::vector<Op> ops, const PlanParams &p);
 
 // Plan without blocking: fused ops, each its own HBM pass (options.region_bits = None).
 std::vector<Step> plan_unblocked(const std::vector<Op> &ops, uint32_t max_fused);

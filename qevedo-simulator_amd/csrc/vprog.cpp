@@ -108,12 +108,23 @@ struct Gen {
     };
     std::vector<PairPhase> prun;
     std::vector<char> in_run;
+    std::vector<uint64_t> qmask;  // each op's qubits
+    std::vector<int> needs;       // need() of each op
 
     Gen(const Stage &s, uint32_t n_, const VGeom &g_, PendingDiag &p, std::vector<C64> &c, std::vector<StageOp> &l,
         std::vector<uint32_t> &ii)
         : st(s), n(n_), g(g_), pend(p), coefs(c), ldsops(l), ints(ii), tbit(n_, -1), pmat(n_), has_pmat(n_, 0),
           in_run(n_, 0) {
         for (size_t j = 0; j < s.local.size(); j++) tbit[s.local[j]] = (int)j;
+        require(n <= 64, "internal: the program generator's qubit masks hold 64 qubits");
+        for (const Op &op : s.ops) {
+            uint64_t m = 0;
+            for (uint32_t q : op.targets) m |= uint64_t(1) << q;
+            for (auto &c : op.controls) m |= uint64_t(1) << c.first;
+            qmask.push_back(m);
+            needs.push_back(need(op));
+        }
+        out.reserve(2 * s.ops.size() + 8);
     }
 
     // Emits the pending run: as one V_SIGNS when every pair phase is -1
@@ -192,8 +203,11 @@ struct Gen {
     }
 
     bool touches_run(const Op &op) const {
-        for (uint32_t q : op.qubits())
+        if (prun.empty()) return false;
+        for (uint32_t q : op.targets)
             if (in_run[q]) return true;
+        for (auto &c : op.controls)
+            if (in_run[c.first]) return true;
         return false;
     }
 
@@ -439,7 +453,33 @@ struct Gen {
     // per-register and per-tile (non-tile qubit) factors.
     void emit_scale() {
         const uint32_t W = 64u << g.w_bits, R = 1u << g.r_bits;
-        std::vector<C64> ft(W, C64(1, 0)), fr(R, C64(1, 0));
+        // The factors of thread (and register) bits in the order of the qubits:
+        // a table over the bits met so far, doubled by each (bit j of its index
+        // is the j-th bit met), so an entry takes one product per bit set
+        // or clear without the product being formed again for every thread.
+        std::vector<C64> tt{C64(1, 0)}, tr{C64(1, 0)};
+        std::vector<uint32_t> tbits, rbits;
+        auto grow = [&](std::vector<C64> &tab, std::vector<uint32_t> &bits, uint32_t x, uint32_t q) {
+            const size_t m = tab.size();
+            tab.resize(2 * m);
+            for (size_t i = 0; i < m; i++) {
+                tab[m + i] = cmul(tab[i], pend.d1[q]);
+                tab[i] = cmul(tab[i], pend.d0[q]);
+            }
+            bits.push_back(x);
+        };
+        auto spread = [](const std::vector<C64> &tab, const std::vector<uint32_t> &bits, uint32_t count) {
+            std::vector<C64> out(count);
+            std::vector<uint32_t> at(count, 0);
+            uint32_t step[16] = {};
+            for (size_t j = 0; j < bits.size(); j++) step[bits[j]] = 1u << j;
+            out[0] = tab[0];
+            for (uint32_t t = 1; t < count; t++) {
+                at[t] = at[t & (t - 1)] | step[__builtin_ctz(t)];
+                out[t] = tab[at[t]];
+            }
+            return out;
+        };
         std::vector<uint32_t> globals;
         bool any = false;
         for (uint32_t q = 0; q < n; q++) {
@@ -447,15 +487,12 @@ struct Gen {
             any = true;
             const uint32_t e = encode(q), x = e & 0xffffu;
             switch (e & VT_KIND) {
-                case VT_THREAD:
-                    for (uint32_t t = 0; t < W; t++) ft[t] = cmul(ft[t], ((t >> x) & 1) ? pend.d1[q] : pend.d0[q]);
-                    break;
-                case VT_REG:
-                    for (uint32_t j = 0; j < R; j++) fr[j] = cmul(fr[j], ((j >> x) & 1) ? pend.d1[q] : pend.d0[q]);
-                    break;
+                case VT_THREAD: grow(tt, tbits, x, q); break;
+                case VT_REG: grow(tr, rbits, x, q); break;
                 default: globals.push_back(q);
             }
         }
+        const std::vector<C64> ft = spread(tt, tbits, W), fr = spread(tr, rbits, R);
         if (!any) return;
         VInstr v = blank(V_SCALE);
         v.coef = (uint32_t)coefs.size();
@@ -489,26 +526,16 @@ struct Gen {
         return b >= (int)g.f_bits ? b : -1;
     }
 
-    bool runnable(const Op &op) const {
-        const int b = need(op);
-        return b < 0 || roles.role[b] != ROLE_WAVE;
-    }
+    bool runnable(size_t i) const { return needs[i] < 0 || roles.role[needs[i]] != ROLE_WAVE; }
 
     template <typename F>
     std::vector<size_t> extract(const std::vector<char> &done, F &&can_run) const {
         std::vector<size_t> taken;
-        std::vector<uint32_t> blocked;
+        uint64_t blocked = 0;
         for (size_t i = 0; i < st.ops.size(); i++) {
             if (done[i]) continue;
-            const std::vector<uint32_t> oq = st.ops[i].qubits();
-            bool touches = false;
-            for (uint32_t q : oq) touches |= contains(blocked, q);
-            if (!touches && can_run(st.ops[i])) {
-                taken.push_back(i);
-            } else {
-                for (uint32_t q : oq)
-                    if (!contains(blocked, q)) blocked.push_back(q);
-            }
+            if (!(qmask[i] & blocked) && can_run(i)) taken.push_back(i);
+            else blocked |= qmask[i];
         }
         return taken;
     }
@@ -518,8 +545,8 @@ struct Gen {
     std::vector<uint8_t> lookahead(const std::vector<char> &done) const {
         const size_t cap = g.r_bits + g.flex_lanes();
         std::vector<uint8_t> wanted;
-        extract(done, [&](const Op &op) {
-            const int b = need(op);
+        extract(done, [&](size_t i) {
+            const int b = needs[i];
             if (b < 0 || has(wanted, (uint32_t)b)) return true;
             if (wanted.size() + 1 > cap) return false;
             wanted.push_back((uint8_t)b);
@@ -531,8 +558,7 @@ struct Gen {
             std::vector<uint32_t> uses(st.local.size(), 0);
             for (size_t i = 0; i < st.ops.size(); i++) {
                 if (done[i]) continue;
-                const int b = need(st.ops[i]);
-                if (b >= 0) uses[b]++;
+                if (needs[i] >= 0) uses[needs[i]]++;
             }
             std::stable_sort(wanted.begin(), wanted.end(), [&](uint8_t a, uint8_t b) { return uses[a] > uses[b]; });
         }
@@ -621,7 +647,7 @@ struct Gen {
         for (size_t s = 0; s < r.size(); s++) p.desc.rmap0[s] = r[s];
         size_t remaining = st.ops.size();
         while (remaining) {
-            std::vector<size_t> taken = extract(done, [&](const Op &op) { return runnable(op); });
+            std::vector<size_t> taken = extract(done, [&](size_t i) { return runnable(i); });
             for (size_t i : taken) {
                 done[i] = 1;
                 emit_op(st.ops[i]);

@@ -199,6 +199,14 @@ struct VProgram {
     VStageDesc desc;
 };
 
+// A stage's program with coefficients, LDS ops and integers of its own.
+struct StageProgram {
+    VProgram p;
+    std::vector<C64> coefs;
+    std::vector<StageOp> ldsops;
+    std::vector<uint32_t> ints;
+};
+
 VProgram build_vprogram(const Stage &stage, uint32_t n, const VGeom &g, PendingDiag &pending,
                         std::vector<C64> &coefs, std::vector<StageOp> &ldsops, std::vector<uint32_t> &ints,
                         bool flush_all);

@@ -116,7 +116,7 @@ def lib():
         L.qvd_sv_copy.argtypes = [vp, vp]
         L.qvd_sv_set_amplitudes.argtypes = [vp, P(d), u64]
         L.qvd_sv_get_amplitudes.argtypes = [vp, P(d), u64]
-        L.qvd_sv_apply.argtypes = [vp, P(d), P(u32), u32, P(u32), P(C.c_uint8), u32]
+        L.qvd_sv_apply.argtypes = [vp, vp, vp, u32, vp, vp, u32]  # addresses: a typed pointer per array costs microseconds
         L.qvd_sv_apply_ops.argtypes = [vp, P(Op), u64, P(Options), P(Stats)]
         L.qvd_sv_norm_sqr.argtypes = [vp, P(d)]
         L.qvd_sv_scale.argtypes = [vp, d]
@@ -194,14 +194,26 @@ def gate_matrix(name: str, params=()) -> np.ndarray:
     return out[: 2 * dim * dim].view(np.complex128).reshape(dim, dim).copy()
 
 
+_LOWER_OUT = C.c_double * (2 * 64)
+# ctypes arrays of up to 8 parameters (a new array type costs more than the call).
+_LOWER_PARAMS = tuple(C.c_double * max(k, 1) for k in range(9))
+
+
 def gate_lower(name: str, params=()) -> tuple:
     """(number of leading controls, base matrix) of a named gate."""
-    p = np.ascontiguousarray(params, dtype=np.float64)
-    out = np.zeros(2 * 64, dtype=np.float64)
+    if not isinstance(params, (list, tuple)):
+        params = np.ascontiguousarray(params, dtype=np.float64).reshape(-1).tolist()
+    n = len(params)
+    array = _LOWER_PARAMS[n] if n < len(_LOWER_PARAMS) else C.c_double * n
+    try:
+        p = array(*params)
+    except TypeError:  # what only NumPy turns into a number
+        p = array(*np.ascontiguousarray(params, dtype=np.float64).tolist())
+    out = _LOWER_OUT()
     nc, nt = C.c_uint32(), C.c_uint32()
-    _check(lib().qvd_gate_lower(name.encode(), _p(p, C.c_double), p.size, C.byref(nc), C.byref(nt), _p(out, C.c_double), 64))
+    _check(lib().qvd_gate_lower(name.encode(), p, n, C.byref(nc), C.byref(nt), out, 64))
     dim = 1 << nt.value
-    return nc.value, out[: 2 * dim * dim].view(np.complex128).reshape(dim, dim).copy()
+    return nc.value, np.frombuffer(out, dtype=np.complex128, count=dim * dim).reshape(dim, dim).copy()
 
 
 def lower_gates(gates) -> list:
@@ -218,22 +230,56 @@ def lower_gates(gates) -> list:
     return ops
 
 
+# The C layout of a qvd_op, its pointers as integers.
+_OP = np.dtype([("targets", "u8"), ("num_targets", "u4"), ("pad0", "u4"), ("controls", "u8"), ("control_values", "u8"),
+                ("num_controls", "u4"), ("pad1", "u4"), ("matrix", "u8")])
+assert _OP.itemsize == C.sizeof(Op)
+
+
 class OpArray:
-    """A qvd_op array plus the NumPy buffers it points into."""
+    """A qvd_op array plus the NumPy buffers it points into: all ops' targets,
+    controls and control values in one buffer each, each matrix object once."""
 
     def __init__(self, ops):
-        self.keep = []
         self.n = len(ops)
-        self.arr = (Op * max(self.n, 1))()
-        for i, (targets, controls, matrix) in enumerate(ops):
-            t = np.ascontiguousarray(targets, dtype=np.uint32)
-            cq = np.ascontiguousarray([c[0] for c in controls], dtype=np.uint32)
-            cv = np.ascontiguousarray([1 if c[1] else 0 for c in controls], dtype=np.uint8)
-            m = np.ascontiguousarray(matrix, dtype=np.complex128)
-            if m.shape != (1 << t.size, 1 << t.size):
-                raise ValueError(f"a gate on {t.size} qubits needs a {1 << t.size}x{1 << t.size} matrix")
-            self.keep += [t, cq, cv, m]
-            self.arr[i] = Op(_p(t, C.c_uint32), t.size, _p(cq, C.c_uint32), _p(cv, C.c_uint8), cq.size, _p(m.view(np.float64), C.c_double))
+        matrices = {}  # id -> (address, rows); self.keep holds the arrays
+        self.keep = []
+        qubits, values, counts, addresses = [], [], [], []
+        for targets, controls, matrix in ops:
+            if not isinstance(targets, (list, tuple)):
+                targets = np.ascontiguousarray(targets, dtype=np.uint32).reshape(-1).tolist()
+            entry = matrices.get(id(matrix))
+            if entry is None:
+                m = np.ascontiguousarray(matrix, dtype=np.complex128)
+                # `matrix` too, so that its id stays its own
+                self.keep += [matrix, m]
+                entry = matrices[id(matrix)] = (m.ctypes.data, m.shape)
+            dim = 1 << len(targets)
+            if entry[1] != (dim, dim):
+                raise ValueError(f"a gate on {len(targets)} qubits needs a {dim}x{dim} matrix")
+            qubits += targets
+            counts.append(len(targets))
+            counts.append(len(controls))
+            addresses.append(entry[0])
+            for c in controls:
+                qubits.append(c[0])
+                values.append(1 if c[1] else 0)
+        qubits = np.array(qubits, dtype=np.uint32)
+        values = np.array(values, dtype=np.uint8)
+        counts = np.array(counts, dtype=np.uint64).reshape(-1, 2)
+        rec = np.zeros(max(self.n, 1), dtype=_OP)
+        if self.n:
+            first = np.zeros(2 * self.n, dtype=np.uint64)  # of each op's targets and controls in `qubits`
+            np.cumsum(counts.reshape(-1)[:-1], out=first[1:])
+            value = np.zeros(self.n, dtype=np.uint64)
+            np.cumsum(counts[:-1, 1], out=value[1:])
+            at = np.uint64(qubits.ctypes.data) + np.uint64(4) * first
+            rec["targets"], rec["controls"] = at[0::2], at[1::2]
+            rec["control_values"] = np.uint64(values.ctypes.data) + value
+            rec["num_targets"], rec["num_controls"] = counts[:, 0], counts[:, 1]
+            rec["matrix"] = addresses
+        self.keep += [qubits, values, rec]
+        self.arr = (Op * max(self.n, 1)).from_buffer(rec)
 
 
 def plan_features(num_qubits: int, ops, precision: str = "single", variant: int = 0,
@@ -355,9 +401,12 @@ class StateVector:
     def apply(self, matrix, targets, controls=()) -> None:
         m = np.ascontiguousarray(matrix, dtype=np.complex128)
         t = np.ascontiguousarray(targets, dtype=np.uint32)
+        if not len(controls):
+            _check(lib().qvd_sv_apply(self.h, m.ctypes.data, t.ctypes.data, t.size, None, None, 0))
+            return
         cq = np.ascontiguousarray([c[0] for c in controls], dtype=np.uint32)
         cv = np.ascontiguousarray([1 if c[1] else 0 for c in controls], dtype=np.uint8)
-        _check(lib().qvd_sv_apply(self.h, _p(m.view(np.float64), C.c_double), _p(t, C.c_uint32), t.size, _p(cq, C.c_uint32), _p(cv, C.c_uint8), cq.size))
+        _check(lib().qvd_sv_apply(self.h, m.ctypes.data, t.ctypes.data, t.size, cq.ctypes.data, cv.ctypes.data, cq.size))
 
     def apply_ops(self, ops, max_fused_qubits: int = 4, tile_bits: int | None = 0, planner: int = PLANNER_HEURISTIC,
                   timing: bool = False, variant: int = 0, dense_valu: bool = False, all_tiles: bool = False,
