@@ -531,7 +531,7 @@ uint64_t run_plan(qvd_sv *sv, T2 *s, std::vector<Step> &steps, qvd_stats &st, ui
     // Register-tile stages: descriptors, and where each one's program,
     // coefficients, LDS ops and integer table lie in the upload.
     std::vector<VStageDesc> vdescs;
-    struct Parts { size_t ins, co, lds, ints; };
+    struct Parts { size_t ins, co, lds, ints; bool half; };
     std::vector<Parts> vparts;
     Upload up;
     VGeom geom = vstage_geom<T2>();
@@ -588,7 +588,9 @@ uint64_t run_plan(qvd_sv *sv, T2 *s, std::vector<Step> &steps, qvd_stats &st, ui
             inline_coefficients(p.instr, co);
             inline_phase_records(p.instr, prog.ints, co);
             vdescs.push_back(p.desc);
-            vparts.push_back({up.put(p.instr), up.put(co), up.put(prog.ldsops), up.put(prog.ints)});
+            vparts.push_back({up.put(p.instr), up.put(co), up.put(prog.ldsops), up.put(prog.ints),
+                              sizeof(T2) == 16 && prog.ldsops.empty() && geom.f_bits == vstage_geom<T2>().f_bits &&
+                                  vstage_half(p.desc.num_tiles, p.desc.ccount, (unsigned)num_cus(sv->device))});
         } else {
             StageDesc d;
             lower_stage<T2>(step.stage, sv->n, sops, coefs, d);
@@ -627,15 +629,15 @@ uint64_t run_plan(qvd_sv *sv, T2 *s, std::vector<Step> &steps, qvd_stats &st, ui
         if (step.is_stage && step.stage.reg_tile) {
             const VStageDesc &d = vdescs[vi];
             st.kernels += step.stage.ops.size();
-            const unsigned grid = (unsigned)std::min<uint64_t>(d.num_tiles, (uint64_t)cus);
+            const Parts &pt = vparts[vi];
+            const unsigned grid = (unsigned)std::min<uint64_t>(d.num_tiles, (uint64_t)cus * (pt.half ? 2 : 1));
             timer.begin(timer.stage);
             reg_launch.push_back(1);
-            const Parts &pt = vparts[vi];
             QVD_HIP(launch_vstage<T2>(s, dvdescs + vi, 1, nullptr, reinterpret_cast<const VInstr *>(base + pt.ins),
                                       reinterpret_cast<const T2 *>(base + pt.co),
                                       reinterpret_cast<const StageOp *>(base + pt.lds),
                                       reinterpret_cast<const uint32_t *>(base + pt.ints), grid, sv->stream,
-                                      d.from_zero != 0 || d.zero_mem != 0, geom.f_bits));
+                                      d.from_zero != 0 || d.zero_mem != 0, geom.f_bits, pt.half, d.ccount));
             vi++;
             timer.end(timer.stage);
             st.stages++;

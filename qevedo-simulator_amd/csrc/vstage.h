@@ -16,10 +16,16 @@ template <typename T2> size_t vstage_lds_bytes();
 // be null when ndesc == 1). All pointers are device pointers. lazy_zero: a
 // descriptor may have from_zero set (its tiles are made, not loaded) or
 // stale qubits in zero_mem (their amplitudes are set to zero, not loaded).
+// half (one descriptor, default geometry, no LDS ops, complex128): the kernel
+// whose LDS tile holds one part of the amplitudes, launched with room for
+// ccount coefficients.
 template <typename T2>
 hipError_t launch_vstage(T2 *s, const VStageDesc *descs, uint32_t ndesc, const uint32_t *block_start,
                          const VInstr *prog, const T2 *coefs, const StageOp *ldsops, const uint32_t *ints, unsigned grid,
-                         hipStream_t st, bool lazy_zero = false, uint32_t fixed_lanes = 0);
+                         hipStream_t st, bool lazy_zero, uint32_t fixed_lanes, bool half, uint32_t ccount);
+// Whether a complex128 stage of ccount coefficients and num_tiles tiles runs
+// there: two workgroups fit on a CU, and there are tiles for two on each.
+bool vstage_half(uint64_t num_tiles, uint32_t ccount, unsigned cus);
 
 // One item of a stage queue: tiles tile0, tile0 + step, ... (count of them)
 // of stage `desc`, which belongs to state `state` and may start once that

@@ -9,7 +9,8 @@
 // program (vprog.h) on each of its tiles: one switch per instruction on the
 // handler the host resolved it to. The complex128 geometry (2 waves per
 // SIMD) prefetches the next tile into a second register set; the complex64
-// one (4 waves per SIMD) relies on the other waves to cover a tile's loads.
+// one (4 waves per SIMD), and two complex128 groups on a CU (HALF), rely on the
+// other waves to cover a tile's loads.
 //
 // Coefficients indexed per lane (diagonal tables, scale tables, LDS-op
 // matrices) are copied to LDS once per workgroup; per-instruction uniform
@@ -51,6 +52,12 @@ __device__ __forceinline__ uint32_t cbyte(const QVD_CONST uint8_t *p, uint32_t i
 
 __device__ __forceinline__ float fma_(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
 __device__ __forceinline__ double fma_(double a, double b, double c) { return __builtin_fma(a, b, c); }
+
+// v, unknown to the optimiser.
+__device__ __forceinline__ uint32_t opaque(uint32_t v) {
+    asm volatile("" : "+v"(v));
+    return v;
+}
 
 template <typename T2>
 __device__ __forceinline__ T2 mk(decltype(T2::x) a, decltype(T2::x) b) {
@@ -617,8 +624,10 @@ __device__ __forceinline__ void inline_coefs(const QVD_CONST VInstr &v, T2 (&c)[
 // loaded; or it may name stale qubits (zero_mem), whose amplitudes it sets to
 // zero instead of loading them. FBC is the number of fixed lane bits, or -1 to read it from the
 // descriptor (it enters only the offsets of the role maps, not the gate
-// handlers).
-template <typename T2, int WB, int RB, int FBC, bool MAY_ZERO>
+// handlers). With HALF the LDS tile holds one part (real or imaginary) of the
+// amplitudes at a time: an exchange moves the parts one after the other, and
+// in-LDS dense ops, which need both, are not available.
+template <typename T2, int WB, int RB, int FBC, bool MAY_ZERO, bool HALF = false>
 __device__ __forceinline__ void stage_tiles(T2 *__restrict__ s, const QVD_CONST VStageDesc &d, uint64_t t_begin,
                                             uint64_t t_end, uint64_t step, const VInstr *__restrict__ prog,
                                             const T2 *__restrict__ coefs, const StageOp *__restrict__ ldsops,
@@ -629,15 +638,18 @@ __device__ __forceinline__ void stage_tiles(T2 *__restrict__ s, const QVD_CONST 
     // kernel's item slot), and a tile at a 4-byte offset would split every
     // 8- and 16-byte LDS access of the exchanges.
     extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
+    using R1 = decltype(T2::x);
     T2 *tile = reinterpret_cast<T2 *>(smem_raw);
-    T2 *cst = tile + (1u << L);  // the stage's coefficients (index = coef - cbegin)
+    R1 *part = reinterpret_cast<R1 *>(smem_raw);  // HALF
+    // the stage's coefficients (index = coef - cbegin)
+    T2 *cst = HALF ? reinterpret_cast<T2 *>(part + (1u << L)) : tile + (1u << L);
     const QVD_CONST VInstr *cprog = (const QVD_CONST VInstr *)prog;
     const QVD_CONST T2 *ccoef = (const QVD_CONST T2 *)coefs;
     const QVD_CONST StageOp *cops = (const QVD_CONST StageOp *)ldsops;
     const QVD_CONST uint32_t *cints = (const QVD_CONST uint32_t *)ints;
-    const uint32_t tid = threadIdx.x, lane = tid & 63;
+    const uint32_t tid_all = threadIdx.x, lane_all = tid_all & 63;
 
-    for (uint32_t i = tid; i < d.ccount; i += W) cst[i] = coefs[d.cbegin + i];
+    for (uint32_t i = tid_all; i < d.ccount; i += W) cst[i] = coefs[d.cbegin + i];
     const T2 *cbase = cst - d.cbegin;  // so cbase[v.coef + i] is the LDS copy
     __syncthreads();
 
@@ -645,18 +657,18 @@ __device__ __forceinline__ void stage_tiles(T2 *__restrict__ s, const QVD_CONST 
     // (stores): thread part per lane, register part per register bit.
     const uint32_t FB = FBC >= 0 ? (uint32_t)FBC : d.fixed_lanes;
     const uint32_t FL = 6 - FB;  // flexible lane bits
-    uint64_t t_off0 = lane & ((1u << FB) - 1), t_offF = t_off0;
+    uint64_t t_off0 = lane_all & ((1u << FB) - 1), t_offF = t_off0;
 #pragma unroll
     for (int s_ = 0; s_ < (int)VMAX_L_FLEX; s_++) {
         if (s_ < (int)FL) {
-            t_off0 |= (uint64_t)((lane >> (FB + s_)) & 1) << d.local_pos[cbyte(d.lmap0, s_)];
-            t_offF |= (uint64_t)((lane >> (FB + s_)) & 1) << d.local_pos[cbyte(d.lmapF, s_)];
+            t_off0 |= (uint64_t)((lane_all >> (FB + s_)) & 1) << d.local_pos[cbyte(d.lmap0, s_)];
+            t_offF |= (uint64_t)((lane_all >> (FB + s_)) & 1) << d.local_pos[cbyte(d.lmapF, s_)];
         }
     }
 #pragma unroll
     for (int s_ = 0; s_ < WB; s_++) {
-        t_off0 |= (uint64_t)((tid >> (6 + s_)) & 1) << d.local_pos[cbyte(d.wmap0, s_)];
-        t_offF |= (uint64_t)((tid >> (6 + s_)) & 1) << d.local_pos[cbyte(d.wmapF, s_)];
+        t_off0 |= (uint64_t)((tid_all >> (6 + s_)) & 1) << d.local_pos[cbyte(d.wmap0, s_)];
+        t_offF |= (uint64_t)((tid_all >> (6 + s_)) & 1) << d.local_pos[cbyte(d.wmapF, s_)];
     }
     uint64_t p0[RB], pF[RB];
 #pragma unroll
@@ -669,12 +681,12 @@ __device__ __forceinline__ void stage_tiles(T2 *__restrict__ s, const QVD_CONST 
     // index (fixed lane bits, flexible lane bits, wave bits) and the
     // register bits' tile bits (uniform).
     auto thread_index = [&](const QVD_CONST uint8_t *lm, const QVD_CONST uint8_t *wmp) {
-        uint32_t ti = lane & ((1u << FB) - 1);
+        uint32_t ti = lane_all & ((1u << FB) - 1);
 #pragma unroll
         for (int s_ = 0; s_ < (int)VMAX_L_FLEX; s_++)
-            if (s_ < (int)FL) ti |= ((lane >> (FB + s_)) & 1) << cbyte(lm, s_);
+            if (s_ < (int)FL) ti |= ((lane_all >> (FB + s_)) & 1) << cbyte(lm, s_);
 #pragma unroll
-        for (int s_ = 0; s_ < WB; s_++) ti |= ((tid >> (6 + s_)) & 1) << cbyte(wmp, s_);
+        for (int s_ = 0; s_ < WB; s_++) ti |= ((tid_all >> (6 + s_)) & 1) << cbyte(wmp, s_);
         return ti;
     };
     const uint32_t ti0 = thread_index(d.lmap0, d.wmap0);
@@ -686,9 +698,9 @@ __device__ __forceinline__ void stage_tiles(T2 *__restrict__ s, const QVD_CONST 
     const QVD_CONST VInstr *const ip_end = ip + d.num_instr;
 
     // With 4 waves per SIMD (16-wave workgroups) the other waves cover a
-    // tile's load latency; with 2 the next tile is prefetched into a second
-    // register set.
-    constexpr bool PREFETCH = WB <= 3;
+    // tile's load latency (with HALF those of the CU's other workgroup); with 2
+    // the next tile is prefetched into a second register set.
+    constexpr bool PREFETCH = WB <= 3 && !HALF;
     T2 x[R], y[PREFETCH ? R : 1];
     auto tile_base = [&](uint64_t t) {
         uint64_t base = 0;
@@ -762,6 +774,11 @@ __device__ __forceinline__ void stage_tiles(T2 *__restrict__ s, const QVD_CONST 
         // rotations fixed at compile time.
         auto handle = [&](auto hc, const QVD_CONST VInstr &v) {
             constexpr uint32_t H = decltype(hc)::value;
+            // With half the registers (HALF) the per-lane signs and predicates
+            // of every lane-bit handler, hoisted out of the loops, would be
+            // spilled: they are recomputed from an index the compiler can't see
+            // through.
+            const uint32_t tid = HALF ? opaque(tid_all) : tid_all, lane = HALF ? tid & 63 : lane_all;
             // Controls on non-tile qubits come only with the full and
             // controlled 1-qubit forms, general diagonals and LDS ops (the
             // host checks this); those arms skip tiles where they do not
@@ -837,6 +854,37 @@ __device__ __forceinline__ void stage_tiles(T2 *__restrict__ s, const QVD_CONST 
                 }
 #pragma unroll
                 for (int j = 0; j < R; j++) x[j] = cm(cm(ccoef[v.coef + W + j], ft), x[j]);
+            } else if constexpr (HALF && H == H_XCHG) {
+                uint32_t rn[RB];
+#pragma unroll
+                for (int b = 0; b < RB; b++) rn[b] = cbyte(v.rmap, b);
+                const uint32_t tn_ = thread_index(v.lmap, v.wmap);
+                R1 *const tp = part + ti;
+                const R1 *const tq = part + tn_;
+                auto at = [](const uint32_t(&r)[RB], int j) {
+                    uint32_t o = 0;
+#pragma unroll
+                    for (int b = 0; b < RB; b++)
+                        if ((j >> b) & 1) o |= 1u << r[b];
+                    return o;
+                };
+                lds_barrier();
+#pragma unroll
+                for (int j = 0; j < R; j++) tp[at(rm, j)] = x[j].x;
+                lds_barrier();
+#pragma unroll
+                for (int j = 0; j < R; j++) x[j].x = tq[at(rn, j)];
+                lds_barrier();
+#pragma unroll
+                for (int j = 0; j < R; j++) tp[at(rm, j)] = x[j].y;
+                lds_barrier();
+#pragma unroll
+                for (int j = 0; j < R; j++) x[j].y = tq[at(rn, j)];
+                ti = tn_;
+#pragma unroll
+                for (int b = 0; b < RB; b++) rm[b] = rn[b];
+            } else if constexpr (HALF && H == H_LDSOP) {
+                // not launched for such a stage
             } else if constexpr (H == H_XCHG || H == H_LDSOP) {
                 lds_barrier();
                 // The thread part ti and the register part o of a tile index
@@ -944,8 +992,8 @@ constexpr int C128_RB = QVD_C128_RB, C128_WB = 7 - C128_RB;
 
 }  // namespace
 
-template <typename T2, int WB, int RB, int FB, bool MAY_ZERO>
-__global__ __launch_bounds__(64 << WB) void k_vstage(T2 *__restrict__ s, const VStageDesc *__restrict__ descs,
+template <typename T2, int WB, int RB, int FB, bool MAY_ZERO, bool HALF = false>
+__global__ __launch_bounds__(64 << WB, HALF ? 4 : 1) void k_vstage(T2 *__restrict__ s, const VStageDesc *__restrict__ descs,
                                                      uint32_t ndesc, const uint32_t *__restrict__ block_start,
                                                      const VInstr *__restrict__ prog, const T2 *__restrict__ coefs,
                                                      const StageOp *__restrict__ ldsops,
@@ -966,7 +1014,7 @@ __global__ __launch_bounds__(64 << WB) void k_vstage(T2 *__restrict__ s, const V
         nb = cbs[di + 1] - cbs[di];
     }
     const QVD_CONST VStageDesc &d = ((const QVD_CONST VStageDesc *)descs)[di];
-    stage_tiles<T2, WB, RB, FB, MAY_ZERO>(s + d.state_off, d, bl, d.num_tiles, nb, prog, coefs, ldsops, ints);
+    stage_tiles<T2, WB, RB, FB, MAY_ZERO, HALF>(s + d.state_off, d, bl, d.num_tiles, nb, prog, coefs, ldsops, ints);
 }
 
 // Every stage of a batch of states in one launch. Items (runs of tiles of one
@@ -1062,18 +1110,32 @@ size_t vstage_lds_bytes() {
     return (sizeof(T2) << g.L()) + VCONST_BYTES;
 }
 
+// Two complex128 workgroups share a CU when the LDS tile holds one part of the
+// amplitudes (64 KiB) and each thread 16 amplitudes without a prefetch set (128
+// VGPRs): 4 waves per SIMD instead of 2, in two groups that wait for their
+// exchanges, loads and instructions independently. One group left the VALU
+// idle 58 % of a deep stage. With fewer tiles than two per CU there is nothing
+// to overlap and the second pair of barriers costs. Kicked Ising, 10 steps, all
+// stages: 26 qubits 4.88 -> 4.06 ms, 24 0.95 -> 0.84, 22 (2 tiles per CU)
+// 0.55 -> 0.45, 21 (1 tile) 0.388 -> 0.402; random, 26: 3.06 -> 2.54.
+bool vstage_half(uint64_t num_tiles, uint32_t ccount, unsigned cus) {
+    constexpr size_t LDS = 160 * 1024;
+    const size_t need = (sizeof(double) << vstage_geom<double2>().L()) + ccount * sizeof(double2);
+    return 2 * need <= LDS && num_tiles >= 2 * (uint64_t)cus;
+}
+
 template <typename T2>
 hipError_t launch_vstage(T2 *s, const VStageDesc *descs, uint32_t ndesc, const uint32_t *block_start,
                          const VInstr *prog, const T2 *coefs, const StageOp *ldsops, const uint32_t *ints, unsigned grid,
-                         hipStream_t st, bool lazy_zero, uint32_t fixed_lanes) {
-    const size_t lds = vstage_lds_bytes<T2>();
+                         hipStream_t st, bool lazy_zero, uint32_t fixed_lanes, bool half, uint32_t ccount) {
+    size_t lds = vstage_lds_bytes<T2>();
     using Kernel = void (*)(T2 *, const VStageDesc *, uint32_t, const uint32_t *, const VInstr *, const T2 *,
                             const StageOp *, const uint32_t *);
     // A stage that starts from |0...0> or names stale qubits has a kernel of
     // its own, so the others keep the code without those branches. The default geometry's
     // fixed lane bits are compiled in; any other count is read from the
     // descriptors.
-    Kernel k, kz, kf, kfz;
+    Kernel k, kz, kf, kfz, kh = nullptr, khz = nullptr;
     if constexpr (sizeof(T2) == 8) {
         k = k_vstage<T2, C64_WB, C64_RB, 4, false>;
         kz = k_vstage<T2, C64_WB, C64_RB, 4, true>;
@@ -1084,6 +1146,8 @@ hipError_t launch_vstage(T2 *s, const VStageDesc *descs, uint32_t ndesc, const u
         kz = k_vstage<T2, C128_WB, C128_RB, 3, true>;
         kf = k_vstage<T2, C128_WB, C128_RB, -1, false>;
         kfz = k_vstage<T2, C128_WB, C128_RB, -1, true>;
+        kh = k_vstage<T2, C128_WB, C128_RB, 3, false, true>;
+        khz = k_vstage<T2, C128_WB, C128_RB, 3, true, true>;
     }
     // The LDS size attribute is set once per device, before any launch a
     // caller may capture into a graph.
@@ -1101,11 +1165,21 @@ hipError_t launch_vstage(T2 *s, const VStageDesc *descs, uint32_t ndesc, const u
         if (e != hipSuccess) return e;
         e = hipFuncSetAttribute((const void *)kfz, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
         if (e != hipSuccess) return e;
+        for (Kernel h : {kh, khz}) {
+            if (!h) continue;
+            e = hipFuncSetAttribute((const void *)h, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+            if (e != hipSuccess) return e;
+        }
         attr_set.fetch_or(bit);
     }
     if (fixed_lanes != 0 && fixed_lanes != vstage_geom<T2>().f_bits) {
         k = kf;
         kz = kfz;
+    }
+    if (half && kh) {
+        k = kh;
+        kz = khz;
+        lds = (sizeof(T2) / 2 << vstage_geom<T2>().L()) + ccount * sizeof(T2);
     }
     if (lazy_zero) k = kz;
     k<<<grid, 64 << vstage_geom<T2>().w_bits, lds, st>>>(s, descs, ndesc, block_start, prog, coefs, ldsops, ints);
@@ -1171,10 +1245,10 @@ template size_t vstage_lds_bytes<float2>();
 template size_t vstage_lds_bytes<double2>();
 template hipError_t launch_vstage<float2>(float2 *, const VStageDesc *, uint32_t, const uint32_t *, const VInstr *,
                                           const float2 *, const StageOp *, const uint32_t *, unsigned, hipStream_t,
-                                          bool, uint32_t);
+                                          bool, uint32_t, bool, uint32_t);
 template hipError_t launch_vstage<double2>(double2 *, const VStageDesc *, uint32_t, const uint32_t *, const VInstr *,
                                            const double2 *, const StageOp *, const uint32_t *, unsigned, hipStream_t,
-                                           bool, uint32_t);
+                                           bool, uint32_t, bool, uint32_t);
 template hipError_t launch_vstage_queue<float2>(float2 *, const VStageDesc *, const VQueueItem *, uint32_t, uint32_t *,
                                                 const VInstr *, const float2 *, const StageOp *, const uint32_t *,
                                                 unsigned, hipStream_t);
