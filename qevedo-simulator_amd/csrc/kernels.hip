@@ -1112,6 +1112,129 @@ __global__ __launch_bounds__(64) void k_walk_marks(const T2 *__restrict__ s, uin
     walked[c] = b;
 }
 
+// The chunk sums and the walk for states of few chunks, where one lane per
+// chunk leaves most of the chip idle and spends 33 cycles an amplitude on
+// conversions and products beside the add that the order of summation asks
+// for. Here one wave only adds: its lane c runs chunk c's sum over
+// probabilities in LDS, one add after the other, while four waves load the
+// coming batches (coalesced) and square them. C chunks per workgroup, batches
+// of CHAIN_BATCH amplitudes over all of them, two in LDS and one in registers.
+// Bound by the latency of the dependent adds: 24 qubits in complex64 (chunks
+// of 2^15) 172 us for the sums where one lane per chunk took 454, 201 us for
+// the walk where it took 545. The sums and marks are the same bit for bit.
+constexpr int CHAIN_THREADS = 64 + 256, CHAIN_BATCH = 2048;
+
+// Workgroup barrier that waits for LDS only: the loads of a coming batch stay
+// in flight across it.
+__device__ __forceinline__ void lds_barrier() {
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_waitcnt(0xC07F);  // gfx9 encoding: lgkmcnt(0), vmcnt and expcnt not waited
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+}
+
+template <typename T2, int C, bool WALK>
+__global__ __launch_bounds__(CHAIN_THREADS) void k_chain(const T2 *__restrict__ s, uint64_t clen, uint32_t mark_bits,
+                                                         const double *__restrict__ prefix,
+                                                         const uint64_t *__restrict__ bounds,
+                                                         const double *__restrict__ targets, uint64_t shots,
+                                                         double *__restrict__ marks, uint32_t *__restrict__ walked,
+                                                         double *__restrict__ sums) {
+    constexpr int BATCH = CHAIN_BATCH / C, PITCH = BATCH + 2, PER = CHAIN_BATCH / 256;
+    __shared__ __attribute__((aligned(16))) double p[2][C * PITCH];
+    __shared__ uint32_t stop[2];
+    const uint64_t c0 = (uint64_t)blockIdx.x * C;
+    const uint32_t tid = threadIdx.x, lane = tid & 63;
+    const bool serial = __builtin_amdgcn_readfirstlane(tid >> 6) == 0;  // wave 0
+    const uint64_t batches = clen / BATCH;
+    double acc = 0, t_last = 0;
+    bool done = lane >= C;
+    uint32_t nb = 0;
+    const uint64_t c = c0 + (lane < C ? lane : 0);
+    if constexpr (WALK) {
+        const uint64_t first = bounds[c0], past = bounds[c0 + C] < shots ? bounds[c0 + C] : shots;
+        if (first >= past) return;  // no shot in these chunks (uniform over the workgroup): nothing is read
+        if (serial && lane < C) {
+            const uint64_t lo = bounds[c], hi = bounds[c + 1] < shots ? bounds[c + 1] : shots;
+            done = lo >= hi;
+            if (!done) t_last = targets[hi - 1];
+            acc = prefix[c];
+        }
+    }
+    double *const m = WALK ? marks + ((c * clen) >> mark_bits) : nullptr;
+    const uint64_t mask = (uint64_t(1) << mark_bits) - 1;
+    T2 r[PER];
+    auto fetch = [&](uint64_t b) {
+#pragma unroll
+        for (int i = 0; i < PER; i++) {
+            const uint32_t e = i * 256 + (tid - 64);
+            r[i] = s[(c0 + e / BATCH) * clen + b * BATCH + e % BATCH];
+        }
+    };
+    auto put = [&](uint64_t b) {
+#pragma unroll
+        for (int i = 0; i < PER; i++) {
+            const uint32_t e = i * 256 + (tid - 64);
+            p[b & 1][(e / BATCH) * PITCH + e % BATCH] = prob(r[i]);
+        }
+    };
+    if (!serial) {
+        fetch(0);
+        put(0);
+        if (batches > 1) fetch(1);
+    }
+    if (serial) __builtin_amdgcn_s_setprio(3);  // its adds are the critical path
+    lds_barrier();
+    for (uint64_t b = 0; b < batches; b++) {
+        if (!serial) {
+            if (b + 1 < batches) put(b + 1);
+            if (b + 2 < batches) fetch(b + 2);
+        } else if (lane < C) {
+            const double2 *const q = reinterpret_cast<const double2 *>(&p[b & 1][lane * PITCH]);
+            // 2 U values are added while the next 2 U come from LDS.
+            constexpr int U = BATCH >= 128 ? 16 : 8;
+            static_assert(BATCH % (4 * U) == 0 && 2 * U <= 64, "a batch is whole steps, and a mark falls on a step's end");
+            double2 a[U], n[U];
+#pragma unroll
+            for (int j = 0; j < U; j++) a[j] = q[j];
+            auto add = [&](const double2(&v)[U], uint32_t at) {  // `at`: the values of the batch added afterwards
+#pragma unroll
+                for (int j = 0; j < U; j++) {
+                    acc += v[j].x;
+                    acc += v[j].y;
+                }
+                if constexpr (WALK) {
+                    const uint64_t pos = b * BATCH + at;
+                    if (!done && ((pos & mask) == 0 || pos == clen)) {
+                        m[nb++] = acc;
+                        done = t_last < acc;  // every shot of the chunk lands in a walked block
+                        if (done || pos == clen) walked[c] = nb;
+                    }
+                }
+            };
+            for (uint32_t k = 0; k < BATCH / 2; k += 2 * U) {
+#pragma unroll
+                for (int j = 0; j < U; j++) n[j] = q[k + U + j];
+                __builtin_amdgcn_sched_barrier(0);
+                add(a, 2 * (k + U));
+                const uint32_t next = k + 2 * U < BATCH / 2 ? k + 2 * U : 0;
+#pragma unroll
+                for (int j = 0; j < U; j++) a[j] = q[next + j];
+                __builtin_amdgcn_sched_barrier(0);
+                add(n, 2 * (k + 2 * U));
+            }
+            if constexpr (WALK) {
+                const bool all = __ballot(!done) == 0;
+                if (lane == 0) stop[b & 1] = all;
+            }
+        }
+        lds_barrier();
+        // Written again only after the next barrier, which needs this read.
+        if (WALK && stop[b & 1]) break;
+    }
+    if (!WALK && serial && lane < C) sums[c] = acc;
+}
+
 template <typename T2>
 __global__ __launch_bounds__(256) void k_walk_place(const T2 *__restrict__ s, uint64_t len, uint64_t chunk,
                                                      uint64_t num_chunks, uint32_t mark_bits,
@@ -1422,11 +1545,39 @@ size_t sort_temp_bytes(uint64_t shots) {
     return bytes;
 }
 
+// Chunks per workgroup of k_chain: one workgroup per CU, up to 16 chunks each;
+// 0 where one lane per chunk is better: chunks shorter than a batch, and more
+// than 4096 of them, which fill the chip.
+static int chain_chunks(uint64_t clen, uint64_t nc) {
+    if (clen < CHAIN_BATCH || nc > 4096) return 0;
+    return nc >= 4096 ? 16 : nc >= 2048 ? 8 : nc >= 1024 ? 4 : nc >= 512 ? 2 : 1;
+}
+
+template <typename T2, bool WALK>
+static void chain_launch(const T2 *s, uint64_t clen, uint64_t nc, int per, const SampleScratch &w, uint64_t shots,
+                         hipStream_t st) {
+    const unsigned grid = (unsigned)(nc / per);  // both are powers of two
+    auto go = [&](auto k) {
+        k<<<grid, CHAIN_THREADS, 0, st>>>(s, clen, w.mark_bits, w.prefix, w.bounds, w.targets, shots, w.marks, w.walked,
+                                          w.sums);
+    };
+    if (per == 16) go(k_chain<T2, 16, WALK>);
+    else if (per == 8) go(k_chain<T2, 8, WALK>);
+    else if (per == 4) go(k_chain<T2, 4, WALK>);
+    else if (per == 2) go(k_chain<T2, 2, WALK>);
+    else go(k_chain<T2, 1, WALK>);
+}
+
 template <typename T2>
 void launch_sample_sums(const T2 *s, uint64_t len, uint64_t chunk, SampleScratch &w, hipStream_t st) {
     const uint64_t nc = (len + chunk - 1) / chunk;
-    // 64-lane workgroups for the per-chunk kernels, so 2^15 chunks spread over every CU.
-    k_chunk_sums<T2><<<grid_for(nc, 64, 1u << 30), 64, 0, st>>>(s, len, chunk, nc, w.sums);
+    const uint64_t clen = std::min(chunk, len);
+    if (const int per = chain_chunks(clen, nc)) {
+        chain_launch<T2, false>(s, clen, nc, per, w, 0, st);
+    } else {
+        // 64-lane workgroups for the per-chunk kernels, so 2^15 chunks spread over every CU.
+        k_chunk_sums<T2><<<grid_for(nc, 64, 1u << 30), 64, 0, st>>>(s, len, chunk, nc, w.sums);
+    }
     k_prefix<<<1, PREFIX_THREADS, 0, st>>>(w.sums, nc, w.prefix);
 }
 
@@ -1442,8 +1593,12 @@ hipError_t launch_sample_walk(const T2 *s, uint64_t len, uint64_t chunk, uint64_
     const uint64_t nc = (len + chunk - 1) / chunk;
     k_targets<<<grid_for(shots, 256), 256, 0, st>>>(w.targets, w.prefix + nc, shots);
     k_bounds<<<grid_for(nc + 1, 256, 1u << 30), 256, 0, st>>>(w.prefix, nc, w.targets, shots, w.bounds);
-    k_walk_marks<T2><<<grid_for(nc, 64, 1u << 30), 64, 0, st>>>(s, len, chunk, nc, w.mark_bits, w.prefix, w.bounds,
-                                                                w.targets, shots, w.marks, w.walked);
+    const uint64_t clen = std::min(chunk, len);
+    if (const int per = chain_chunks(clen, nc))
+        chain_launch<T2, true>(s, clen, nc, per, w, shots, st);
+    else
+        k_walk_marks<T2><<<grid_for(nc, 64, 1u << 30), 64, 0, st>>>(s, len, chunk, nc, w.mark_bits, w.prefix, w.bounds,
+                                                                    w.targets, shots, w.marks, w.walked);
     k_walk_place<T2><<<grid_for(shots, 256), 256, 0, st>>>(s, len, chunk, nc, w.mark_bits, w.prefix, w.bounds,
                                                            w.targets, shots, w.marks, w.walked, out);
     return hipGetLastError();
