@@ -79,6 +79,71 @@ double now() {
     return std::chrono::duration<double>(std::chrono::steady_clock::now().time_since_epoch()).count();
 }
 
+// A stream and a page of pinned host memory that kernels write small results
+// to (no copy behind them: a copy to pageable memory adds 11 us to a call of
+// 11). Making and destroying a stream takes 60 us and the page 25, as long as
+// everything else a small state does, so up to LANES_KEPT lanes that destroyed
+// handles gave back wait for the next handle on their device; more are freed.
+constexpr size_t MAIL_DOUBLES = 512;
+constexpr size_t LANES_KEPT = 8;
+struct Lane {
+    int device = 0;
+    hipStream_t stream = nullptr;
+    double *mail = nullptr;      // host address
+    double *mail_dev = nullptr;  // the same memory as kernels see it
+};
+struct LanePool {
+    std::mutex mu;
+    std::vector<Lane> idle;
+};
+LanePool &lane_pool() {
+    static LanePool *pool = new LanePool();  // never destroyed: handles may outlive static objects
+    return *pool;
+}
+void free_lane(Lane &l) {
+    if (l.mail) (void)hipHostFree(l.mail);
+    if (l.stream) (void)hipStreamDestroy(l.stream);
+    l = Lane();
+}
+// A lane on the current device.
+Lane take_lane(int device) {
+    {
+        LanePool &pool = lane_pool();
+        std::lock_guard<std::mutex> lock(pool.mu);
+        for (size_t i = pool.idle.size(); i-- > 0;) {
+            if (pool.idle[i].device != device) continue;
+            const Lane l = pool.idle[i];
+            pool.idle.erase(pool.idle.begin() + (ptrdiff_t)i);
+            if (hipStreamQuery(l.stream) == hipSuccess) return l;
+            (void)hipGetLastError();  // gone with a device reset, its page too
+        }
+    }
+    Lane l;
+    l.device = device;
+    try {
+        QVD_HIP(hipStreamCreateWithFlags(&l.stream, hipStreamNonBlocking));
+        QVD_HIP(hipHostMalloc((void **)&l.mail, MAIL_DOUBLES * sizeof(double), hipHostMallocDefault));
+        QVD_HIP(hipHostGetDevicePointer((void **)&l.mail_dev, l.mail, 0));
+    } catch (...) {
+        free_lane(l);
+        throw;
+    }
+    return l;
+}
+// Nothing may be left running on the lane. One whose stream reported an error is not kept.
+void give_lane(Lane &l, bool keep) {
+    if (keep) {
+        LanePool &pool = lane_pool();
+        std::lock_guard<std::mutex> lock(pool.mu);
+        if (pool.idle.size() < LANES_KEPT) {
+            pool.idle.push_back(l);
+            l = Lane();
+            return;
+        }
+    }
+    free_lane(l);
+}
+
 }  // namespace
 }  // namespace qvd
 
@@ -88,7 +153,8 @@ struct qvd_sv {
     int device = 0;
     uint64_t len = 0;
     DBuf amps;
-    hipStream_t stream = nullptr;
+    Lane lane;                       // its stream and its page for small results
+    hipStream_t stream = nullptr;    // lane.stream
     hipStream_t side = nullptr;      // sampling: the uniforms' copy and sort (made by the first qvd_sv_sample)
     hipEvent_t side_done = nullptr;  // recorded after them
     void *sample_host = nullptr;     // pinned host staging of the outcomes, grown to the largest call and kept
@@ -318,10 +384,39 @@ std::vector<T2> full_coefficients(const Op &op) {
     return c;
 }
 
-// One op as its own HBM pass, its coefficients (full_coefficients) already
-// in device memory at `coef`; enqueued on the handle's stream, not waited for.
+// Targets of a dense op inside a 128-byte line.
 template <typename T2>
-void apply_full(qvd_sv *sv, T2 *s, const Op &op, const T2 *coef, bool valu_only = false) {
+uint32_t targets_in_line(const Op &op) {
+    uint32_t n = 0;
+    for (uint32_t t : op.targets) n += (sizeof(T2) << t) < 128;
+    return n;
+}
+
+// Matrix cores for 5- and 6-qubit gates, and in complex128 for 3- and
+// 4-qubit ones with two or more targets inside a 128-byte line, whose
+// groups k_dense would load as pieces of a line (28 qubits, targets 0-3:
+// 2.63 ms against 1.76). With at most one target there k_dense moves whole
+// lines and is ahead (targets 4-7: 1.60 against 1.77): it needs no
+// staging through LDS. In complex64 3- and 4-qubit gates keep k_dense
+// and its order of the FP32 sums.
+template <typename T2>
+bool on_matrix_cores(const Op &op) {
+    const size_t k = op.targets.size();
+    return k >= 5 || (sizeof(T2) == 16 && k >= 3 && targets_in_line<T2>(op) >= 2);
+}
+
+// Whether a single op's coefficients go with its launch, as kernel arguments
+// (at most 1 KiB), instead of through a copy in front of it (3 us a call).
+template <typename T2>
+bool by_argument(const Op &op) {
+    return !op.targets.empty() && op.targets.size() <= DENSE_ARG_QUBITS && !op.diagonal && !on_matrix_cores<T2>(op);
+}
+
+// One op as its own HBM pass, its coefficients (full_coefficients) already
+// in device memory at `coef`, or at `coef` on the host (by_arg, where
+// by_argument holds); enqueued on the handle's stream, not waited for.
+template <typename T2>
+void apply_full(qvd_sv *sv, T2 *s, const Op &op, const T2 *coef, bool valu_only = false, bool by_arg = false) {
     const uint32_t k = (uint32_t)op.targets.size();
     if (k == 0) return;
     if (k > MAX_GATE_QUBITS)
@@ -352,20 +447,12 @@ void apply_full(qvd_sv *sv, T2 *s, const Op &op, const T2 *coef, bool valu_only 
     }
     d.ctrl_val = cval;
     d.iterations = uint64_t(1) << (sv->n - d.nins);
-    // Matrix cores for 5- and 6-qubit gates, and in complex128 for 3- and
-    // 4-qubit ones with two or more targets inside a 128-byte line, whose
-    // groups k_dense would load as pieces of a line (28 qubits, targets 0-3:
-    // 2.63 ms against 1.76). With at most one target there k_dense moves whole
-    // lines and is ahead (targets 4-7: 1.60 against 1.77): it needs no
-    // staging through LDS. In complex64 3- and 4-qubit gates keep k_dense
-    // and its order of the FP32 sums.
-    uint32_t in_line = 0;
-    for (uint32_t t : op.targets) in_line += (sizeof(T2) << t) < 128;
-    if ((k >= 5 || (sizeof(T2) == 16 && k >= 3 && in_line >= 2)) && !valu_only) {
+    if (on_matrix_cores<T2>(op) && !valu_only) {
         QVD_HIP(launch_dense_mfma<T2>(s, d, coef, (unsigned)num_cus(sv->device), sv->stream));
         return;
     }
-    launch_dense<T2>(s, d, coef, sv->stream);
+    if (by_arg) launch_dense_arg<T2>(s, d, coef, sv->stream);
+    else launch_dense<T2>(s, d, coef, sv->stream);
     QVD_HIP(hipGetLastError());
 }
 
@@ -1597,8 +1684,9 @@ int qvd_sv_create(uint32_t num_qubits, int precision, qvd_sv **out) {
         if (hipGetDeviceCount(&count) != hipSuccess || count == 0) fail(QVD_EHIP, "no HIP device is visible");
         QVD_HIP(hipGetDevice(&sv->device));
         sv->bind();
-        QVD_HIP(hipStreamCreateWithFlags(&sv->stream, hipStreamNonBlocking));
         sv->amps.alloc(bytes);
+        sv->lane = take_lane(sv->device);
+        sv->stream = sv->lane.stream;
         sv->zero_pending = true;
         sv->zero_qubits = qubit_mask(num_qubits);
         *out = sv.release();
@@ -1609,14 +1697,14 @@ int qvd_sv_destroy(qvd_sv *sv) {
     return guard([&] {
         if (!sv) return;
         sv->bind();
-        if (sv->stream) (void)hipStreamSynchronize(sv->stream);
+        const bool clean = !sv->stream || hipStreamSynchronize(sv->stream) == hipSuccess;
         sv->amps.alloc(0);
         sv->scratch.alloc(0);
         if (sv->side) (void)hipStreamSynchronize(sv->side);
         if (sv->sample_host) (void)hipHostFree(sv->sample_host);
         if (sv->side_done) (void)hipEventDestroy(sv->side_done);
         if (sv->side) (void)hipStreamDestroy(sv->side);
-        if (sv->stream) (void)hipStreamDestroy(sv->stream);
+        if (sv->stream) give_lane(sv->lane, clean);
         delete sv;
     });
 }
@@ -1716,9 +1804,14 @@ int qvd_sv_apply(qvd_sv *sv, const double *matrix, const uint32_t *targets, uint
         sv->bind();
         with_type(sv, [&](auto *s) {
             using T2 = std::remove_pointer_t<decltype(s)>;
-            Upload up;
-            const size_t o = up.put(full_coefficients<T2>(op));
-            apply_full(sv, s, op, reinterpret_cast<const T2 *>(up.to_device(sv) + o));
+            const std::vector<T2> coefs = full_coefficients<T2>(op);
+            if (by_argument<T2>(op)) {
+                apply_full(sv, s, op, coefs.data(), false, true);
+            } else {
+                Upload up;
+                const size_t o = up.put(coefs);
+                apply_full(sv, s, op, reinterpret_cast<const T2 *>(up.to_device(sv) + o));
+            }
             sv->sync();
             return 0;
         });
@@ -1861,14 +1954,14 @@ int qvd_sv_norm_sqr(const qvd_sv *sv_c, double *out) {
         require(out != nullptr, "null output");
         qvd_sv *sv = const_cast<qvd_sv *>(sv_c);
         sv->bind();
-        double *buf = sv->scratch_doubles(NORM_BLOCKS + 1);
+        double *buf = sv->scratch_doubles(NORM_BLOCKS);
         with_type(sv, [&](auto *s) {
-            launch_norm(s, sv->len, -1, buf, buf + NORM_BLOCKS, sv->stream);
+            launch_norm(s, sv->len, -1, buf, sv->lane.mail_dev, sv->stream);
             return 0;
         });
         QVD_HIP(hipGetLastError());
-        QVD_HIP(hipMemcpyAsync(out, buf + NORM_BLOCKS, sizeof(double), hipMemcpyDeviceToHost, sv->stream));
         sv->sync();
+        *out = sv->lane.mail[0];
     });
 }
 
@@ -1885,24 +1978,25 @@ int qvd_sv_scale(qvd_sv *sv, double factor) {
     });
 }
 
-// Queues P(qubit = 1) into device memory (returned).
-static const double *enqueue_probability_one(qvd_sv *sv, uint32_t qubit) {
-    require(qubit < sv->n, "qubit " + std::to_string(qubit) + " out of range for " + std::to_string(sv->n) + " qubits");
+// Queues P(qubit = 1) into `out` (device memory or the lane's page).
+static void enqueue_probability_one(qvd_sv *sv, uint32_t qubit, double *out) {
     double *buf = sv->scratch_doubles(NORM_BLOCKS + 1);
     with_type(sv, [&](auto *s) {
-        launch_norm(s, sv->len, (int)qubit, buf, buf + NORM_BLOCKS, sv->stream);
+        launch_norm(s, sv->len, (int)qubit, buf, out, sv->stream);
         return 0;
     });
     QVD_HIP(hipGetLastError());
-    return buf + NORM_BLOCKS;
+}
+
+static void check_qubit(const qvd_sv *sv, uint32_t qubit) {
+    require(qubit < sv->n, "qubit " + std::to_string(qubit) + " out of range for " + std::to_string(sv->n) + " qubits");
 }
 
 static double probability_one_impl(qvd_sv *sv, uint32_t qubit) {
-    double r = 0;
-    const double *p = enqueue_probability_one(sv, qubit);
-    QVD_HIP(hipMemcpyAsync(&r, p, sizeof(double), hipMemcpyDeviceToHost, sv->stream));
+    check_qubit(sv, qubit);
+    enqueue_probability_one(sv, qubit, sv->lane.mail_dev);
     sv->sync();
-    return r;
+    return sv->lane.mail[0];
 }
 
 int qvd_sv_probability_one(const qvd_sv *sv_c, uint32_t qubit, double *out) {
@@ -1991,19 +2085,22 @@ int qvd_sv_expect_pauli(const qvd_sv *sv_c, const uint64_t *x_masks, const uint6
             std::vector<uint64_t> up(gw + k);
             std::memcpy(up.data(), groups.data(), groups.size() * sizeof(PauliGroup));
             std::memcpy(up.data() + gw, zs.data(), k * sizeof(uint64_t));
-            // sums, descriptors and Z parts, then the blocks' partial sums
+            // sums, descriptors and Z parts, then the blocks' partial sums;
+            // a page's worth of sums goes straight to the host
             double *buf = sv->scratch_doubles(k + up.size() + k * blocks);
+            const bool mail = k <= MAIL_DOUBLES;
             uint64_t *dg = reinterpret_cast<uint64_t *>(buf + k);
             QVD_HIP(hipMemcpyAsync(dg, up.data(), up.size() * sizeof(uint64_t), hipMemcpyHostToDevice, sv->stream));
             with_type(sv, [&](auto *s) {
                 launch_expect_pauli(s, sv->len, reinterpret_cast<const PauliGroup *>(dg), widths, dg + gw, (uint32_t)k,
-                                    buf + k + up.size(), blocks, buf, sv->stream);
+                                    buf + k + up.size(), blocks, mail ? sv->lane.mail_dev : buf, sv->stream);
                 return 0;
             });
             QVD_HIP(hipGetLastError());
             h.resize(k);
-            QVD_HIP(hipMemcpyAsync(h.data(), buf, k * sizeof(double), hipMemcpyDeviceToHost, sv->stream));
+            if (!mail) QVD_HIP(hipMemcpyAsync(h.data(), buf, k * sizeof(double), hipMemcpyDeviceToHost, sv->stream));
             sv->sync();
+            if (mail) std::copy(sv->lane.mail, sv->lane.mail + k, h.begin());
             for (size_t t = 0; t < k; t++) {
                 // P = i^popcount(x & z) X^x Z^z; the sum is over half of the
                 // indices where x != 0.
@@ -2026,35 +2123,32 @@ int qvd_sv_expect_z(const qvd_sv *sv_c, double *z, double *zz) {
         sv->bind();
         const uint32_t B = expect_segment_bits(n);
         const uint64_t segs = uint64_t(1) << (n - B);
-        // segment sums, then the results, in the handle's reduction scratch
-        double *seg = sv->scratch_doubles(segs * 2 * B + 2 * n);
-        double *res = seg + segs * 2 * B;
+        static_assert(2 * MAX_QUBITS <= MAIL_DOUBLES, "a state's values fit the lane's page");
+        double *seg = sv->scratch_doubles(segs * 2 * B);
         with_type(sv, [&](auto *s) {
-            launch_expect_z(s, n, seg, res, res + n, sv->stream);
+            launch_expect_z(s, n, seg, sv->lane.mail_dev, sv->lane.mail_dev + n, sv->stream);
             return 0;
         });
         QVD_HIP(hipGetLastError());
-        std::vector<double> h(2 * n);
-        QVD_HIP(hipMemcpyAsync(h.data(), res, (2 * n - 1) * sizeof(double), hipMemcpyDeviceToHost, sv->stream));
         sv->sync();
-        std::copy(h.begin(), h.begin() + n, z);
-        if (zz) std::copy(h.begin() + n, h.begin() + 2 * n - 1, zz);
+        std::copy(sv->lane.mail, sv->lane.mail + n, z);
+        if (zz) std::copy(sv->lane.mail + n, sv->lane.mail + 2 * n - 1, zz);
     });
 }
 
 // Measures a qubit (flip: and resets it). The collapse reads P(1) from device
-// memory and comes to the outcome found here.
+// memory, comes to the outcome found here and hands P(1) on.
 static uint8_t measure_impl(qvd_sv *sv, uint32_t qubit, double uniform, bool flip) {
-    double p1 = 0;
-    const double *p = enqueue_probability_one(sv, qubit);
+    check_qubit(sv, qubit);
+    double *p = sv->scratch_doubles(NORM_BLOCKS + 1) + NORM_BLOCKS;
+    enqueue_probability_one(sv, qubit, p);
     with_type(sv, [&](auto *s) {
-        launch_collapse(s, sv->len, qubit, uniform, p, flip, sv->stream);
+        launch_collapse(s, sv->len, qubit, uniform, p, flip, sv->lane.mail_dev, sv->stream);
         return 0;
     });
     QVD_HIP(hipGetLastError());
-    QVD_HIP(hipMemcpyAsync(&p1, p, sizeof(double), hipMemcpyDeviceToHost, sv->stream));
     sv->sync();
-    p1 = std::min(std::max(p1, 0.0), 1.0);
+    const double p1 = std::min(std::max(sv->lane.mail[0], 0.0), 1.0);
     return uniform < p1 ? 1 : 0;
 }
 

@@ -65,6 +65,10 @@ template <typename T2> void launch_widen(const T2 *s, double2 *out, uint64_t cou
 template <typename T2> void launch_narrow(const double2 *in, T2 *s, uint64_t count, hipStream_t st);
 template <typename T2> void launch_scale(T2 *s, uint64_t len, double factor, hipStream_t st);
 template <typename T2> void launch_dense(T2 *s, const GateDesc &d, const T2 *mat, hipStream_t st);
+// The same for up to DENSE_ARG_QUBITS targets with the matrix in host memory,
+// passed as kernel arguments.
+constexpr uint32_t DENSE_ARG_QUBITS = 3;
+template <typename T2> void launch_dense_arg(T2 *s, const GateDesc &d, const T2 *mat, hipStream_t st);
 template <typename T2>
 void launch_diag(T2 *s, uint64_t len, uint32_t k, const DiagTargets &t, uint64_t cmask, uint64_t cval,
                  const T2 *entries, hipStream_t st);
@@ -103,10 +107,11 @@ void launch_zero_words(uint32_t *p, uint32_t n, hipStream_t st);
 // Zero-fills `len` amplitudes and sets amplitude offs[i] to 1 for each state i.
 template <typename T2>
 void launch_batch_init(T2 *s, uint64_t len, const uint64_t *offs, uint32_t count, hipStream_t st);
-// Measures `qubit` given P(1) at p_one (device memory); flip: and resets it.
+// Measures `qubit` given P(1) at p_one (device memory), which is also copied to
+// p_copy; flip: and resets it.
 template <typename T2>
 void launch_collapse(T2 *s, uint64_t len, uint32_t qubit, double uniform, const double *p_one, bool flip,
-                     hipStream_t st);
+                     double *p_copy, hipStream_t st);
 size_t sort_temp_bytes(uint64_t shots);
 // Two-pass sampling (src/measure.rs:104-174) in three parts: the chunk sums
 // and their prefix; the uniforms' sort into w.targets (on any stream); then,

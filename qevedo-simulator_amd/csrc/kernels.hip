@@ -139,10 +139,25 @@ __global__ void k_scale(T2 *__restrict__ s, uint64_t len, double factor) {
 // to K = 4 (28 qubits, targets 4-7: 0.82 ms in complex64 and 1.60 ms in
 // complex128, a copy of the state taking 0.79 and 1.58; read from LDS, each
 // element per FMA pair, the matrix bound it at 1.72 and 7.9 ms).
+//
+// The matrix is in device memory, or is itself an argument of the launch
+// (MatArg; a gate applied by itself needs no copy in front of its pass then).
 template <typename T2, int K>
-__global__ __launch_bounds__(256) void k_dense(T2 *__restrict__ s, const GateDesc d, const T2 *__restrict__ mat) {
+struct MatArg {
+    T2 m[1 << (2 * K)];
+};
+template <typename T2>
+__device__ __forceinline__ T2 mat_at(const T2 *mat, int i) {
+    return (T2)((const QVD_CONST T2 *)mat)[i];
+}
+template <typename T2, int K>
+__device__ __forceinline__ T2 mat_at(const MatArg<T2, K> &mat, int i) {
+    return mat.m[i];
+}
+
+template <typename T2, int K, typename M>
+__global__ __launch_bounds__(256) void k_dense(T2 *__restrict__ s, const GateDesc d, const M mat) {
     constexpr int D = 1 << K;
-    const QVD_CONST T2 *const m = (const QVD_CONST T2 *)mat;
     const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
     for (uint64_t it = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; it < d.iterations; it += stride) {
         T2 *const g = s + (insert_zeros(it, d.ins, d.nins) | d.ctrl_val);
@@ -158,7 +173,7 @@ __global__ __launch_bounds__(256) void k_dense(T2 *__restrict__ s, const GateDes
             acc.x = 0;
             acc.y = 0;
 #pragma unroll
-            for (int c = 0; c < D; c++) cmac(acc, (T2)m[r * D + c], a[c]);
+            for (int c = 0; c < D; c++) cmac(acc, mat_at(mat, r * D + c), a[c]);
             g[d.offsets[r]] = acc;
         }
     }
@@ -802,9 +817,10 @@ __global__ void k_zero_words(uint32_t *__restrict__ p, uint32_t n) {
 // ---------------------------------------------------------------------------
 template <typename T2, bool FLIP>
 __global__ __launch_bounds__(256) void k_collapse(T2 *__restrict__ s, uint64_t len, uint32_t qubit, double uniform,
-                                                  const double *__restrict__ p_one) {
+                                                  const double *__restrict__ p_one, double *__restrict__ p_copy) {
     using T = typename Real<T2>::T;
     double p1 = *p_one;
+    if (blockIdx.x == 0 && threadIdx.x == 0) *p_copy = p1;
     p1 = p1 < 0.0 ? 0.0 : p1;  // a NaN stays one, as in the host's clamp
     p1 = 1.0 < p1 ? 1.0 : p1;
     const bool outcome = uniform < p1;
@@ -1344,14 +1360,28 @@ template <typename T2>
 void launch_dense(T2 *s, const GateDesc &d, const T2 *mat, hipStream_t st) {
     const unsigned grid = grid_for(d.iterations, 256, 65536);
     switch (d.k) {
-        case 1: k_dense<T2, 1><<<grid, 256, 0, st>>>(s, d, mat); break;
-        case 2: k_dense<T2, 2><<<grid, 256, 0, st>>>(s, d, mat); break;
-        case 3: k_dense<T2, 3><<<grid, 256, 0, st>>>(s, d, mat); break;
-        case 4: k_dense<T2, 4><<<grid, 256, 0, st>>>(s, d, mat); break;
-        case 5: k_dense<T2, 5><<<grid, 256, 0, st>>>(s, d, mat); break;
-        case 6: k_dense<T2, 6><<<grid, 256, 0, st>>>(s, d, mat); break;
+        case 1: k_dense<T2, 1, const T2 *><<<grid, 256, 0, st>>>(s, d, mat); break;
+        case 2: k_dense<T2, 2, const T2 *><<<grid, 256, 0, st>>>(s, d, mat); break;
+        case 3: k_dense<T2, 3, const T2 *><<<grid, 256, 0, st>>>(s, d, mat); break;
+        case 4: k_dense<T2, 4, const T2 *><<<grid, 256, 0, st>>>(s, d, mat); break;
+        case 5: k_dense<T2, 5, const T2 *><<<grid, 256, 0, st>>>(s, d, mat); break;
+        case 6: k_dense<T2, 6, const T2 *><<<grid, 256, 0, st>>>(s, d, mat); break;
         default: break;
     }
+}
+
+template <typename T2, int K>
+static void dense_arg(T2 *s, const GateDesc &d, const T2 *mat, hipStream_t st) {
+    MatArg<T2, K> m;
+    std::copy(mat, mat + (1 << (2 * K)), m.m);
+    k_dense<T2, K, MatArg<T2, K>><<<grid_for(d.iterations, 256, 65536), 256, 0, st>>>(s, d, m);
+}
+
+template <typename T2>
+void launch_dense_arg(T2 *s, const GateDesc &d, const T2 *mat, hipStream_t st) {
+    if (d.k == 1) dense_arg<T2, 1>(s, d, mat, st);
+    else if (d.k == 2) dense_arg<T2, 2>(s, d, mat, st);
+    else if (d.k == 3) dense_arg<T2, 3>(s, d, mat, st);
 }
 
 template <typename T2>
@@ -1508,10 +1538,10 @@ uint32_t expect_batch_segment_bits(uint32_t n) { return std::min<uint32_t>(n, EZ
 
 template <typename T2>
 void launch_collapse(T2 *s, uint64_t len, uint32_t qubit, double uniform, const double *p_one, bool flip,
-                     hipStream_t st) {
+                     double *p_copy, hipStream_t st) {
     const unsigned grid = grid_for(len >> 1, 256, 65536);
-    if (flip) k_collapse<T2, true><<<grid, 256, 0, st>>>(s, len, qubit, uniform, p_one);
-    else k_collapse<T2, false><<<grid, 256, 0, st>>>(s, len, qubit, uniform, p_one);
+    if (flip) k_collapse<T2, true><<<grid, 256, 0, st>>>(s, len, qubit, uniform, p_one, p_copy);
+    else k_collapse<T2, false><<<grid, 256, 0, st>>>(s, len, qubit, uniform, p_one, p_copy);
 }
 
 // Workspace of the allocation-free sampler. In host code `scratch` names a
@@ -1611,6 +1641,7 @@ hipError_t launch_sample_walk(const T2 *s, uint64_t len, uint64_t chunk, uint64_
     template void launch_narrow<T2>(const double2 *, T2 *, uint64_t, hipStream_t);                              \
     template void launch_scale<T2>(T2 *, uint64_t, double, hipStream_t);                                        \
     template void launch_dense<T2>(T2 *, const GateDesc &, const T2 *, hipStream_t);                            \
+    template void launch_dense_arg<T2>(T2 *, const GateDesc &, const T2 *, hipStream_t);                        \
     template void launch_diag<T2>(T2 *, uint64_t, uint32_t, const DiagTargets &, uint64_t, uint64_t, const T2 *, \
                                   hipStream_t);                                                                 \
     template size_t stage_lds_bytes<T2>(uint32_t);                                                              \
@@ -1625,7 +1656,7 @@ hipError_t launch_sample_walk(const T2 *s, uint64_t len, uint64_t chunk, uint64_
                                           const uint32_t *, uint32_t, double *, double *, double *, const ExpDesc &, \
                                           hipStream_t);                                                         \
     template void launch_batch_init<T2>(T2 *, uint64_t, const uint64_t *, uint32_t, hipStream_t);              \
-    template void launch_collapse<T2>(T2 *, uint64_t, uint32_t, double, const double *, bool, hipStream_t);     \
+    template void launch_collapse<T2>(T2 *, uint64_t, uint32_t, double, const double *, bool, double *, hipStream_t); \
     template void launch_sample_sums<T2>(const T2 *, uint64_t, uint64_t, SampleScratch &, hipStream_t);         \
     template hipError_t launch_sample_walk<T2>(const T2 *, uint64_t, uint64_t, uint64_t, SampleScratch &,       \
                                                uint64_t *, hipStream_t);

@@ -96,3 +96,56 @@ def test_batch_values(sizes):
                 wz, wzz = sv.expect_z()
             assert np.max(np.abs(z - wz)) < TOL
             assert zz.size == n - 1 and (n == 1 or np.max(np.abs(zz - wzz)) < TOL)
+
+
+def test_lanes_of_destroyed_handles():
+    """More handles at once than are kept for reuse, from several threads, each
+    measuring its own state: no result reaches another handle's caller."""
+    import threading
+
+    wrong = []
+
+    def work(seed):
+        for i in range(6):
+            svs = [StateVector(4 + (seed + k) % 5, "double") for k in range(3)]
+            for k, sv in enumerate(svs):
+                a = random_state(rng(100 * seed + 10 * i + k), sv.num_qubits)
+                sv.set_amplitudes(a)
+                p = np.abs(a.reshape(-1, 2, 2)[:, 1]) ** 2
+                if abs(sv.probability_one(1) - p.sum()) > TOL or abs(sv.norm_sqr() - 1) > TOL:
+                    wrong.append((seed, i, k))
+            for sv in svs:
+                sv.close()
+
+    threads = [threading.Thread(target=work, args=(s,)) for s in range(5)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not wrong
+
+
+@pytest.mark.parametrize("precision,tol", [("single", 1e-6), ("double", 1e-14)])
+@pytest.mark.parametrize("k,controls", [(1, 0), (1, 2), (2, 0), (2, 1), (3, 0), (3, 1)])
+def test_single_gates_by_argument(k, controls, precision, tol):
+    """A gate by itself on high, low and controlled qubits against the dense
+    product: 2^k complex products and sums of numbers below 1, 34 roundings."""
+    from helpers import full_operator, random_unitary
+
+    n = 7
+    r = rng(60 + k)
+    for qubits in (list(range(k + controls)), list(range(n - k - controls, n))[::-1], [3, 0, 6, 2, 5][: k + controls]):
+        m = random_unitary(r, k)
+        a = random_state(r, n)
+        t, c = qubits[:k], qubits[k:]
+        with StateVector(n, precision) as sv:
+            sv.set_amplitudes(a)
+            start = sv.amplitudes()
+            sv.apply(m, t, [(q, j % 2 == 0) for j, q in enumerate(c)])
+            got = sv.amplitudes()
+        want = full_operator(n, m, t) @ start
+        i = np.arange(1 << n)
+        on = np.ones(1 << n, dtype=bool)
+        for j, q in enumerate(c):
+            on &= ((i >> q) & 1) == (1 if j % 2 == 0 else 0)
+        assert np.max(np.abs(got - np.where(on, want, start))) < tol
