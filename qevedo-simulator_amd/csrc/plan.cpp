@@ -51,11 +51,11 @@ struct Group {
 
 }  // namespace
 
-template <typename F>
-std::vector<Op> fuse_where(const std::vector<Op> &ops, size_t max_qubits, const F &fusable) {
+// fuse_where, handing each group to emit(Op &&) as soon as it is known.
+template <typename F, typename E>
+void fuse_where_each(const std::vector<Op> &ops, size_t max_qubits, const F &fusable, E &&emit) {
     auto width = [&](const Op &op) { return fusable(op) ? op.width() : SIZE_MAX; };
     std::vector<char> done(ops.size(), 0);
-    std::vector<Op> out;
     for (size_t seed = 0; seed < ops.size(); seed++) {
         if (done[seed]) continue;
         done[seed] = 1;
@@ -65,7 +65,7 @@ std::vector<Op> fuse_where(const std::vector<Op> &ops, size_t max_qubits, const 
             g.grow(ops, done, max_qubits, false, width);
         }
         if (g.members.size() == 1) {
-            out.push_back(ops[seed]);
+            emit(Op(ops[seed]));
             continue;
         }
         std::sort(g.qubits.begin(), g.qubits.end());
@@ -80,8 +80,14 @@ std::vector<Op> fuse_where(const std::vector<Op> &ops, size_t max_qubits, const 
         f.targets = g.qubits;
         f.m = std::move(m);
         f.diagonal = f.m.is_diagonal();
-        out.push_back(std::move(f));
+        emit(std::move(f));
     }
+}
+
+template <typename F>
+std::vector<Op> fuse_where(const std::vector<Op> &ops, size_t max_qubits, const F &fusable) {
+    std::vector<Op> out;
+    fuse_where_each(ops, max_qubits, fusable, [&](Op &&op) { out.push_back(std::move(op)); });
     return out;
 }
 
@@ -154,14 +160,18 @@ std::vector<uint32_t> qubits_of(uint64_t mask) {
 
 }  // namespace
 
+void plan_unblocked_each(const std::vector<Op> &ops, uint32_t max_fused, const std::function<void(Op &&)> &emit) {
+    fuse_where_each(ops, std::max<uint32_t>(max_fused, 1), [](const Op &) { return true; }, emit);
+}
+
 std::vector<Step> plan_unblocked(const std::vector<Op> &ops, uint32_t max_fused) {
     std::vector<Step> steps;
-    for (Op &op : fuse(ops, std::max<uint32_t>(max_fused, 1))) {
+    plan_unblocked_each(ops, max_fused, [&](Op &&op) {
         Step s;
         s.is_stage = false;
         s.op = std::move(op);
         steps.push_back(std::move(s));
-    }
+    });
     return steps;
 }
 

@@ -11,6 +11,7 @@
 #pragma once
 
 #include <cstdint>
+#include <functional>
 #include <memory>
 #include <vector>
 
@@ -73,5 +74,7 @@ std::vector<Step> plan_heuristic(std::vector<Op> ops, const PlanParams &p);
 
 // Plan without blocking: fused ops, each its own HBM pass (options.region_bits = None).
 std::vector<Step> plan_unblocked(const std::vector<Op> &ops, uint32_t max_fused);
+// The same ops in the same order, each handed over as soon as it is fused.
+void plan_unblocked_each(const std::vector<Op> &ops, uint32_t max_fused, const std::function<void(Op &&)> &emit);
 
 }  // namespace qvd
