@@ -649,9 +649,39 @@ __device__ __forceinline__ void stage_tiles(T2 *__restrict__ s, const QVD_CONST 
     const QVD_CONST uint32_t *cints = (const QVD_CONST uint32_t *)ints;
     const uint32_t tid_all = threadIdx.x, lane_all = tid_all & 63;
 
-    for (uint32_t i = tid_all; i < d.ccount; i += W) cst[i] = coefs[d.cbegin + i];
+    // The program is read one instruction at a time by scalar loads that every
+    // wave waits for, so on the first tile each line would be a round trip to
+    // memory of its own (stage kernels of a 20-qubit random circuit, one tile per
+    // CU: 381 us, with these loads 292; of a 16-qubit ansatz in complex128: 150
+    // and 88). Its lines are touched here all at once, behind the coefficients'
+    // loads: they are in L2 when the interpreter asks for them, and the
+    // lines that hold the common fields in the scalar cache.
+    {
+        constexpr uint32_t LINE = 64, PER = sizeof(VInstr) / LINE;
+        const uint32_t *const lines = reinterpret_cast<const uint32_t *>(prog + d.instr_off);
+        const uint32_t n = d.num_instr;
+        uint32_t seen = 0;
+        for (uint32_t i = tid_all; i < n * PER; i += W) seen |= lines[i * (LINE / 4)];
+        for (uint32_t i = tid_all; i < d.ccount; i += W) cst[i] = coefs[d.cbegin + i];
+        asm volatile("" ::"v"(seen));
+    }
     const T2 *cbase = cst - d.cbegin;  // so cbase[v.coef + i] is the LDS copy
     __syncthreads();
+    {
+        const QVD_CONST VInstr *const p = cprog + d.instr_off;
+        const uint32_t n = d.num_instr, wave = __builtin_amdgcn_readfirstlane(tid_all >> 6);
+        constexpr uint32_t U = 8, WAVES = W / 64;
+        for (uint32_t i = wave; i < n; i += U * WAVES) {
+            uint32_t w[U];
+#pragma unroll
+            for (uint32_t u = 0; u < U; u++) {
+                const uint32_t at = i + u * WAVES;
+                w[u] = p[at < n ? at : i].op;
+            }
+#pragma unroll
+            for (uint32_t u = 0; u < U; u++) asm volatile("" ::"s"(w[u]));
+        }
+    }
 
     // Physical offsets of the initial role map (loads) and the final one
     // (stores): thread part per lane, register part per register bit.
