@@ -20,18 +20,16 @@
 // is in flight from memory, and it is written to the other buffer before the
 // one barrier of the iteration.
 //
-// Bounds at 28 qubits (2^28 columns x amplitudes): one pass is 0.79 ms in
-// complex64 and 1.58 ms in complex128 at the 5.4 TB/s of a large copy; the
-// products of a 6-qubit gate are 0.87 ms at the FP32 matrix peak and 1.75 ms
-// at the FP64 one (78.6 TFLOP/s, as the FP64 vector rate), half of that for 5
-// qubits. Measured, host call included: K = 6 1.23 ms and 2.14 ms (the
-// products, at 71 and 82 % of their peak), K = 5 0.95 ms and 1.67-1.84 ms
-// (memory). Before, with one LDS buffer, outputs through LDS and four barriers
-// per block, FP32 K = 6 took 1.38 ms and K = 5 0.97 ms; complex128 ran on
-// vector FMAs with the matrix in LDS: 12.0 ms and 9.1 ms. Blocks of 64
-// columns: 1.26 and 2.46 ms. Workgroups per CU: two for K = 6, what its
-// registers allow (12: 1.28 ms, each workgroup loading its rows of R again);
-// many small ones for the others (K = 5 in FP32: 2 1.04, 3 0.92, 12 0.92 ms).
+// Bounds at 28 qubits: one pass is 0.79 ms in complex64 and 1.58 ms in
+// complex128 at the 5.4 TB/s of a large copy; the products of a 6-qubit gate
+// are 0.87 ms at the FP32 matrix peak and 1.75 ms at the FP64 one
+// (78.6 TFLOP/s, as the FP64 vector rate), half of that for 5 qubits. Measured
+// kernels: K = 6 1.16-1.21 ms and 2.06-2.10 ms (the products, at 72 to 75 and
+// 83 to 85 % of their peak), K = 5 0.87-0.92 ms and 1.62-1.80 ms (memory); one
+// LDS buffer, outputs through LDS and four barriers per block took 1.32-1.50
+// and 0.89-1.19 ms in complex64. At 32 qubits K = 6 takes 18.1-19.7 ms
+// (20.2-22.9). 74 registers in complex64 leave room for three workgroups of
+// K = 6 on a CU; with 84 there were two (28 qubits: 1.24-1.43 ms).
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -80,6 +78,21 @@ static_assert(NC == 1 << CB, "a block's columns are all values of its column bit
 template <typename T2> constexpr int PITCH = sizeof(T2) == 8 ? NC + 16 : NC + 1;
 template <typename T2, int K> constexpr int BLOCK = (1 << K) * PITCH<T2>;  // amplitudes of one staged block
 constexpr int SLOTS = 3;       // column bases of the block multiplied, loaded and prepared
+constexpr int PER = 4;         // amplitudes staged per thread (8 D threads, D x NC amplitudes)
+
+// Where a staged amplitude belongs: its column in the block, its place in the
+// buffer and its offset within the column. Each is a sum over the bits of the
+// amplitude's number tid + i * threads, so tid's part is a thread's own and i's
+// part the same for the workgroup (three registers a thread instead of 16).
+struct Place {
+    uint64_t off;
+    uint32_t col, at;
+};
+template <int K>
+struct Places {
+    Place bit[K + 3];  // of each bit of tid
+    Place elem[PER];   // of each i
+};
 
 __device__ __forceinline__ uint64_t spread(uint64_t x, const uint32_t *pos, uint32_t m) {
     for (uint32_t j = 0; j < m; j++) {
@@ -90,6 +103,13 @@ __device__ __forceinline__ uint64_t spread(uint64_t x, const uint32_t *pos, uint
     return x;
 }
 
+// v, unknown to the optimiser: what is computed from it is not kept in registers
+// across a loop.
+__device__ __forceinline__ uint32_t opaque(uint32_t v) {
+    asm volatile("" : "+v"(v));
+    return v;
+}
+
 template <typename T2, int K>
 constexpr size_t mfma_lds_bytes() {
     return 2 * sizeof(T2) * (size_t)BLOCK<T2, K> + SLOTS * NC * sizeof(uint64_t);
@@ -97,13 +117,13 @@ constexpr size_t mfma_lds_bytes() {
 
 template <typename T2, int K>
 __global__ __launch_bounds__(64 << (K - 3)) void k_dense_mfma(T2 *__restrict__ s, const GateDesc d,
-                                                              const T2 *__restrict__ mat) {
+                                                              const T2 *__restrict__ mat, const Places<K> p) {
     using M = Mfma<T2>;
     using R = typename M::R;
     using V = typename M::V;
     constexpr int D = 1 << K, THREADS = 8 * D;  // 2D / 16 waves
     constexpr int KS = 2 * D / 4;               // k steps of 4
-    constexpr int PER = D * NC / THREADS;       // amplitudes staged per thread
+    static_assert(D * NC == PER * THREADS, "a block is PER amplitudes a thread");
     constexpr uint64_t NONE = ~uint64_t(0);     // a column past the last one
     extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
     T2 *const buf = reinterpret_cast<T2 *>(smem_raw);                       // two blocks
@@ -124,62 +144,46 @@ __global__ __launch_bounds__(64 << (K - 3)) void k_dense_mfma(T2 *__restrict__ s
     // lane's accumulators e are index 2q + e / 2 of the wave's 8 and part
     // e % 2. k = 4 ks + q is index k % D, part k / D in complex64, index k / 2,
     // part k % 2 in complex128.
+    // Every load is unconditional: where a part was chosen after the load, the
+    // compiler branched around each one and waited for it (20 qubits, K = 6:
+    // 27.5 us a pass, 14.8 so).
     constexpr bool PLANES = sizeof(T2) == 8;
     R ra[KS];
     {
         const uint32_t jr = wave * 8 + 2 * M::q_of(cl) + (M::e_of(cl) >> 1), im = M::e_of(cl) & 1;
+        if constexpr (PLANES) {
 #pragma unroll
-        for (int ks = 0; ks < KS; ks++) {
-            const uint32_t k = 4 * ks + q;
-            const T2 u = mat[jr * D + (PLANES ? k & (D - 1) : k >> 1)];
-            ra[ks] = (PLANES ? k >> K : k & 1) == im ? u.x : (im ? u.y : -u.y);
-        }
-    }
-    // Staging order: element e of a block takes its index bits in ascending
-    // order of the qubits they stand for (targets, and the lowest free qubits
-    // that the columns of a block span), so neighbouring threads load
-    // neighbouring amplitudes whichever qubits the targets are. `tq` and `fq`
-    // walk both sets; a free bit past the last qubit is a column past the
-    // last one.
-    uint32_t tbits[K + CB];  // bit i of e: index bit (below K) or K + column bit
-    {
-        uint32_t f = 0, fq = 0, ins = 0;  // next column bit, its qubit, the inserted (target or control) qubits passed
-        uint32_t used = 0;                // targets taken
-        for (int i = 0; i < K + CB; i++) {
-            while (ins < d.nins && d.ins[ins] <= fq) {  // fq: the next qubit that is no target or control
-                if (d.ins[ins] == fq) fq++;
-                ins++;
+            for (int ks = 0; ks < KS / 2; ks++) {
+                const T2 u = mat[jr * D + 4 * ks + q];
+                ra[ks] = im ? u.y : u.x;
+                ra[ks + KS / 2] = im ? u.x : -u.y;
             }
-            uint32_t lowest = 0;
-            uint64_t lo = ~uint64_t(0);
+        } else {
+            const R *const row = reinterpret_cast<const R *>(mat + jr * D + (q >> 1)) + ((q & 1) ^ im);
+            const bool neg = (q & 1) > im;
 #pragma unroll
-            for (int t = 0; t < K; t++)
-                if (!((used >> t) & 1) && d.offsets[1 << t] < lo) {
-                    lo = d.offsets[1 << t];
-                    lowest = t;
-                }
-            if (f < (uint32_t)CB && (used == (1u << K) - 1 || (uint64_t(1) << fq) < lo)) {
-                tbits[i] = K + f++;
-                fq++;
-            } else {
-                tbits[i] = lowest;
-                used |= 1u << lowest;
+            for (int ks = 0; ks < KS; ks++) {
+                const R v = row[4 * ks];
+                ra[ks] = neg ? -v : v;
             }
         }
     }
-    uint64_t eo[PER];           // offset of each staged amplitude within its column
-    uint32_t ec[PER], ea[PER];  // its column in the block, its place in the buffer
+    // The thread's part of the place of its elements tid + i * THREADS.
+    uint32_t c_tid = 0, a_tid = 0;
+    uint64_t o_tid = 0;
 #pragma unroll
-    for (int i = 0; i < PER; i++) {
-        const uint32_t e = tid + i * THREADS;
-        uint32_t jc = 0;
-        for (int b = 0; b < K + CB; b++) jc |= ((e >> b) & 1) << tbits[b];
-        const uint32_t j = jc & (D - 1);
-        ec[i] = jc >> K;
-        ea[i] = j * PITCH<T2> + ec[i];
-        eo[i] = d.offsets[j];
+    for (int b = 0; b < K + 3; b++) {
+        const uint32_t bit = (tid >> b) & 1;
+        c_tid += bit ? p.bit[b].col : 0;
+        a_tid += bit ? p.bit[b].at : 0;
+        o_tid += bit ? p.bit[b].off : 0;
     }
-    const uint64_t so0 = d.offsets[wave * 8 + 2 * q], so1 = d.offsets[wave * 8 + 2 * q + 1];
+    // Accumulators 0, 1 are index `wave * 8 + 2 q`, 2 and 3 the next one.
+    uint64_t so = 0;
+    const uint64_t so_next = d.offsets[1];
+#pragma unroll
+    for (int t = 1; t < K; t++)
+        if (((t < 3 ? 2 * q : wave * 8) >> t) & 1) so += d.offsets[1u << t];
 
     // Qubit 0 is matrix bit 0: a lane's two amplitudes are neighbours, the
     // first at an even index (16-byte aligned in complex64).
@@ -190,24 +194,26 @@ __global__ __launch_bounds__(64 << (K - 3)) void k_dense_mfma(T2 *__restrict__ s
     __syncthreads();
     T2 pre[PER];
     auto fetch = [&](uint32_t slot) {
+        const uint32_t c = opaque(c_tid);
 #pragma unroll
         for (int i = 0; i < PER; i++) {
-            const uint64_t b = colbase[slot * NC + ec[i]];
+            const uint64_t b = colbase[slot * NC + c + p.elem[i].col];
             pre[i].x = pre[i].y = 0;
-            if (b != NONE) pre[i] = s[b + eo[i]];
+            if (b != NONE) pre[i] = s[b + o_tid + p.elem[i].off];
         }
     };
     auto stage = [&](T2 *b) {
+        const uint32_t a = opaque(a_tid);
         if constexpr (PLANES) {
             R *const f = reinterpret_cast<R *>(b);
 #pragma unroll
             for (int i = 0; i < PER; i++) {
-                f[ea[i]] = pre[i].x;
-                f[BLOCK<T2, K> + ea[i]] = pre[i].y;
+                f[a + p.elem[i].at] = pre[i].x;
+                f[BLOCK<T2, K> + a + p.elem[i].at] = pre[i].y;
             }
         } else {
 #pragma unroll
-            for (int i = 0; i < PER; i++) b[ea[i]] = pre[i];
+            for (int i = 0; i < PER; i++) b[a + p.elem[i].at] = pre[i];
         }
     };
     fetch(0);
@@ -243,10 +249,10 @@ __global__ __launch_bounds__(64 << (K - 3)) void k_dense_mfma(T2 *__restrict__ s
                 o1.x = acc[g][2];
                 o1.y = acc[g][3];
                 if (sizeof(T2) == 8 && adjacent) {
-                    *reinterpret_cast<float4 *>(s + b + so0) = make_float4(o0.x, o0.y, o1.x, o1.y);
+                    *reinterpret_cast<float4 *>(s + b + so) = make_float4(o0.x, o0.y, o1.x, o1.y);
                 } else {
-                    s[b + so0] = o0;
-                    s[b + so1] = o1;
+                    s[b + so] = o0;
+                    s[b + so + so_next] = o1;
                 }
             }
         }
@@ -257,6 +263,71 @@ __global__ __launch_bounds__(64 << (K - 3)) void k_dense_mfma(T2 *__restrict__ s
         slot = slot1;
         blk = next;
     }
+}
+
+// The staging order: bit b of an amplitude's number is an index bit of the gate
+// or a column bit. The lowest ones follow the qubits they stand for (targets,
+// and the lowest free qubits, which the columns of a block span) over a
+// 128-byte line, so neighbouring threads load whole lines whichever qubits the
+// targets are. Then come the other column bits, then the other index bits: a
+// wave writes a few rows of the buffer, not one per thread, whose starts share
+// banks in complex64 (targets 0 to 5, 28 qubits, two workgroups per CU: 1434 us a
+// pass with a row per thread, 1311 so). A free bit past the last qubit is a column past the last one.
+template <typename T2, int K>
+Places<K> staging_places(const GateDesc &d) {
+    constexpr int LINE = sizeof(T2) == 8 ? 4 : 3;  // bits of an amplitude's place in a line
+    Place bits[K + CB];
+    int at = 0, f = 0;  // bits and column bits placed
+    uint32_t used = 0, fq = 0, ins = 0;  // targets placed, the next free qubit, targets and controls below it
+    auto column = [&] {
+        bits[at++] = {0, 1u << f, 1u << f};
+        f++;
+        fq++;
+    };
+    auto target = [&](int t) {
+        bits[at++] = {d.offsets[1 << t], 0, (uint32_t)PITCH<T2> << t};
+        used |= 1u << t;
+    };
+    auto lowest = [&] {  // of the targets left, or -1
+        int t = -1;
+        for (int k = 0; k < K; k++)
+            if (!((used >> k) & 1) && (t < 0 || d.offsets[1 << k] < d.offsets[1 << t])) t = k;
+        return t;
+    };
+    while (at < LINE) {
+        for (; ins < d.nins && d.ins[ins] <= fq; ins++) fq += d.ins[ins] == fq;
+        const int t = lowest();
+        if (t < 0 || (f < CB && (uint64_t(1) << fq) < d.offsets[1 << t])) column();
+        else target(t);
+    }
+    while (f < CB) column();
+    for (int t; (t = lowest()) >= 0;) target(t);
+    Places<K> p;
+    std::copy(bits, bits + K + 3, p.bit);
+    for (int i = 0; i < PER; i++) {
+        p.elem[i] = {0, 0, 0};
+        for (int b = 0; b < 2; b++) {
+            const Place &x = bits[K + 3 + b];
+            if ((i >> b) & 1) p.elem[i] = {p.elem[i].off + x.off, p.elem[i].col + x.col, p.elem[i].at + x.at};
+        }
+    }
+    return p;
+}
+
+// Workgroups launched per CU, given the blocks per CU. K = 6: two are resident
+// in complex128 and three in complex64, where an odd number of them leaves the last
+// round uneven unless there are many rounds (22 qubits, 8 blocks per CU: two 45 us,
+// three 51, six 71; 24 qubits: 103, 106, 119). From 128 blocks per CU on, more
+// of them than are resident start as others end, which evens their
+// rounds out (26 qubits: two 337 us, six 337; 28: 1264 and 1215; 32: 21.6 and
+// 19.7 ms). K = 5 in complex64 is the same from 512 on (28 qubits, 12 per CU 922 us,
+// 24 899; 24 qubits: 71 and 84); in complex128 12 are as good (28 qubits: 1.67
+// ms, 24 1.69). Fewer targets: many small ones.
+template <typename T2, int K>
+uint64_t groups_per_cu(uint64_t blocks) {
+    if (K == 6) return sizeof(T2) == 8 && blocks >= 128 ? 6 : 2;
+    if (K == 5) return sizeof(T2) == 8 && blocks >= 512 ? 24 : 12;
+    return 32;
 }
 
 template <typename T2, int K>
@@ -273,8 +344,8 @@ hipError_t launch_k(T2 *s, const GateDesc &d, const T2 *mat, unsigned cus, hipSt
         attr_set.fetch_or(bit);
     }
     const uint64_t blocks = (d.iterations + NC - 1) / NC;
-    const unsigned grid = (unsigned)std::min<uint64_t>(blocks, (uint64_t)cus * (K == 6 ? 2 : K == 5 ? 12 : 32));
-    k_dense_mfma<T2, K><<<grid, 64 << (K - 3), lds, st>>>(s, d, mat);
+    const unsigned grid = (unsigned)std::min<uint64_t>(blocks, cus * groups_per_cu<T2, K>(blocks / cus));
+    k_dense_mfma<T2, K><<<grid, 64 << (K - 3), lds, st>>>(s, d, mat, staging_places<T2, K>(d));
     return hipGetLastError();
 }
 
