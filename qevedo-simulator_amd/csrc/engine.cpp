@@ -455,8 +455,8 @@ void apply_full(qvd_sv *sv, T2 *s, const Op &op, const T2 *coef, bool valu_only 
         QVD_HIP(launch_dense_mfma<T2>(s, d, coef, (unsigned)num_cus(sv->device), sv->stream));
         return;
     }
-    if (by_arg) launch_dense_arg<T2>(s, d, coef, sv->stream);
-    else launch_dense<T2>(s, d, coef, sv->stream);
+    if (by_arg) launch_dense_arg<T2>(s, sv->len, d, coef, sv->stream);
+    else launch_dense<T2>(s, sv->len, d, coef, sv->stream);
     QVD_HIP(hipGetLastError());
 }
 

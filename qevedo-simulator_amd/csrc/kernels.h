@@ -64,11 +64,13 @@ void launch_expect_pauli(const T2 *s, uint64_t len, const PauliGroup *groups, co
 template <typename T2> void launch_widen(const T2 *s, double2 *out, uint64_t count, hipStream_t st);
 template <typename T2> void launch_narrow(const double2 *in, T2 *s, uint64_t count, hipStream_t st);
 template <typename T2> void launch_scale(T2 *s, uint64_t len, double factor, hipStream_t st);
-template <typename T2> void launch_dense(T2 *s, const GateDesc &d, const T2 *mat, hipStream_t st);
+// len: the state's amplitudes.
+template <typename T2> void launch_dense(T2 *s, uint64_t len, const GateDesc &d, const T2 *mat, hipStream_t st);
 // The same for up to DENSE_ARG_QUBITS targets with the matrix in host memory,
 // passed as kernel arguments.
 constexpr uint32_t DENSE_ARG_QUBITS = 3;
-template <typename T2> void launch_dense_arg(T2 *s, const GateDesc &d, const T2 *mat, hipStream_t st);
+template <typename T2>
+void launch_dense_arg(T2 *s, uint64_t len, const GateDesc &d, const T2 *mat, hipStream_t st);
 template <typename T2>
 void launch_diag(T2 *s, uint64_t len, uint32_t k, const DiagTargets &t, uint64_t cmask, uint64_t cval,
                  const T2 *entries, hipStream_t st);

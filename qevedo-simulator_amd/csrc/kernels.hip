@@ -134,11 +134,20 @@ __global__ void k_scale(T2 *__restrict__ s, uint64_t len, double factor) {
 
 // A dense op on K targets: each thread owns one group of 2^K amplitudes
 // (the iteration index spread over the non-target, non-control bits). The
-// matrix is the same for every thread: its rows come through the scalar
-// cache and enter the FMAs as scalar operands, so a pass is bound by memory up
-// to K = 4 (28 qubits, targets 4-7: 0.82 ms in complex64 and 1.60 ms in
-// complex128, a copy of the state taking 0.79 and 1.58; read from LDS, each
-// element per FMA pair, the matrix bound it at 1.72 and 7.9 ms).
+// matrix is the same for every thread. For K <= 2 it sits in scalar registers
+// as a whole and enters the FMAs from there. From K = 3 on its rows come from
+// LDS, a few at a time: that keeps the registers to what a wave needs (all
+// rows unrolled, the compiler holds the matrix and one wave per SIMD is left),
+// and a row is there in the time of an LDS read. Rows through the scalar
+// cache are waited for one by one (20 qubits, complex64, 4 targets: 12.0 us, 9.1
+// so; 18 qubits, complex128, 3 targets: 7.5 and 6.6), and a 6-qubit matrix in
+// complex128 does not fit it (24 qubits: 950 us, 648 so). Only the
+// 4-qubit gates of complex128 stay there: their states are read by half as many
+// threads, which covers the waits (27 qubits, targets 23-26: 0.85 ms, 0.94
+// from LDS).
+//
+// A pass is bound by memory up to K = 4 (28 qubits, targets 4-7: 0.78 ms in
+// complex64 and 1.60 ms in complex128, a copy of the state taking 0.79 and 1.58).
 //
 // The matrix is in device memory, or is itself an argument of the launch
 // (MatArg; a gate applied by itself needs no copy in front of its pass then).
@@ -155,25 +164,37 @@ __device__ __forceinline__ T2 mat_at(const MatArg<T2, K> &mat, int i) {
     return mat.m[i];
 }
 
+template <typename T2>
+constexpr bool dense_in_lds(int k) {
+    return k >= 3 && !(sizeof(T2) == 16 && k == 4);
+}
+
 template <typename T2, int K, typename M>
 __global__ __launch_bounds__(256) void k_dense(T2 *__restrict__ s, const GateDesc d, const M mat) {
     constexpr int D = 1 << K;
+    constexpr bool LDS = dense_in_lds<T2>(K);
+    extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
+    T2 *const m = reinterpret_cast<T2 *>(smem_raw);
+    if (LDS) {
+        for (int i = threadIdx.x; i < D * D; i += blockDim.x) m[i] = mat_at(mat, i);
+        __syncthreads();
+    }
     const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
     for (uint64_t it = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; it < d.iterations; it += stride) {
         T2 *const g = s + (insert_zeros(it, d.ins, d.nins) | d.ctrl_val);
         T2 a[D];
 #pragma unroll
         for (int j = 0; j < D; j++) a[j] = g[d.offsets[j]];
-        // One row at a time from K = 3 on: unrolled, the compiler loads the
-        // whole matrix ahead and spills it.
-        constexpr int U = K < 3 ? D : 1;
+        // Rows in batches whose matrix elements are 64 registers at most.
+        constexpr int FIT = 256 / (D * (int)sizeof(T2));
+        constexpr int U = K < 3 ? D : FIT > 1 ? FIT : 1;
 #pragma unroll U
         for (int r = 0; r < D; r++) {
             T2 acc;
             acc.x = 0;
             acc.y = 0;
 #pragma unroll
-            for (int c = 0; c < D; c++) cmac(acc, mat_at(mat, r * D + c), a[c]);
+            for (int c = 0; c < D; c++) cmac(acc, LDS ? m[r * D + c] : mat_at(mat, r * D + c), a[c]);
             g[d.offsets[r]] = acc;
         }
     }
@@ -1356,32 +1377,53 @@ void launch_scale(T2 *s, uint64_t len, double factor, hipStream_t st) {
     k_scale<T2><<<grid_for(len, 256), 256, 0, st>>>(s, len, factor);
 }
 
+// Dynamic LDS of a k_dense launch: the matrix, or so much that three workgroups
+// fit on a CU. On states far beyond the Infinity Cache, three waves per SIMD read and
+// write memory in fewer places at a time than eight (28 qubits in complex64, 1
+// target 0.81-0.87 ms, so 0.79-0.80; 2 targets 0.80-1.02 and 0.76-0.94; in
+// complex128 2 targets 1.62-1.93 and 1.57-1.82). From 1 GiB on that holds
+// for every gate; at 512 MiB for threads that hold more than 32 bytes
+// (25 qubits in complex128, 2 targets: 183-219 us, so 181-214; 26 qubits in
+// complex64, 1 target: 185-198 us, so 197-209). Below, three are too few (25
+// qubits in complex64, 1 target: 69 us, 83 so). 4 targets and more in
+// complex128 have few waves by their registers.
 template <typename T2>
-void launch_dense(T2 *s, const GateDesc &d, const T2 *mat, hipStream_t st) {
+static size_t dense_lds(uint64_t len, uint32_t k) {
+    const size_t matrix = dense_in_lds<T2>(k) ? sizeof(T2) << (2 * k) : 0;
+    const uint64_t bytes = len * sizeof(T2);
+    const bool large = bytes >= (uint64_t(1) << 30) || (bytes >= (uint64_t(1) << 29) && (sizeof(T2) << k) > 32);
+    // 52 KiB: LDS is handed out in pieces of 1280 bytes, 128 to a CU.
+    return large && k <= (sizeof(T2) == 8 ? 4 : 3) ? std::max<size_t>(matrix, 52 * 1024) : matrix;
+}
+
+template <typename T2>
+void launch_dense(T2 *s, uint64_t len, const GateDesc &d, const T2 *mat, hipStream_t st) {
     const unsigned grid = grid_for(d.iterations, 256, 65536);
+    const size_t lds = dense_lds<T2>(len, d.k);
     switch (d.k) {
-        case 1: k_dense<T2, 1, const T2 *><<<grid, 256, 0, st>>>(s, d, mat); break;
-        case 2: k_dense<T2, 2, const T2 *><<<grid, 256, 0, st>>>(s, d, mat); break;
-        case 3: k_dense<T2, 3, const T2 *><<<grid, 256, 0, st>>>(s, d, mat); break;
-        case 4: k_dense<T2, 4, const T2 *><<<grid, 256, 0, st>>>(s, d, mat); break;
-        case 5: k_dense<T2, 5, const T2 *><<<grid, 256, 0, st>>>(s, d, mat); break;
-        case 6: k_dense<T2, 6, const T2 *><<<grid, 256, 0, st>>>(s, d, mat); break;
+        case 1: k_dense<T2, 1, const T2 *><<<grid, 256, lds, st>>>(s, d, mat); break;
+        case 2: k_dense<T2, 2, const T2 *><<<grid, 256, lds, st>>>(s, d, mat); break;
+        case 3: k_dense<T2, 3, const T2 *><<<grid, 256, lds, st>>>(s, d, mat); break;
+        case 4: k_dense<T2, 4, const T2 *><<<grid, 256, lds, st>>>(s, d, mat); break;
+        case 5: k_dense<T2, 5, const T2 *><<<grid, 256, lds, st>>>(s, d, mat); break;
+        case 6: k_dense<T2, 6, const T2 *><<<grid, 256, lds, st>>>(s, d, mat); break;
         default: break;
     }
 }
 
 template <typename T2, int K>
-static void dense_arg(T2 *s, const GateDesc &d, const T2 *mat, hipStream_t st) {
+static void dense_arg(T2 *s, uint64_t len, const GateDesc &d, const T2 *mat, hipStream_t st) {
     MatArg<T2, K> m;
     std::copy(mat, mat + (1 << (2 * K)), m.m);
-    k_dense<T2, K, MatArg<T2, K>><<<grid_for(d.iterations, 256, 65536), 256, 0, st>>>(s, d, m);
+    k_dense<T2, K, MatArg<T2, K>>
+        <<<grid_for(d.iterations, 256, 65536), 256, dense_lds<T2>(len, K), st>>>(s, d, m);
 }
 
 template <typename T2>
-void launch_dense_arg(T2 *s, const GateDesc &d, const T2 *mat, hipStream_t st) {
-    if (d.k == 1) dense_arg<T2, 1>(s, d, mat, st);
-    else if (d.k == 2) dense_arg<T2, 2>(s, d, mat, st);
-    else if (d.k == 3) dense_arg<T2, 3>(s, d, mat, st);
+void launch_dense_arg(T2 *s, uint64_t len, const GateDesc &d, const T2 *mat, hipStream_t st) {
+    if (d.k == 1) dense_arg<T2, 1>(s, len, d, mat, st);
+    else if (d.k == 2) dense_arg<T2, 2>(s, len, d, mat, st);
+    else if (d.k == 3) dense_arg<T2, 3>(s, len, d, mat, st);
 }
 
 template <typename T2>
@@ -1640,8 +1682,8 @@ hipError_t launch_sample_walk(const T2 *s, uint64_t len, uint64_t chunk, uint64_
     template void launch_widen<T2>(const T2 *, double2 *, uint64_t, hipStream_t);                               \
     template void launch_narrow<T2>(const double2 *, T2 *, uint64_t, hipStream_t);                              \
     template void launch_scale<T2>(T2 *, uint64_t, double, hipStream_t);                                        \
-    template void launch_dense<T2>(T2 *, const GateDesc &, const T2 *, hipStream_t);                            \
-    template void launch_dense_arg<T2>(T2 *, const GateDesc &, const T2 *, hipStream_t);                        \
+    template void launch_dense<T2>(T2 *, uint64_t, const GateDesc &, const T2 *, hipStream_t);                  \
+    template void launch_dense_arg<T2>(T2 *, uint64_t, const GateDesc &, const T2 *, hipStream_t);              \
     template void launch_diag<T2>(T2 *, uint64_t, uint32_t, const DiagTargets &, uint64_t, uint64_t, const T2 *, \
                                   hipStream_t);                                                                 \
     template size_t stage_lds_bytes<T2>(uint32_t);                                                              \

@@ -35,3 +35,21 @@ def test_against_the_vector_kernel(precision, n, targets, controls):
             sv.apply_ops(state)
             sv.apply_ops(op, len(targets), None, dense_valu=vector)
         assert a.compare(b)["rel_l2"] < (3e-6 if precision == "single" else 3e-14)
+
+
+@pytest.mark.parametrize("precision,n", [("single", 25), ("single", 26), ("single", 27), ("double", 25), ("double", 26)])
+@pytest.mark.parametrize("targets,controls", [([1], [(0, True)]), ([24], []), ([0, 3], []), ([7, 2], [(24, False)]),
+                                              ([1, 3, 5], []), ([23, 0, 12], [(1, True)]), ([9, 4, 7, 2], [])])
+def test_vector_kernel_on_large_states(precision, n, targets, controls):
+    """Sizes on both sides of the lines (512 MiB, 1 GiB) at which the vector
+    kernel's launches change, against the stage kernel on the device."""
+    state = lower_gates(library.random_circuit(n, 2, 5))
+    u = unitary(n, len(targets))
+    with StateVector(n, precision) as a, StateVector(n, precision) as b:
+        a.apply_ops(state)
+        a.apply(u, targets, controls)
+        a.apply_ops([(targets, controls, u)], len(targets), None)
+        b.apply_ops(state)
+        b.apply_ops([(targets, controls, u)])
+        b.apply_ops([(targets, controls, u)])
+        assert a.compare(b)["rel_l2"] < (3e-6 if precision == "single" else 3e-14)
