@@ -788,8 +788,8 @@ void run_unblocked(qvd_sv *sv, T2 *s, const std::vector<Op> &ops, const qvd_opti
         materialize(sv, false);  // ordered before the passes by the stream
     }
     // Coefficients go up one op behind the other through the handle's plan
-    // arena; when it is full the queued passes are waited for. The host copies
-    // live until the end.
+    // arena; when it is full the queued passes are waited for, and the host copies
+    // of what they read are let go.
     size_t widest = std::max<uint32_t>(opt.max_fused_qubits, 1);
     for (const Op &op : ops) widest = std::max(widest, op.targets.size());
     widest = std::min<size_t>(widest, MAX_GATE_QUBITS);
@@ -807,14 +807,16 @@ void run_unblocked(qvd_sv *sv, T2 *s, const std::vector<Op> &ops, const qvd_opti
         plan_unblocked_each(ops, opt.max_fused_qubits, [&](Op &&op) {
             const double t1 = now();
             check_full_width(op);
-            sent.push_back(full_coefficients<T2>(op));
-            const std::vector<T2> &c = sent.back();
-            const size_t bytes = (c.size() * sizeof(T2) + 255) & ~size_t(255);
+            std::vector<T2> coefs = full_coefficients<T2>(op);
+            const size_t bytes = (coefs.size() * sizeof(T2) + 255) & ~size_t(255);
             require(bytes <= arena, "internal: an op's matrix exceeds the plan arena");
             if (at + bytes > arena) {
                 sv->sync();
+                sent.clear();
                 at = 0;
             }
+            sent.push_back(std::move(coefs));
+            const std::vector<T2> &c = sent.back();
             char *const coef = sv->plan_ws.as<char>() + at;
             at += bytes;
             QVD_HIP(hipMemcpyAsync(coef, c.data(), c.size() * sizeof(T2), hipMemcpyHostToDevice, sv->stream));
