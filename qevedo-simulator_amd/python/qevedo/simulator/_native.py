@@ -197,18 +197,16 @@ def gate_matrix(name: str, params=()) -> np.ndarray:
 _LOWER_OUT = C.c_double * (2 * 64)
 # ctypes arrays of up to 8 parameters (a new array type costs more than the call).
 _LOWER_PARAMS = tuple(C.c_double * max(k, 1) for k in range(9))
+_NUMBERS = {float, int, np.float64}
 
 
 def gate_lower(name: str, params=()) -> tuple:
     """(number of leading controls, base matrix) of a named gate."""
-    if not isinstance(params, (list, tuple)):
+    if not (isinstance(params, (list, tuple)) and set(map(type, params)) <= _NUMBERS):
+        # numbers of NumPy's own, texts, nested lists
         params = np.ascontiguousarray(params, dtype=np.float64).reshape(-1).tolist()
     n = len(params)
-    array = _LOWER_PARAMS[n] if n < len(_LOWER_PARAMS) else C.c_double * n
-    try:
-        p = array(*params)
-    except TypeError:  # what only NumPy turns into a number
-        p = array(*np.ascontiguousarray(params, dtype=np.float64).tolist())
+    p = (_LOWER_PARAMS[n] if n < len(_LOWER_PARAMS) else C.c_double * n)(*params)
     out = _LOWER_OUT()
     nc, nt = C.c_uint32(), C.c_uint32()
     _check(lib().qvd_gate_lower(name.encode(), p, n, C.byref(nc), C.byref(nt), out, 64))
@@ -236,6 +234,13 @@ _OP = np.dtype([("targets", "u8"), ("num_targets", "u4"), ("pad0", "u4"), ("cont
 assert _OP.itemsize == C.sizeof(Op)
 
 
+def _qubit_list(qubits):
+    """Qubits as a flat list, from any form NumPy takes as an array of them."""
+    if isinstance(qubits, (list, tuple)) and set(map(type, qubits)) <= {int}:
+        return qubits
+    return np.ascontiguousarray(qubits, dtype=np.uint32).reshape(-1).tolist()
+
+
 class OpArray:
     """A qvd_op array plus the NumPy buffers it points into: all ops' targets,
     controls and control values in one buffer each, each matrix object once."""
@@ -246,8 +251,7 @@ class OpArray:
         self.keep = []
         qubits, values, counts, addresses = [], [], [], []
         for targets, controls, matrix in ops:
-            if not isinstance(targets, (list, tuple)):
-                targets = np.ascontiguousarray(targets, dtype=np.uint32).reshape(-1).tolist()
+            targets = _qubit_list(targets)
             entry = matrices.get(id(matrix))
             if entry is None:
                 m = np.ascontiguousarray(matrix, dtype=np.complex128)
@@ -261,9 +265,9 @@ class OpArray:
             counts.append(len(targets))
             counts.append(len(controls))
             addresses.append(entry[0])
-            for c in controls:
-                qubits.append(c[0])
-                values.append(1 if c[1] else 0)
+            if len(controls):
+                qubits += _qubit_list([c[0] for c in controls])
+                values += [1 if c[1] else 0 for c in controls]
         qubits = np.array(qubits, dtype=np.uint32)
         values = np.array(values, dtype=np.uint8)
         counts = np.array(counts, dtype=np.uint64).reshape(-1, 2)
