@@ -2189,19 +2189,19 @@ int qvd_sv_expect_pauli(const qvd_sv *sv_c, const uint64_t *x_masks, const uint6
                 widths.push_back(g.nterms);
             }
             const size_t k = zs.size(), gw = sizeof(PauliGroup) / sizeof(double) * groups.size();
-            const unsigned blocks = pauli_blocks(sv->len, (uint32_t)groups.size());
+            const PauliLaunches launches = pauli_launches(sv->len, widths);
             std::vector<uint64_t> up(gw + k);
             std::memcpy(up.data(), groups.data(), groups.size() * sizeof(PauliGroup));
             std::memcpy(up.data() + gw, zs.data(), k * sizeof(uint64_t));
             // sums, descriptors and Z parts, then the blocks' partial sums;
             // a page's worth of sums goes straight to the host
-            double *buf = sv->scratch_doubles(k + up.size() + k * blocks);
+            double *buf = sv->scratch_doubles(k + up.size() + launches.partials);
             const bool mail = k <= MAIL_DOUBLES;
             uint64_t *dg = reinterpret_cast<uint64_t *>(buf + k);
             QVD_HIP(hipMemcpyAsync(dg, up.data(), up.size() * sizeof(uint64_t), hipMemcpyHostToDevice, sv->stream));
             with_type(sv, [&](auto *s) {
-                launch_expect_pauli(s, sv->len, reinterpret_cast<const PauliGroup *>(dg), widths, dg + gw, (uint32_t)k,
-                                    buf + k + up.size(), blocks, mail ? sv->lane.mail_dev : buf, sv->stream);
+                launch_expect_pauli(s, sv->len, reinterpret_cast<const PauliGroup *>(dg), launches, dg + gw,
+                                    (uint32_t)k, buf + k + up.size(), mail ? sv->lane.mail_dev : buf, sv->stream);
                 return 0;
             });
             QVD_HIP(hipGetLastError());

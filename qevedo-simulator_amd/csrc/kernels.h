@@ -52,15 +52,26 @@ struct PauliGroup {
     uint64_t x;
     uint32_t first, nterms, odd, pad;
 };
-// Blocks per group for a launch over ngroups groups.
-unsigned pauli_blocks(uint64_t len, uint32_t ngroups);
+// One launch: groups with the same number of term slots, their strings, and
+// the blocks each group gets.
+struct PauliLaunch {
+    uint32_t slots, group, ngroups, first, nterms, blocks;
+    uint64_t partial;  // first of its nterms * blocks partial sums
+};
+constexpr uint32_t PAULI_LAUNCHES = 5;  // 1, 2, 4, 8 and 16 slots
+struct PauliLaunches {
+    uint32_t n = 0;
+    uint64_t partials = 0;  // of all launches
+    PauliLaunch at[PAULI_LAUNCHES];
+};
+// widths: the groups' nterms, in descending order.
+PauliLaunches pauli_launches(uint64_t len, const std::vector<uint32_t> &widths);
 // out[t] = string t's sum over half of the indices where x != 0 (the value is
-// twice that), over all where x = 0. widths: the groups' nterms; partial holds
-// nterms * blocks doubles; groups and zs (one per string) are in device memory.
+// twice that), over all where x = 0. groups and zs (one per string) are in device
+// memory.
 template <typename T2>
-void launch_expect_pauli(const T2 *s, uint64_t len, const PauliGroup *groups, const std::vector<uint32_t> &widths,
-                         const uint64_t *zs, uint32_t nterms, double *partial, unsigned blocks, double *out,
-                         hipStream_t st);
+void launch_expect_pauli(const T2 *s, uint64_t len, const PauliGroup *groups, const PauliLaunches &launches,
+                         const uint64_t *zs, uint32_t nterms, double *partial, double *out, hipStream_t st);
 template <typename T2> void launch_widen(const T2 *s, double2 *out, uint64_t count, hipStream_t st);
 template <typename T2> void launch_narrow(const double2 *in, T2 *s, uint64_t count, hipStream_t st);
 template <typename T2> void launch_scale(T2 *s, uint64_t len, double factor, hipStream_t st);

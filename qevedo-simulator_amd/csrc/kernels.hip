@@ -524,7 +524,7 @@ __global__ void k_probabilities(const T2 *__restrict__ s, uint64_t len, double *
 // x != 0 only the j without x's highest bit are visited, each amplitude is
 // read once, and only the part that stays is summed: the imaginary one where
 // popcount(x & z) is odd. Per block and string the sum goes to
-// partial[string * blocks + block]. KT >= a group's strings (a power of two, so
+// partial[(string - first) * blocks + block]. KT >= a group's strings (a power of two, so
 // a group of few strings does not pay for PAULI_TERMS).
 //
 // Bound by memory (one read of the state per group): 30 qubits in complex64,
@@ -533,7 +533,7 @@ __global__ void k_probabilities(const T2 *__restrict__ s, uint64_t len, double *
 template <typename T2, int KT>
 __global__ __launch_bounds__(RED_THREADS) void k_expect_pauli(const T2 *__restrict__ s, uint64_t len,
                                                               const PauliGroup *__restrict__ groups,
-                                                              const uint64_t *__restrict__ zs,
+                                                              const uint64_t *__restrict__ zs, uint32_t first,
                                                               double *__restrict__ partial) {
     __shared__ double scratch[RED_THREADS / 64];
     const PauliGroup g = groups[blockIdx.y];
@@ -581,7 +581,7 @@ __global__ __launch_bounds__(RED_THREADS) void k_expect_pauli(const T2 *__restri
 #pragma unroll
     for (int t = 0; t < KT; t++) {
         const double r = block_sum(sum[t], scratch);
-        if (threadIdx.x == 0 && t < (int)g.nterms) partial[(uint64_t)(g.first + t) * gridDim.x + blockIdx.x] = r;
+        if (threadIdx.x == 0 && t < (int)g.nterms) partial[(uint64_t)(g.first - first + t) * gridDim.x + blockIdx.x] = r;
     }
 }
 
@@ -594,6 +594,20 @@ __global__ __launch_bounds__(RED_THREADS) void k_sum_rows(const double *__restri
     const double *const row = partial + (uint64_t)blockIdx.x * m;
     double r = 0;
     for (uint32_t i = threadIdx.x; i < m; i += RED_THREADS) r += row[i];
+    r = block_sum(r, scratch);
+    if (threadIdx.x == 0) out[blockIdx.x] = r;
+}
+
+// The same for the strings of several launches, whose rows differ in length.
+__global__ __launch_bounds__(RED_THREADS) void k_sum_paulis(const double *__restrict__ partial, const PauliLaunches l,
+                                                            double *__restrict__ out) {
+    __shared__ double scratch[RED_THREADS / 64];
+    uint32_t i = 0;
+    while (i + 1 < l.n && blockIdx.x >= l.at[i + 1].first) i++;
+    const uint32_t m = l.at[i].blocks;
+    const double *const row = partial + l.at[i].partial + (uint64_t)(blockIdx.x - l.at[i].first) * m;
+    double r = 0;
+    for (uint32_t j = threadIdx.x; j < m; j += RED_THREADS) r += row[j];
     r = block_sum(r, scratch);
     if (threadIdx.x == 0) out[blockIdx.x] = r;
 }
@@ -1511,39 +1525,52 @@ void launch_probabilities(const T2 *s, uint64_t len, double *out, hipStream_t st
     k_probabilities<T2><<<grid_for(len, 256), 256, 0, st>>>(s, len, out);
 }
 
-template <typename T2>
-static void pauli_group_launch(const T2 *s, uint64_t len, const PauliGroup *groups, uint32_t ngroups, uint32_t width,
-                               const uint64_t *zs, double *partial, unsigned blocks, hipStream_t st) {
-    const dim3 grid(blocks, ngroups);
-    if (width <= 1) k_expect_pauli<T2, 1><<<grid, RED_THREADS, 0, st>>>(s, len, groups, zs, partial);
-    else if (width <= 2) k_expect_pauli<T2, 2><<<grid, RED_THREADS, 0, st>>>(s, len, groups, zs, partial);
-    else if (width <= 4) k_expect_pauli<T2, 4><<<grid, RED_THREADS, 0, st>>>(s, len, groups, zs, partial);
-    else if (width <= 8) k_expect_pauli<T2, 8><<<grid, RED_THREADS, 0, st>>>(s, len, groups, zs, partial);
-    else k_expect_pauli<T2, PAULI_TERMS><<<grid, RED_THREADS, 0, st>>>(s, len, groups, zs, partial);
-}
-
-// Four pairs of amplitudes a thread where the state is small, and enough
-// blocks over all groups of a launch to fill the chip where it is large.
-unsigned pauli_blocks(uint64_t len, uint32_t ngroups) {
+// Four pairs of amplitudes a thread where the state is small, and enough blocks
+// over the groups of a launch to fill the chip where it is large. Launches follow
+// one another, so each has to fill it by itself (28 qubits in complex64, a group each
+// of 16, 8, 4 and 2 strings and 16 single ones, on low qubits: 13.3 ms with the blocks
+// shared out over all 20 groups, 6.1 so). A power of two of them: every block
+// then runs the same rounds (31 groups of one string and one of 16: 10.4 ms with 66
+// blocks a group, 7.2 with 64).
+PauliLaunches pauli_launches(uint64_t len, const std::vector<uint32_t> &widths) {
+    auto slots = [](uint32_t w) { return w <= 1 ? 1u : w <= 2 ? 2u : w <= 4 ? 4u : w <= 8 ? 8u : PAULI_TERMS; };
     const uint64_t want = std::max<uint64_t>(1, len / (2 * 4 * RED_THREADS));
-    const uint64_t cap = std::max<uint64_t>(64, 2048 / std::max<uint32_t>(ngroups, 1));
-    return (unsigned)std::min(want, cap);
+    PauliLaunches l;
+    uint32_t first = 0;
+    for (size_t g = 0; g < widths.size();) {
+        PauliLaunch &p = l.at[l.n++];
+        p = {slots(widths[g]), (uint32_t)g, 0, first, 0, 0, l.partials};
+        for (; g < widths.size() && slots(widths[g]) == p.slots; g++) {
+            p.ngroups++;
+            p.nterms += widths[g];
+        }
+        uint64_t cap = 64;
+        while (2 * cap * p.ngroups <= 2048) cap *= 2;
+        p.blocks = (uint32_t)std::min(want, cap);
+        first += p.nterms;
+        l.partials += (uint64_t)p.nterms * p.blocks;
+    }
+    return l;
 }
 
 template <typename T2>
-void launch_expect_pauli(const T2 *s, uint64_t len, const PauliGroup *groups, const std::vector<uint32_t> &widths,
-                         const uint64_t *zs, uint32_t nterms, double *partial, unsigned blocks, double *out,
-                         hipStream_t st) {
-    double *const to = blocks == 1 ? out : partial;
-    // Runs of groups with the same number of term slots are one launch.
-    auto slots = [](uint32_t w) { return w <= 1 ? 1 : w <= 2 ? 2 : w <= 4 ? 4 : w <= 8 ? 8 : 16; };
-    for (size_t g = 0; g < widths.size();) {
-        size_t e = g + 1;
-        while (e < widths.size() && slots(widths[e]) == slots(widths[g])) e++;
-        pauli_group_launch(s, len, groups + g, (uint32_t)(e - g), widths[g], zs, to, blocks, st);
-        g = e;
+void launch_expect_pauli(const T2 *s, uint64_t len, const PauliGroup *groups, const PauliLaunches &launches,
+                         const uint64_t *zs, uint32_t nterms, double *partial, double *out, hipStream_t st) {
+    bool direct = true;  // a block per group everywhere: its sums are the results
+    for (uint32_t i = 0; i < launches.n; i++) direct = direct && launches.at[i].blocks == 1;
+    for (uint32_t i = 0; i < launches.n; i++) {
+        const PauliLaunch &p = launches.at[i];
+        auto go = [&](auto k) {
+            k<<<dim3(p.blocks, p.ngroups), RED_THREADS, 0, st>>>(s, len, groups + p.group, zs, p.first,
+                                                                 direct ? out + p.first : partial + p.partial);
+        };
+        if (p.slots == 1) go(k_expect_pauli<T2, 1>);
+        else if (p.slots == 2) go(k_expect_pauli<T2, 2>);
+        else if (p.slots == 4) go(k_expect_pauli<T2, 4>);
+        else if (p.slots == 8) go(k_expect_pauli<T2, 8>);
+        else go(k_expect_pauli<T2, PAULI_TERMS>);
     }
-    if (blocks > 1) k_sum_rows<<<nterms, RED_THREADS, 0, st>>>(partial, blocks, out);
+    if (!direct) k_sum_paulis<<<nterms, RED_THREADS, 0, st>>>(partial, launches, out);
 }
 
 // Segments of 2^16 amplitudes, 64 a thread; a single state of fewer than 24
@@ -1723,8 +1750,8 @@ hipError_t launch_sample_walk(const T2 *s, uint64_t len, uint64_t chunk, uint64_
     template void launch_norm<T2>(const T2 *, uint64_t, int, double *, double *, hipStream_t);                  \
     template void launch_expect_z<T2>(const T2 *, uint32_t, double *, double *, double *, hipStream_t);         \
     template void launch_probabilities<T2>(const T2 *, uint64_t, double *, hipStream_t);                        \
-    template void launch_expect_pauli<T2>(const T2 *, uint64_t, const PauliGroup *, const std::vector<uint32_t> &, \
-                                          const uint64_t *, uint32_t, double *, unsigned, double *, hipStream_t); \
+    template void launch_expect_pauli<T2>(const T2 *, uint64_t, const PauliGroup *, const PauliLaunches &,      \
+                                          const uint64_t *, uint32_t, double *, double *, hipStream_t);         \
     template void launch_expect_batch<T2>(const T2 *, const ExpDesc *, uint32_t, const uint64_t *, uint64_t,    \
                                           const uint32_t *, uint32_t, double *, double *, double *, const ExpDesc &, \
                                           hipStream_t);                                                         \

@@ -1,0 +1,41 @@
+"""Pauli strings beyond one page and one submission (X parts that straddle one), and
+groups of every width in one call."""
+import numpy as np
+import pytest
+
+from helpers import random_state, rng
+from qevedo.simulator import StateVector
+
+pytestmark = pytest.mark.gpu
+
+
+def small_calls(sv, x, z):
+    return np.concatenate([sv.expect_pauli(x[i:i + 9], z[i:i + 9]) for i in range(0, len(x), 9)])
+
+
+@pytest.mark.parametrize("n,count", [(10, 512), (10, 513), (10, 5000), (13, 4100)])
+@pytest.mark.parametrize("precision", ["single", "double"])
+def test_many_strings(n, count, precision):
+    """Sums of 2^n products of amplitudes, at most 1 in all: below 1e-12 apart in any order."""
+    r = np.random.Generator(np.random.PCG64(count))
+    xs = r.integers(0, 1 << n, count // 7)
+    x = [int(v) for v in r.choice(xs, count)]
+    z = [int(v) for v in r.integers(0, 1 << n, count)]
+    with StateVector(n, precision) as sv:
+        sv.set_amplitudes(random_state(rng(n), n))
+        assert np.max(np.abs(sv.expect_pauli(x, z) - small_calls(sv, x, z))) < 1e-12
+
+
+@pytest.mark.parametrize("n", [12, 17, 21])
+@pytest.mark.parametrize("narrow", [0, 3, 40])
+def test_groups_of_every_width(n, narrow):
+    r = np.random.Generator(np.random.PCG64(n + narrow))
+    x, z = [], []
+    for part, width in [(0, 16), (0, 5), (3, 8), (1 << (n - 1), 3), (6, 2)] + [(8 + i, 1) for i in range(narrow)]:
+        x += [part] * width
+        z += [int(v) for v in r.integers(0, 1 << n, width)]
+    order = r.permutation(len(x))
+    x, z = [x[i] for i in order], [z[i] for i in order]
+    with StateVector(n, "double") as sv:
+        sv.set_amplitudes(random_state(rng(n), n))
+        assert np.max(np.abs(sv.expect_pauli(x, z) - small_calls(sv, x, z))) < 1e-12
