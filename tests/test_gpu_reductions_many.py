@@ -1,10 +1,11 @@
-"""Pauli strings beyond one page and one submission (X parts that straddle one), and
-groups of every width in one call."""
+"""Reductions beyond one page, one submission or one wave: Pauli strings by the
+hundreds and thousands (X parts that straddle a submission), groups of every width
+in one call, and <Z>, <ZZ> of states with more segments than a wave walks."""
 import numpy as np
 import pytest
 
 from helpers import random_state, rng
-from qevedo.simulator import StateVector
+from qevedo.simulator import Batch, StateVector, lower_gates
 
 pytestmark = pytest.mark.gpu
 
@@ -39,3 +40,24 @@ def test_groups_of_every_width(n, narrow):
     with StateVector(n, "double") as sv:
         sv.set_amplitudes(random_state(rng(n), n))
         assert np.max(np.abs(sv.expect_pauli(x, z) - small_calls(sv, x, z))) < 1e-12
+
+
+@pytest.mark.parametrize("n,precision,tol", [(24, "single", 1e-5), (25, "single", 1e-5), (26, "double", 1e-12)])
+def test_z_of_many_segments(n, precision, tol):
+    """A product of rx(t_q)|0>: <Z_q> = cos t_q. Two roundings of a factor per qubit."""
+    t = 0.1 + 0.11 * np.arange(n)
+    with StateVector(n, precision) as sv:
+        sv.apply_ops(lower_gates([("rx", (q,), (float(t[q]),)) for q in range(n)]))
+        z, zz = sv.expect_z()
+    c = np.cos(t)
+    assert np.max(np.abs(z - c)) < tol and np.max(np.abs(zz - c[:-1] * c[1:])) < tol
+
+
+@pytest.mark.parametrize("n,precision,tol", [(5, "double", 1e-12), (14, "single", 1e-5), (17, "double", 1e-12)])
+def test_batch_of_one_circuit(n, precision, tol):
+    t = 0.1 + 0.11 * np.arange(n)
+    batch = Batch([(n, lower_gates([("rx", (q,), (float(t[q]),)) for q in range(n)]))], precision)
+    (z, zz), = batch.run()
+    batch.close()
+    c = np.cos(t)
+    assert np.max(np.abs(z - c)) < tol and np.max(np.abs(zz - c[:-1] * c[1:])) < tol
