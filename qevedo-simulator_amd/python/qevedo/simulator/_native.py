@@ -234,10 +234,11 @@ _OP = np.dtype([("targets", "u8"), ("num_targets", "u4"), ("pad0", "u4"), ("cont
 assert _OP.itemsize == C.sizeof(Op)
 
 
-def _qubit_list(qubits):
+_WHOLE = {int, bool} | {np.dtype(c).type for c in np.typecodes["AllInteger"]}
+
+
+def _qubit_list(qubits) -> list:
     """Qubits as a flat list, from any form NumPy takes as an array of them."""
-    if isinstance(qubits, (list, tuple)) and set(map(type, qubits)) <= {int}:
-        return qubits
     return np.ascontiguousarray(qubits, dtype=np.uint32).reshape(-1).tolist()
 
 
@@ -245,13 +246,15 @@ class OpArray:
     """A qvd_op array plus the NumPy buffers it points into: all ops' targets,
     controls and control values in one buffer each, each matrix object once."""
 
-    def __init__(self, ops):
-        self.n = len(ops)
+    def _collect(self, ops, flatten: bool):
+        """All targets and controls, control values, counts of both, and matrix
+        addresses. flatten: lists are not taken as flat lists of whole numbers."""
         matrices = {}  # id -> (address, rows); self.keep holds the arrays
         self.keep = []
         qubits, values, counts, addresses = [], [], [], []
         for targets, controls, matrix in ops:
-            targets = _qubit_list(targets)
+            if flatten or not isinstance(targets, (list, tuple)):
+                targets = _qubit_list(targets)
             entry = matrices.get(id(matrix))
             if entry is None:
                 m = np.ascontiguousarray(matrix, dtype=np.complex128)
@@ -265,9 +268,23 @@ class OpArray:
             counts.append(len(targets))
             counts.append(len(controls))
             addresses.append(entry[0])
-            if len(controls):
-                qubits += _qubit_list([c[0] for c in controls])
-                values += [1 if c[1] else 0 for c in controls]
+            for c in controls:
+                if flatten:
+                    qubits += _qubit_list(c[0])
+                else:
+                    qubits.append(c[0])
+                values.append(1 if c[1] else 0)
+        return qubits, values, counts, addresses
+
+    def __init__(self, ops):
+        self.n = len(ops)
+        try:
+            qubits, values, counts, addresses = self._collect(ops, False)
+            flat = set(map(type, qubits)) <= _WHOLE
+        except ValueError:
+            flat = False
+        if not flat:
+            qubits, values, counts, addresses = self._collect(ops, True)
         qubits = np.array(qubits, dtype=np.uint32)
         values = np.array(values, dtype=np.uint8)
         counts = np.array(counts, dtype=np.uint64).reshape(-1, 2)
