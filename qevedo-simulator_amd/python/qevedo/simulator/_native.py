@@ -197,16 +197,19 @@ def gate_matrix(name: str, params=()) -> np.ndarray:
 _LOWER_OUT = C.c_double * (2 * 64)
 # ctypes arrays of up to 8 parameters (a new array type costs more than the call).
 _LOWER_PARAMS = tuple(C.c_double * max(k, 1) for k in range(9))
-_NUMBERS = {float, int, np.float64}
 
 
 def gate_lower(name: str, params=()) -> tuple:
     """(number of leading controls, base matrix) of a named gate."""
-    if not (isinstance(params, (list, tuple)) and set(map(type, params)) <= _NUMBERS):
-        # numbers of NumPy's own, texts, nested lists
+    if not isinstance(params, (list, tuple)):
         params = np.ascontiguousarray(params, dtype=np.float64).reshape(-1).tolist()
     n = len(params)
-    p = (_LOWER_PARAMS[n] if n < len(_LOWER_PARAMS) else C.c_double * n)(*params)
+    try:
+        p = (_LOWER_PARAMS[n] if n < len(_LOWER_PARAMS) else C.c_double * n)(*params)
+    except (TypeError, DeprecationWarning):  # what only NumPy turns into numbers: texts, nested lists
+        params = np.ascontiguousarray(params, dtype=np.float64).reshape(-1).tolist()
+        n = len(params)
+        p = (C.c_double * max(n, 1))(*params)
     out = _LOWER_OUT()
     nc, nt = C.c_uint32(), C.c_uint32()
     _check(lib().qvd_gate_lower(name.encode(), p, n, C.byref(nc), C.byref(nt), out, 64))
