@@ -91,8 +91,9 @@ typedef struct qvd_options {
 /* qvd_options.flags: time every kernel launch with HIP events on the
  * handle's stream and report the sums in qvd_stats. */
 #define QVD_FLAG_TIMING 1u
-/* qvd_options.flags: apply 5- and 6-qubit dense ops in complex64 with VALU
- * FMAs instead of the FP32 matrix cores (for comparisons). */
+/* qvd_options.flags: apply the dense ops that go to the matrix cores (5 and 6
+ * targets, in complex128 also 3 and 4 with two or more of them inside a
+ * 128-byte line) with VALU FMAs instead (for comparisons). */
 #define QVD_FLAG_DENSE_VALU 2u
 /* qvd_options.flags: pick the register-tile geometry (qvd_circuit.fixed_lanes
  * or qvd_options.fixed_lanes left 0) by timing. Circuits of the same size and

@@ -1,5 +1,5 @@
-// Launcher of the matrix-core dense kernel for fused 5- and 6-qubit gates
-// (dense_mfma.hip).
+// Launcher of the matrix-core dense kernel for fused gates of 5 and 6 targets,
+// in complex128 also 3 and 4 (dense_mfma.hip).
 #pragma once
 
 #include <hip/hip_runtime.h>

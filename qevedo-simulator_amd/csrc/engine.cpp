@@ -226,9 +226,9 @@ auto with_type(const qvd_sv *sv, F &&f) {
 }
 
 // |0...0> is written lazily: qvd_sv_create and qvd_sv_set_zero only mark the
-// state, the next qvd_sv_apply_ops whose plan starts with a register-tile
-// stage makes that stage's tiles from |0...0> in registers (no init pass and
-// no tile loads), and a plan of register-tile stages only may leave the
+// state, the next qvd_sv_apply_ops whose plan starts with a stage makes that
+// stage's tiles from |0...0> in registers or in LDS (no init pass and no tile
+// loads), and a plan of register-tile stages only may leave the
 // amplitudes of stale qubits unwritten (run_plan). Any other use of the
 // state writes the missing zeros first.
 void materialize(qvd_sv *sv, bool wait = true) {

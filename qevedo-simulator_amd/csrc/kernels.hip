@@ -233,7 +233,8 @@ __global__ __launch_bounds__(256) void k_diag(T2 *__restrict__ s, uint64_t len, 
 // matrices of a run of ops are therefore copied to LDS together (a load per
 // op was a memory round trip per op), and an op of fewer groups than threads
 // deals the rows of its matrix out as well: 12 qubits in complex128, 120 gates
-// fused to 4 qubits, 541 -> 91 us.
+// fused to 4 qubits, 541 -> 91 us. (With 1024 threads in complex128 the 128 VGPRs a
+// thread gets leave 64 bytes of it in scratch.)
 // ---------------------------------------------------------------------------
 constexpr uint32_t STAGE_OPS = 48;             // op records held in LDS
 constexpr uint32_t STAGE_COEF_BYTES = 8192;    // their matrices and diagonals

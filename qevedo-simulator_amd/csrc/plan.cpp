@@ -98,29 +98,8 @@ std::vector<Op> fuse(const std::vector<Op> &ops, size_t max_qubits) {
 namespace {
 
 // Take every pending op that can run now and whose qubits no earlier
-// pending op blocks (src/blocking.rs:157-179).
-template <typename F>
-std::vector<size_t> extract(const std::vector<Op> &ops, const std::vector<char> &done, F &&can_run) {
-    std::vector<size_t> taken;
-    std::vector<uint32_t> blocked;
-    for (size_t i = 0; i < ops.size(); i++) {
-        if (done[i]) continue;
-        const std::vector<uint32_t> oq = ops[i].qubits();
-        bool touches = false;
-        for (uint32_t q : oq) touches |= contains(blocked, q);
-        if (!touches && can_run(ops[i])) {
-            taken.push_back(i);
-        } else {
-            for (uint32_t q : oq)
-                if (!contains(blocked, q)) blocked.push_back(q);
-        }
-    }
-    return taken;
-}
-
-// extract over qubit masks (bit q = qubit q): the same ops in the same
-// order, without building each op's qubit list on every pass. can_run takes
-// the op's index.
+// pending op blocks (src/blocking.rs:157-179). Qubits are masks (bit q = qubit
+// q); can_run takes the op's index.
 template <typename F>
 std::vector<size_t> extract_masked(const std::vector<uint64_t> &qmask, const std::vector<char> &done, F &&can_run) {
     std::vector<size_t> taken;

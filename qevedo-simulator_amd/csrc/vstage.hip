@@ -1178,9 +1178,11 @@ size_t vstage_lds_bytes() {
 }
 
 // Two complex128 workgroups share a CU when the LDS tile holds one part of the
-// amplitudes (64 KiB) and each thread 16 amplitudes without a prefetch set (128
-// VGPRs): 4 waves per SIMD instead of 2, in two groups that wait for their
-// exchanges, loads and instructions independently. One group left the VALU
+// amplitudes (64 KiB) and each thread 16 amplitudes without a prefetch set: 4
+// waves per SIMD instead of 2, in two groups that wait for their exchanges, loads and
+// instructions independently. The 128 VGPRs that leaves do not quite hold the
+// interpreter: 27 registers (34 with unwritten zeros) spill to 112 (132) bytes
+// of scratch a thread. One group left the VALU
 // idle 58 % of a deep stage. With fewer tiles than two per CU there is nothing
 // to overlap and the second pair of barriers costs. Kicked Ising, 10 steps, all
 // stages: 26 qubits 4.88 -> 4.06 ms, 24 0.95 -> 0.84, 22 (2 tiles per CU)
